@@ -1818,6 +1818,45 @@ hipError_t fused_bars_dispatch(hipStream_t s, const FusedFields& ff, const float
 
 }  // namespace
 
+// Small volumes (FP32 fields, at most SMALL_VOXELS or SMALL_VOXELS_ODD, 8 planes
+// or more): the launch
+// is bound by the latency of a block's zc + 2 dependent plane steps (load, two
+// barriers, two chains of square roots and divisions), not by bandwidth, so the
+// plan minimises, in units of one step's latency,
+//   (zc + 2) + c (waves on the busiest CU) (zc + 1) + e (waves of a block) (zc + 2),
+// whole rows, two voxels per thread with the prefetch (c 0.4, e 0) or one on odd
+// widths (c 0.15, e 0.05).  c and e are fits to every band of 1 .. 20 rows x chunk
+// of 1 .. 16 planes on 18 shapes; the plans they choose against the ones of the
+// bandwidth model below (us per launch): 32x30x24 6.8 / 13.6, 48^3 8.8 / 20.1,
+// 64^3 11.3 / 17.2, 16x100x180 12.8 / 22.7, 72^3 15.0 / 20.4, 63x45x31 7.4 / 10.1.
+// Beyond the limits the bandwidth model is as good or better: 80x80x76 18.0 /
+// 18.1 (masked 24.6 / 20.9), 88^3 25.0 / 21.9; odd 33x33x250 14.1 / 12.6, 67x63x41
+// 11.1 / 11.2 (masked 16.7 / 13.1).  BF16 fields keep the bandwidth model: its plans
+// already have short chunks there (the same fit gained 5% in the mean and lost 8%
+// at 34x32x250), and so do images and slabs of fewer than 8 planes (500^2: 17.1
+// / 11.3).
+constexpr size_t SMALL_VOXELS = 400000, SMALL_VOXELS_ODD = 170000;
+
+bool small_fused_plan(const Geometry& g, int cus, int max_lds, FusedPlan* plan) {
+    const bool even = g.w % 2 == 0;
+    const int L = even ? g.w / 2 : g.w;
+    const double c = even ? 0.4 : 0.15, e = even ? 0.0 : 0.05;
+    double best = 1e300;
+    for (int ty = 1; L * (ty + 2) <= 768 && ty <= g.h; ++ty) {
+        const size_t lds = (even ? fused_lds_floats<2>(g.w, ty) : fused_lds_floats<1>(g.w, ty)) *
+                           sizeof(float);
+        if (lds > size_t(max_lds)) break;
+        const long waves = (L * (ty + 2) + 63) / 64, bands = (g.h + ty - 1) / ty;
+        for (int zc = 1; zc <= std::min(g.d, 16); ++zc) {
+            const long blocks = bands * ((g.d + zc - 1) / zc);
+            const double cu_waves = double((blocks + cus - 1) / cus * waves);
+            const double cost = (zc + 2) + c * cu_waves * (zc + 1) + e * waves * (zc + 2);
+            if (cost < best) { best = cost; *plan = FusedPlan{ty, zc, even ? 1 : 0, even ? 2 : 1, 0}; }
+        }
+    }
+    return best < 1e300;
+}
+
 // Plan of the fused sweep for a geometry: voxels per thread (vx), band height
 // ty and z chunk.  Cost model: rounds of resident blocks x blocks per CU x the
 // rows and planes each block marches (the halo row / plane on each side does
@@ -1860,6 +1899,13 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
             *plan = ip;
             return true;
         }
+    }
+    if (storage == 0 && !big_index && g.n() <= (g.w % 2 ? SMALL_VOXELS_ODD : SMALL_VOXELS) &&
+        g.d >= 8 && !want_vx && !want_ty && !want_zc && want_tx == 0 &&
+        small_fused_plan(g, cus, max_lds, &bp)) {
+        if (bp.vx == 2 && (want_pf == 0 || want_pf == 1)) bp.pf = want_pf;
+        *plan = bp;
+        return true;
     }
     // odd widths: one voxel per thread (the two- and four-voxel forms need
     // lanes that lie wholly inside the row), whole rows only while bands of two

@@ -307,3 +307,27 @@ def test_fused_wide_rows_run_tiled(ctx, orc, shape):
     np.testing.assert_array_equal(u, st.u)
     for k, v in enumerate((vx, vy, vz)):
         np.testing.assert_array_equal(v, st.v[k])
+
+
+# the small-volume plans: short chunks and tall bands, partial ones among them,
+# the thread limit (widths 8 and 300 cap the band at opposite ends), and both
+# sides of the size limits (even 400000, odd 170000 voxels)
+@pytest.mark.parametrize("shape", [(8, 9, 10), (24, 30, 32), (300, 8, 8), (8, 300, 8), (8, 8, 300),
+                                   (9, 13, 21), (8, 45, 63), (50, 80, 100), (50, 80, 102),
+                                   (17, 100, 99), (18, 100, 99)])
+def test_fused_small_volume_plans(ctx, orc, shape):
+    from ambient_image_processor_amd import native
+    _say("small", shape)
+    f = _f(shape, 11)
+    act = np.random.default_rng(5).random(shape) < 0.4
+    for data_term in ("l1", "l2"):
+        p = _params(native, 4, data_term)
+        out = ctx.tgv2_deshade(f, p)
+        st = orc.tgv2(f, 4, data_term=data_term, dtype=np.float32, **PRM)
+        np.testing.assert_array_equal(out[0], st.u)
+        for c in range(3):
+            np.testing.assert_array_equal(out[1 + c], st.v[c])
+    st = orc.tgv2(f, 4, data_term="l1", dtype=np.float32, mask=act.astype(np.float32), **PRM)
+    out = ctx.tgv2_deshade_masked(f, _params(native, 4, "l1"), act)
+    np.testing.assert_array_equal(out[0], st.u)
+    np.testing.assert_array_equal(out[2], st.v[1])
