@@ -249,11 +249,26 @@ hipError_t launch_divergence(hipStream_t s, const float* vx, const float* vy, co
 hipError_t launch_dct_reference_pass(hipStream_t s, const float* in, float* out,
                                      const double* table, Geometry g, int axis, int inverse,
                                      int last);
-hipError_t launch_dct_mfma_pass(hipStream_t s, const float* in, float* out, const float* table,
-                                const uint16_t* table_hi, const uint16_t* table_lo, Geometry g,
-                                int axis, int inverse, int last, int precision,
+// One MFMA pass along `axis`.  precision 1 (F32): table = the n x n FP32 matrix
+// [k][m]; 2 (BF16x3): the bf16 split table in fragment order (dct_fragments).
+// scale multiplies every output; fuse_poisson divides it by its eigenvalue.
+// in and out must not overlap.
+hipError_t launch_dct_mfma_pass(hipStream_t s, const float* in, float* out, const void* table,
+                                Geometry g, int axis, float scale, int precision,
                                 const float* eig_x, const float* eig_y, const float* eig_z,
                                 int fuse_poisson, int quirk);
+// Element (row k, column m) of an n x n table in BF16x3 fragment order: the
+// index of its hi value in the uint16 array; its lo value lies 512 further on.
+// Fragments cover 16 rows x 32 columns (zero beyond n): lane = 16 (m % 32 / 8) +
+// k % 16 holds 8 consecutive columns.
+inline size_t dct_fragment_index(int n, int k, int m) {
+    const size_t chunks = size_t((n + 31) / 32);
+    const size_t frag = (size_t(k / 16) * chunks + size_t(m / 32)) * 2;
+    return frag * 512 + size_t(m % 32 / 8 * 16 + k % 16) * 8 + size_t(m % 8);
+}
+inline size_t dct_fragment_count(int n) {
+    return size_t((n + 15) / 16) * size_t((n + 31) / 32) * 1024;
+}
 int dct_mfma_max_extent();
 hipError_t launch_poisson_divide(hipStream_t s, const float* in, float* out, const float* cx,
                                  const float* cy, const float* cz, Geometry g, int quirk);

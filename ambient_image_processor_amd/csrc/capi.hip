@@ -64,12 +64,10 @@ struct AxisTables {
     int n = 0;
     double* fwd64 = nullptr;     // [m][k] cospi((m+0.5)k/n)
     double* inv64 = nullptr;     // [m][k] cospi((k+0.5)m/n)
-    float* fwd32 = nullptr;      // FP32 copies for the MFMA passes, [k][m] layout
+    float* fwd32 = nullptr;      // FP32, [k][m] layout
     float* inv32 = nullptr;
-    uint16_t* fwd_hi = nullptr;  // bf16 splits, [k][m]
-    uint16_t* fwd_lo = nullptr;
-    uint16_t* inv_hi = nullptr;
-    uint16_t* inv_lo = nullptr;
+    uint16_t* fwd_split = nullptr;  // bf16 splits in fragment order
+    uint16_t* inv_split = nullptr;
     float* eig = nullptr;        // float(cospi(float(k)/float(n))), n + 1 entries
 };
 
@@ -298,7 +296,7 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
 }
 
 void free_axis(AxisTables& t) {
-    void* ptrs[] = {t.fwd64, t.inv64, t.fwd32, t.inv32, t.fwd_hi, t.fwd_lo, t.inv_hi, t.inv_lo, t.eig};
+    void* ptrs[] = {t.fwd64, t.inv64, t.fwd32, t.inv32, t.fwd_split, t.inv_split, t.eig};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     t = AxisTables();
@@ -323,89 +321,86 @@ float host_bf16_to_float(uint16_t h) {
 // no such limit.
 constexpr int DCT_MAX_EXTENT = 16384;
 
-// Cosine tables for one axis of extent n (built once per extent, host FP64,
-// uploaded in row chunks so that host memory stays O(n)): the FP64 [m][k]
-// tables of the reference-numerics passes always, the FP32 and bf16-split
-// [k][m] tables of the MFMA passes only for n <= dct_mfma_max_extent().
-amb_status ensure_axis(amb_context* c, int axis, int n) {
+// Cosine tables for one axis of extent n (host FP64, uploaded in row chunks so
+// that host memory stays O(n)), built when a precision first needs them and
+// kept while the extent stays: the FP64 [m][k] tables of the
+// reference-numerics passes, the FP32 [k][m] tables of the F32 passes, the bf16
+// splits of the BF16x3 passes in fragment order.  precision < 0: the Poisson
+// eigenvalues' cosines only.
+amb_status ensure_axis(amb_context* c, int axis, int n, int precision) {
     AxisTables& t = c->axes[axis];
-    if (t.n == n) return AMB_OK;
-    if (n > DCT_MAX_EXTENT)
-        return fail(AMB_ERR_NOT_SUPPORTED,
-                    "DCT Poisson solve: extent " + std::to_string(n) +
-                        " exceeds 16384 (the cosine tables would exceed 4 GiB per axis)");
-    free_axis(t);
-    const size_t nn = size_t(n) * n;
-    const bool mfma = n <= dct_mfma_max_extent();
+    if (t.n != n) {
+        if (n > DCT_MAX_EXTENT)
+            return fail(AMB_ERR_NOT_SUPPORTED,
+                        "DCT Poisson solve: extent " + std::to_string(n) +
+                            " exceeds 16384 (the cosine tables would exceed 4 GiB per axis)");
+        free_axis(t);
+        std::vector<float> eig(size_t(n) + 1);
+        for (int k = 0; k <= n; ++k) eig[k] = float(host_cospi(double(float(k) / float(n))));
+        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.eig), (size_t(n) + 1) * 4));
+        AMB_HIP(hipMemcpy(t.eig, eig.data(), (size_t(n) + 1) * 4, hipMemcpyHostToDevice));
+        t.n = n;
+    }
     const double size = double(float(n));
-    AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.fwd64), nn * 8));
-    AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.inv64), nn * 8));
-    if (mfma) {
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.fwd32), nn * 4));
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.inv32), nn * 4));
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.fwd_hi), nn * 2));
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.fwd_lo), nn * 2));
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.inv_hi), nn * 2));
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.inv_lo), nn * 2));
-    }
-    AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.eig), (size_t(n) + 1) * 4));
-    const size_t rows = std::max<size_t>(1, (size_t(1) << 21) / size_t(n));   // ~2M entries
-    std::vector<double> a64, b64;
-    std::vector<float> a32, b32;
-    std::vector<uint16_t> ah, al, bh, bl;
-    for (size_t r0 = 0; r0 < size_t(n); r0 += rows) {
-        const size_t nr = std::min(rows, size_t(n) - r0), cnt = nr * size_t(n);
-        // FP64 reference tables, row r = m: [m][k] cospi((m+0.5)k/n), cospi((k+0.5)m/n)
-        a64.resize(cnt);
-        b64.resize(cnt);
-        for (size_t r = 0; r < nr; ++r) {
-            const int m = int(r0 + r);
-            for (int k = 0; k < n; ++k) {
-                a64[r * n + k] = host_cospi((double(m) + 0.5) * double(k) / size);
-                b64[r * n + k] = host_cospi((double(k) + 0.5) * double(m) / size);
-            }
+    // the inverse folds the reference's "X[0] + 2 sum_{m>=1}" into weights 1, 2
+    auto fwd = [&](int k, int m) { return host_cospi((double(m) + 0.5) * double(k) / size); };
+    auto inv = [&](int k, int m) {
+        return (m == 0 ? 1.0 : 2.0) * host_cospi((double(k) + 0.5) * double(m) / size);
+    };
+    // an n x n table of T: rows through the host in chunks of ~2M entries
+    auto upload = [&](auto** dst, auto value) -> amb_status {
+        typedef typename std::remove_reference<decltype(**dst)>::type T;
+        T* dev = nullptr;
+        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&dev), size_t(n) * n * sizeof(T)));
+        const size_t rows = std::max<size_t>(1, (size_t(1) << 21) / size_t(n));
+        std::vector<T> h;
+        for (size_t r0 = 0; r0 < size_t(n); r0 += rows) {
+            const size_t nr = std::min(rows, size_t(n) - r0), cnt = nr * size_t(n);
+            h.resize(cnt);
+            for (size_t r = 0; r < nr; ++r)
+                for (int j = 0; j < n; ++j) h[r * n + j] = T(value(int(r0 + r), j));
+            const hipError_t e = hipMemcpy(dev + r0 * n, h.data(), cnt * sizeof(T), hipMemcpyHostToDevice);
+            if (e != hipSuccess) { (void)hipFree(dev); return fail_hip(e, "hipMemcpy", __LINE__); }
         }
-        AMB_HIP(hipMemcpy(t.fwd64 + r0 * n, a64.data(), cnt * 8, hipMemcpyHostToDevice));
-        AMB_HIP(hipMemcpy(t.inv64 + r0 * n, b64.data(), cnt * 8, hipMemcpyHostToDevice));
-        if (!mfma) continue;
-        // MFMA tables, row r = k: [k][m] (contiguous over the summed index); the
-        // inverse folds the reference's "X[0] + 2 sum_{m>=1}" into weights 1, 2
-        a32.resize(cnt); b32.resize(cnt);
-        ah.resize(cnt); al.resize(cnt); bh.resize(cnt); bl.resize(cnt);
-        for (size_t r = 0; r < nr; ++r) {
-            const int k = int(r0 + r);
+        *dst = dev;
+        return AMB_OK;
+    };
+    auto upload_split = [&](uint16_t** dst, auto value) -> amb_status {
+        std::vector<uint16_t> h(dct_fragment_count(n), uint16_t(0));
+        for (int k = 0; k < n; ++k)
             for (int m = 0; m < n; ++m) {
-                const double cf = host_cospi((double(m) + 0.5) * double(k) / size);
-                const double ci = (m == 0 ? 1.0 : 2.0) * host_cospi((double(k) + 0.5) * double(m) / size);
-                const size_t o = r * n + size_t(m);
-                a32[o] = float(cf);
-                b32[o] = float(ci);
-                const uint16_t h1 = host_bf16_rne(float(cf));
-                ah[o] = h1;
-                al[o] = host_bf16_rne(float(cf - double(host_bf16_to_float(h1))));
-                const uint16_t h2 = host_bf16_rne(float(ci));
-                bh[o] = h2;
-                bl[o] = host_bf16_rne(float(ci - double(host_bf16_to_float(h2))));
+                const double v = value(k, m);
+                const size_t i = dct_fragment_index(n, k, m);
+                h[i] = host_bf16_rne(float(v));
+                h[i + 512] = host_bf16_rne(float(v - double(host_bf16_to_float(h[i]))));
             }
-        }
-        AMB_HIP(hipMemcpy(t.fwd32 + r0 * n, a32.data(), cnt * 4, hipMemcpyHostToDevice));
-        AMB_HIP(hipMemcpy(t.inv32 + r0 * n, b32.data(), cnt * 4, hipMemcpyHostToDevice));
-        AMB_HIP(hipMemcpy(t.fwd_hi + r0 * n, ah.data(), cnt * 2, hipMemcpyHostToDevice));
-        AMB_HIP(hipMemcpy(t.fwd_lo + r0 * n, al.data(), cnt * 2, hipMemcpyHostToDevice));
-        AMB_HIP(hipMemcpy(t.inv_hi + r0 * n, bh.data(), cnt * 2, hipMemcpyHostToDevice));
-        AMB_HIP(hipMemcpy(t.inv_lo + r0 * n, bl.data(), cnt * 2, hipMemcpyHostToDevice));
+        uint16_t* dev = nullptr;
+        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&dev), h.size() * 2));
+        const hipError_t e = hipMemcpy(dev, h.data(), h.size() * 2, hipMemcpyHostToDevice);
+        if (e != hipSuccess) { (void)hipFree(dev); return fail_hip(e, "hipMemcpy", __LINE__); }
+        *dst = dev;
+        return AMB_OK;
+    };
+    if (precision == AMB_DCT_REFERENCE) {
+        if (!t.fwd64) AMB_TRY(upload(&t.fwd64, [&](int m, int k) { return fwd(k, m); }));
+        if (!t.inv64)
+            AMB_TRY(upload(&t.inv64, [&](int m, int k) {
+                return host_cospi((double(k) + 0.5) * double(m) / size);
+            }));
+    } else if (precision == AMB_DCT_F32) {
+        if (!t.fwd32) AMB_TRY(upload(&t.fwd32, fwd));
+        if (!t.inv32) AMB_TRY(upload(&t.inv32, inv));
+    } else if (precision == AMB_DCT_BF16X3) {
+        if (!t.fwd_split) AMB_TRY(upload_split(&t.fwd_split, fwd));
+        if (!t.inv_split) AMB_TRY(upload_split(&t.inv_split, inv));
     }
-    std::vector<float> eig(size_t(n) + 1);
-    for (int k = 0; k <= n; ++k) eig[k] = float(host_cospi(double(float(k) / float(n))));
-    AMB_HIP(hipMemcpy(t.eig, eig.data(), (size_t(n) + 1) * 4, hipMemcpyHostToDevice));
-    t.n = n;
     return AMB_OK;
 }
 
-amb_status ensure_tables(amb_context* c, Geometry g) {
-    AMB_TRY(ensure_axis(c, 0, g.w));
-    AMB_TRY(ensure_axis(c, 1, g.h));
-    AMB_TRY(ensure_axis(c, 2, g.d));
+amb_status ensure_tables(amb_context* c, Geometry g, int precision) {
+    AMB_TRY(ensure_axis(c, 0, g.w, precision));
+    AMB_TRY(ensure_axis(c, 1, g.h, precision));
+    AMB_TRY(ensure_axis(c, 2, g.d, precision));
     return AMB_OK;
 }
 
@@ -1032,46 +1027,66 @@ amb_status check_precision(const Geometry& g, int precision) {
     return AMB_OK;
 }
 
-// One separable 3-pass transform from src into dst (src is overwritten as
-// scratch).  poisson_flags >= 0 fuses the eigenvalue divide into the last
-// forward pass (MFMA precisions only).
-amb_status transform3(amb_context* c, float* src, float* tmp, float* dst, int inverse,
-                      int precision, int poisson_flags = -1) {
+// One separable transform of src into dst through the scratch volumes a and b
+// (src is read by the first pass only, so b and dst may be src's buffer).  poisson_flags >= 0 fuses
+// the eigenvalue divide into the last forward pass (MFMA precisions only).
+amb_status transform3(amb_context* c, const float* src, float* a, float* b, float* dst,
+                      int inverse, int precision, int poisson_flags = -1) {
     const Geometry g = c->g;
     AMB_TRY(check_precision(g, precision));
-    AMB_TRY(ensure_tables(c, g));
-    float* bufs[4] = {src, tmp, src, dst};   // x: src->tmp, y: tmp->src, z: src->dst
-    for (int axis = 0; axis < 3; ++axis) {
-        ProfScope ps(c, P_DCT);
-        const AxisTables& t = c->axes[axis];
-        const int last = axis == 2;
-        if (precision == AMB_DCT_REFERENCE) {
-            AMB_HIP(launch_dct_reference_pass(c->stream, bufs[axis], bufs[axis + 1],
-                                              inverse ? t.inv64 : t.fwd64, g, axis, inverse, last));
-        } else {
-            const int fuse = (last && !inverse && poisson_flags >= 0) ? 1 : 0;
-            const int quirk = (poisson_flags > 0 && (poisson_flags & AMB_FLAG_POISSON_INDEX_QUIRK)) ? 1 : 0;
-            AMB_HIP(launch_dct_mfma_pass(c->stream, bufs[axis], bufs[axis + 1],
-                                         inverse ? t.inv32 : t.fwd32, inverse ? t.inv_hi : t.fwd_hi,
-                                         inverse ? t.inv_lo : t.fwd_lo, g, axis, inverse, last,
-                                         precision, c->axes[0].eig, c->axes[1].eig, c->axes[2].eig,
-                                         fuse, quirk));
+    AMB_TRY(ensure_tables(c, g, precision));
+    if (precision == AMB_DCT_REFERENCE) {
+        const float* in[3] = {src, a, b};
+        float* out[3] = {a, b, dst};
+        for (int axis = 0; axis < 3; ++axis) {
+            ProfScope ps(c, P_DCT);
+            const AxisTables& t = c->axes[axis];
+            AMB_HIP(launch_dct_reference_pass(c->stream, in[axis], out[axis],
+                                              inverse ? t.inv64 : t.fwd64, g, axis, inverse,
+                                              axis == 2));
         }
+        return AMB_OK;
+    }
+    // along an axis of one voxel the transform is the identity: no pass
+    const int ext[3] = {g.w, g.h, g.d};
+    int axes[3], np = 0;
+    for (int axis = 0; axis < 3; ++axis)
+        if (ext[axis] > 1 || (axis == 2 && np == 0)) axes[np++] = axis;
+    if (np == 1) {   // a single pass cannot run in place, and the caller's buffers may overlap
+        AMB_HIP(hipMemcpyAsync(a, src, g.n() * 4, hipMemcpyDeviceToDevice, c->stream));
+        src = a;
+    }
+    for (int k = 0; k < np; ++k) {
+        ProfScope ps(c, P_DCT);
+        const AxisTables& t = c->axes[axes[k]];
+        const bool last = k == np - 1;
+        float* out = last ? dst : (k == 0 ? a : b);
+        const float scale = !last ? 1.0f : inverse ? float(1.0 / (double(g.n()) * 8.0)) : 8.0f;
+        const int fuse = (last && !inverse && poisson_flags >= 0) ? 1 : 0;
+        const int quirk = (poisson_flags > 0 && (poisson_flags & AMB_FLAG_POISSON_INDEX_QUIRK)) ? 1 : 0;
+        const void* table = precision == AMB_DCT_F32
+                                ? static_cast<const void*>(inverse ? t.inv32 : t.fwd32)
+                                : static_cast<const void*>(inverse ? t.inv_split : t.fwd_split);
+        AMB_HIP(launch_dct_mfma_pass(c->stream, src, out, table, g, axes[k], scale, precision,
+                                     c->axes[0].eig, c->axes[1].eig, c->axes[2].eig, fuse, quirk));
+        src = out;
     }
     return AMB_OK;
 }
 
 amb_status poisson(amb_context* c, const float* in, float* out, uint32_t flags) {
-    AMB_TRY(ensure_tables(c, c->g));
+    AMB_TRY(ensure_tables(c, c->g, -1));
     ProfScope ps(c, P_POISSON);
     AMB_HIP(launch_poisson_divide(c->stream, in, out, c->axes[0].eig, c->axes[1].eig,
                                   c->axes[2].eig, c->g, (flags & AMB_FLAG_POISSON_INDEX_QUIRK) ? 1 : 0));
     return AMB_OK;
 }
 
-// l = iDCT(P(DCT(B-div(vx, vy, vz)))) into scratch[1]; vx.. are device FP32.
+// dst = iDCT(P(DCT(B-div(vx, vy, vz)))); vx.. and dst are device FP32.  dst may
+// be one of vx.. (they are read before it is written) or scratch[1], no other
+// scratch volume of the first three.
 amb_status integrate(amb_context* c, const float* vx, const float* vy, const float* vz,
-                     int precision, uint32_t flags, float** result) {
+                     int precision, uint32_t flags, float* dst) {
     float* s0 = c->scratch[0];
     float* s1 = c->scratch[1];
     float* s2 = c->scratch[2];
@@ -1080,15 +1095,14 @@ amb_status integrate(amb_context* c, const float* vx, const float* vy, const flo
         AMB_HIP(launch_divergence(c->stream, vx, vy, vz, s0, c->g));
     }
     if (precision == AMB_DCT_REFERENCE) {
-        AMB_TRY(transform3(c, s0, s1, s2, 0, precision));  // DCT -> s2
-        AMB_TRY(poisson(c, s2, s0, flags));                 // -> s0
-        AMB_TRY(transform3(c, s0, s2, s1, 1, precision));  // iDCT -> s1
+        AMB_TRY(transform3(c, s0, s1, s2, s0, 0, precision));   // DCT -> s0
+        AMB_TRY(poisson(c, s0, s1, flags));                     // -> s1
+        AMB_TRY(transform3(c, s1, s2, s0, dst, 1, precision));  // iDCT
     } else {
-        // eigenvalue divide fused into the forward z pass
-        AMB_TRY(transform3(c, s0, s1, s2, 0, precision, int(flags & AMB_FLAG_POISSON_INDEX_QUIRK)));
-        AMB_TRY(transform3(c, s2, s0, s1, 1, precision));  // iDCT -> s1
+        // eigenvalue divide fused into the last forward pass
+        AMB_TRY(transform3(c, s0, s1, s2, s0, 0, precision, int(flags & AMB_FLAG_POISSON_INDEX_QUIRK)));
+        AMB_TRY(transform3(c, s0, s2, s0, dst, 1, precision));  // iDCT
     }
-    *result = s1;
     return AMB_OK;
 }
 
@@ -1485,9 +1499,14 @@ static amb_status transform_entry(amb_context* c, amb_memory mem, const float* i
     if (!c || !image || !out) return fail(AMB_ERR_INVALID_ARGUMENT, "NULL argument");
     if (precision > 2) return fail(AMB_ERR_INVALID_ARGUMENT, "unknown dct_precision");
     AMB_TRY(geometry_only(c, w, h, d));
-    AMB_HIP(hipMemcpyAsync(c->scratch[0], image, c->g.n() * 4, kind_in(mem), c->stream));
-    AMB_TRY(transform3(c, c->scratch[0], c->scratch[1], c->scratch[2], inverse, int(precision)));
-    AMB_TRY(copy_out(c, mem, out, c->scratch[2]));
+    if (mem == AMB_MEM_DEVICE) {
+        AMB_TRY(transform3(c, image, c->scratch[0], c->scratch[1], out, inverse, int(precision)));
+    } else {
+        AMB_HIP(hipMemcpyAsync(c->scratch[0], image, c->g.n() * 4, kind_in(mem), c->stream));
+        AMB_TRY(transform3(c, c->scratch[0], c->scratch[1], c->scratch[2], c->scratch[0], inverse,
+                           int(precision)));
+        AMB_TRY(copy_out(c, mem, out, c->scratch[0]));
+    }
     AMB_HIP(hipStreamSynchronize(c->stream));
     return AMB_OK;
 }
@@ -1531,9 +1550,10 @@ AMB_API amb_status amb_integrate_gradients_poisson(amb_context* c, amb_memory me
     AMB_TRY(geometry_only(c, w, h, d));
     const float* v[3];
     AMB_TRY(stage3(c, mem, vx, vy, vz, v));
-    float* l = nullptr;
-    AMB_TRY(integrate(c, v[0], v[1], v[2], int(precision), flags, &l));
-    AMB_TRY(copy_out(c, mem, shading, l));
+    // a device result is written by the last pass itself
+    float* l = mem == AMB_MEM_DEVICE ? shading : c->scratch[1];
+    AMB_TRY(integrate(c, v[0], v[1], v[2], int(precision), flags, l));
+    if (mem != AMB_MEM_DEVICE) AMB_TRY(copy_out(c, mem, shading, l));
     AMB_HIP(hipStreamSynchronize(c->stream));
     return AMB_OK;
 } catch (...) {
@@ -1582,8 +1602,8 @@ static amb_status deshade_tail(amb_context* c, amb_memory mem, const float* mask
             v[k] = c->scratch[2 + k];
         }
     }
-    float* l = nullptr;
-    AMB_TRY(integrate(c, v[0], v[1], v[2], int(precision), flags, &l));   // l in scratch[1]
+    float* l = c->scratch[1];
+    AMB_TRY(integrate(c, v[0], v[1], v[2], int(precision), flags, l));
     // u as FP32 (scratch[2] for BF16), mask into scratch[3], r into scratch[4]
     const float* uf = static_cast<const float*>(c->fields[F_U]);
     if (c->storage == 1) {

@@ -33,25 +33,50 @@ __device__ __forceinline__ void axis_info(const Geometry& g, int axis, size_t& s
 
 // A14: g = (B_x v_x + B_y v_y) + B_z v_z (B_z only when depth > 1),
 // B a = -a[i] + a[i-1], -a[0] at i = 0 (tgv_cuda/tgv_common.cu:133-197).
-__global__ void divergence_kernel(const float* __restrict__ vx, const float* __restrict__ vy,
-                                  const float* __restrict__ vz, float* __restrict__ out,
-                                  Geometry g) {
-    const size_t n = g.n();
-    const size_t plane = size_t(g.w) * g.h;
-    const size_t stride = size_t(gridDim.x) * blockDim.x;
-    for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
-        const int x = int(i % g.w);
-        const int y = int((i / g.w) % g.h);
-        const int z = int(i / plane);
-        const float bx = x > 0 ? -vx[i] + vx[i - 1] : -vx[i];
-        const float by = y > 0 ? -vy[i] + vy[i - g.w] : -vy[i];
-        float r = bx + by;
-        if (g.d > 1) {
-            const float bz = z > 0 ? -vz[i] + vz[i - plane] : -vz[i];
-            r = r + bz;
+// Bound by HBM (three fields read, one written; the y and z neighbours come from
+// L2 and the Infinity Cache): VX = 4 consecutive voxels per thread where the rows
+// and pointers allow 16-byte accesses, 32-bit indices, and a launch order that
+// gives each XCD a contiguous range of rows.
+template <int VX>
+__global__ __launch_bounds__(256) void divergence_kernel(const float* __restrict__ vx,
+                                                         const float* __restrict__ vy,
+                                                         const float* __restrict__ vz,
+                                                         float* __restrict__ out, Geometry g) {
+    const uint32_t W = uint32_t(g.w), H = uint32_t(g.h), plane = W * H, lanes = W / VX;
+    const uint32_t e = xcd_contiguous(blockIdx.x, gridDim.x) * 256u + threadIdx.x;
+    const uint32_t row = e / lanes;
+    const uint32_t z = row / H, y = row - z * H, x = (e - row * lanes) * VX;
+    if (z >= uint32_t(g.d)) return;
+    const uint32_t i = row * W + x;
+    auto ld = [](const float* p, uint32_t k, float (&v)[VX]) {
+        if constexpr (VX == 4) {
+            const float4 t = *reinterpret_cast<const float4*>(p + k);
+            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+        } else {
+            v[0] = p[k];
         }
-        out[i] = r;
+    };
+    float a[VX], b[VX], c[VX], bn[VX], cn[VX], r[VX];
+    ld(vx, i, a);
+    ld(vy, i, b);
+    const float an = x > 0 ? vx[i - 1] : 0.0f;
+    if (y > 0) ld(vy, i - W, bn);
+    if (g.d > 1) {
+        ld(vz, i, c);
+        if (z > 0) ld(vz, i - plane, cn);
     }
+#pragma unroll
+    for (int k = 0; k < VX; ++k) {
+        const float bx = x + k > 0 ? -a[k] + (k ? a[k ? k - 1 : 0] : an) : -a[k];
+        const float by = y > 0 ? -b[k] + bn[k] : -b[k];
+        r[k] = bx + by;
+        if (g.d > 1) {
+            const float bz = z > 0 ? -c[k] + cn[k] : -c[k];
+            r[k] = r[k] + bz;
+        }
+    }
+    if constexpr (VX == 4) *reinterpret_cast<float4*>(out + i) = make_float4(r[0], r[1], r[2], r[3]);
+    else out[i] = r[0];
 }
 
 // A15/A17 in the reference's numerics: every output is its own sequence of
@@ -234,8 +259,14 @@ inline int elem_blocks(size_t n) {
 
 hipError_t launch_divergence(hipStream_t s, const float* vx, const float* vy, const float* vz,
                              float* out, Geometry g) {
-    hipLaunchKernelGGL(divergence_kernel, dim3(elem_blocks(g.n())), dim3(256), 0, s, vx, vy, vz,
-                       out, g);
+    const uintptr_t at = reinterpret_cast<uintptr_t>(vx) | reinterpret_cast<uintptr_t>(vy) |
+                         reinterpret_cast<uintptr_t>(out) |
+                         (g.d > 1 ? reinterpret_cast<uintptr_t>(vz) : 0);
+    const bool vec = g.w % 4 == 0 && at % 16 == 0;
+    const size_t threads = vec ? g.n() / 4 : g.n();
+    const dim3 grid{unsigned((threads + 255) / 256), 1, 1};
+    if (vec) hipLaunchKernelGGL(divergence_kernel<4>, grid, dim3(256), 0, s, vx, vy, vz, out, g);
+    else hipLaunchKernelGGL(divergence_kernel<1>, grid, dim3(256), 0, s, vx, vy, vz, out, g);
     return hipGetLastError();
 }
 
