@@ -4,12 +4,14 @@
 // itk::ResampleImageFilter with itk::BSplineInterpolateImageFunction (order 3).
 // The algorithm (M. Unser, "Splines: a perfect fit for signal and image
 // processing", IEEE SPM 1999, Box 2) in FP64:
-//   coefficients - per axis x, y, z (skipped for length 1), one thread per line
-//     (x: lines staged through LDS in chunks):
+//   coefficients - per axis x, y, z (skipped for length 1): lines kept in LDS
+//     whole where they are short enough, else one thread per line (x: lines
+//     staged through LDS in chunks):
 //     gain (1 - z)(1 - 1/z), pole z = sqrt(3) - 2, mirror-boundary causal start
 //     (18-term truncated sum for lines longer than 18, exact otherwise), causal
 //     and anticausal recursions;
-//   resampling  - one thread per output voxel: continuous input index
+//   resampling  - a thread per output column along z with the support in
+//     registers (output spacings up to 2.5), else per output voxel: continuous input index
 //     j * spacing per axis (spacing = 1 / (float(new) / float(old)), with the
 //     +2 geometry of ResizeProcessor's upsampling branch), 0 outside
 //     [-0.5, N - 0.5), the 4 x 4 x 4 cubic B-spline weights and mirrored
@@ -21,6 +23,7 @@
 // (and its not-masked form).
 #include "amb_internal.hpp"
 
+#include <algorithm>
 #include <cmath>
 
 namespace amb {
@@ -189,6 +192,105 @@ __global__ __launch_bounds__(XD_LINES) void spline3_decompose_x_kernel(double* _
     }
 }
 
+// The prefilter of lines that fit LDS: one wave per block loads LINES of them
+// (x: rows of the FP32 input, converted here; y and z: adjacent columns), one
+// lane each runs its line's recursions in LDS with the operations of
+// spline3_decompose_kernel in the same order, and the wave stores the
+// coefficients: one read and one write of the volume where the kernels above
+// read and write it twice.  Bound by the chains (two dependent FP64 operations
+// per sample and direction) of the lines that LDS holds at a time, so the
+// shorter the lines, the better: per pass of 67 M samples, x at 512 samples 908
+// (with the conversion to FP64, which the other kernel needs first) -> 624 us, y
+// at 512 samples 670 -> 480 us, z at 256 samples 410 -> 370 us.  Longer lines
+// (fewer than four blocks per CU) keep the other kernels.  Reading 16 samples
+// ahead into registers was slower (660, 580 and 390 us).
+constexpr long RESIDENT_ROW = 1024, RESIDENT_COLUMN = 512;
+
+template <int AXIS0>
+__global__ __launch_bounds__(64) void spline3_decompose_resident_kernel(
+    const float* __restrict__ in, double* __restrict__ c, Geometry g, int axis, int N,
+    uint32_t lines, Spline3Line sp) {
+    constexpr int LINES = AXIS0 ? 4 : 8;
+    extern __shared__ __align__(16) double rows[];   // [LINES][P]
+    const int P = N | 1, lane = int(threadIdx.x);
+    const uint32_t l0 = xcd_contiguous(blockIdx.x, gridDim.x) * LINES;
+    const uint32_t W = uint32_t(g.w), st = axis == 1 ? W : W * uint32_t(g.h);
+    // y and z: lane -> column lane % 8 of the group, samples lane / 8 + 8 k
+    const uint32_t l = l0 + uint32_t(lane & (LINES - 1));
+    const bool has = l < lines;
+    const uint32_t z0 = axis == 1 ? l / W : 0u;
+    const size_t base = axis == 1 ? size_t(z0) * W * uint32_t(g.h) + (l - z0 * W) : l;
+    if (AXIS0) {
+#pragma unroll
+        for (int r = 0; r < LINES; ++r) {
+            if (l0 + r >= lines) break;
+            const float* src = in + size_t(l0 + r) * N;
+#pragma unroll 4
+            for (int n = lane; n < N; n += 64) rows[r * P + n] = double(src[n]) * sp.gain;
+        }
+    } else if (has) {
+        double* dst = rows + (lane & (LINES - 1)) * P;
+#pragma unroll 8
+        for (int n = lane / LINES; n < N; n += 64 / LINES) dst[n] = c[base + size_t(n) * st] * sp.gain;
+    }
+    __syncthreads();
+    if (lane < LINES && has) {
+        double* const a = rows + lane * P;
+        const double z = sp.z;
+        double prev;
+        if (sp.horizon < N) {
+            double zn = z, sum = a[0];
+            for (long n = 1; n < sp.horizon; ++n) {
+                sum += zn * a[n];
+                zn *= z;
+            }
+            prev = sum;
+        } else {
+            double zn = z;
+            const double iz = 1.0 / z;
+            double z2n = sp.z2n0;
+            double sum = a[0] + z2n * a[N - 1];
+            z2n *= z2n * iz;
+            for (int n = 1; n <= N - 2; ++n) {
+                sum += (zn + z2n) * a[n];
+                zn *= z;
+                z2n *= iz;
+            }
+            prev = sum / (1.0 - zn * zn);
+        }
+        a[0] = prev;
+        double last = 0.0;
+#pragma unroll 8
+        for (int n = 1; n < N; ++n) {
+            const double v = a[n] + z * prev;
+            a[n] = v;
+            last = prev;
+            prev = v;
+        }
+        double next = sp.pole_factor * (z * last + prev);
+        a[N - 1] = next;
+#pragma unroll 8
+        for (int n = N - 2; n >= 0; --n) {
+            next = z * (next - a[n]);
+            a[n] = next;
+        }
+    }
+    __syncthreads();
+    if (AXIS0) {
+#pragma unroll
+        for (int r = 0; r < LINES; ++r) {
+            if (l0 + r >= lines) break;
+            double* dst = c + size_t(l0 + r) * N;
+#pragma unroll 4
+            for (int n = lane; n < N; n += 64) dst[n] = rows[r * P + n];
+        }
+    } else if (has) {
+        const double* src = rows + (lane & (LINES - 1)) * P;
+#pragma unroll 8
+        for (int n = lane / LINES; n < N; n += 64 / LINES) c[base + size_t(n) * st] = src[n];
+    }
+}
+
 // Whole-sample mirror about 0 and N - 1 (period 2N - 2); all 0 for N = 1.
 // (Volumes hold fewer than 2^31 voxels, so indices fit in int.)
 __device__ __forceinline__ int mirror_index(int k, int N) {
@@ -248,6 +350,88 @@ __global__ void spline3_resample_kernel(const double* __restrict__ c, Geometry g
     }
 }
 
+// The same samples for output spacings up to RESAMPLE_MARCH_SPACING along z: a
+// thread owns one (x, y) of the output and walks along z with the 4 x 16
+// coefficients of its support in registers, so a step of the support loads one
+// plane's 16 values instead of an output's 64 (a factor of 2 upwards: 8 loads per
+// output, downwards: 32).  Products and their order are spline3_resample_kernel's.
+// Bound by the FP64 pipe (208 operations per output, 0.41 ms of 67 M outputs at
+// the card's FP64 rate) where that one is bound by its gathers: 256 x 256 x 128 to
+// 512 x 512 x 256 in 600 us (2490), the other way in 205 us (420).  Loading the
+// next plane a step ahead does not fit the registers (70 spilled).  Beyond a
+// spacing of 2.5 most of the planes a walk would load serve one output only.
+constexpr double RESAMPLE_MARCH_SPACING = 2.5;
+
+__device__ __forceinline__ void spline3_weights(double x, int& i1, double (&wt)[4]) {
+    i1 = int(floor(x));
+    const double w = x - double(i1);
+    wt[3] = (1.0 / 6.0) * w * w * w;
+    wt[0] = (1.0 / 6.0) + 0.5 * w * (w - 1.0) - wt[3];
+    wt[2] = w + wt[0] - 2.0 * wt[3];
+    wt[1] = 1.0 - wt[0] - wt[2] - wt[3];
+}
+
+__global__ __launch_bounds__(256, 2) void spline3_resample_march_kernel(
+    const double* __restrict__ c, Geometry gi, float* __restrict__ out, Geometry go, double sp0,
+    double sp1, double sp2, int zchunk) {
+    const uint32_t OW = uint32_t(go.w), plane = OW * uint32_t(go.h);
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+    if (t >= plane) return;
+    const uint32_t oy = t / OW;
+    const double xx = double(t - oy * OW) * sp0, xy = double(oy) * sp1;
+    const bool inside = xx >= -0.5 && xx < double(gi.w) - 0.5 && xy >= -0.5 && xy < double(gi.h) - 0.5;
+    int ix, iy;
+    double wx[4], wy[4], wxy[16];
+    spline3_weights(xx, ix, wx);
+    spline3_weights(xy, iy, wy);
+    uint32_t ax[4], ay[4];   // the support's offsets in a plane (elements)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        ax[k] = inside ? uint32_t(mirror_index(ix - 1 + k, gi.w)) : 0u;
+        ay[k] = inside ? uint32_t(mirror_index(iy - 1 + k, gi.h)) * uint32_t(gi.w) : 0u;
+    }
+#pragma unroll
+    for (int k = 0; k < 16; ++k) wxy[k] = wx[k & 3] * wy[k >> 2];
+    const size_t ip = size_t(gi.w) * size_t(gi.h);
+    const int z0 = int(blockIdx.y) * zchunk, z1 = min(z0 + zchunk, go.d);
+    double p[4][16];   // planes base - 1 .. base + 2
+    auto load = [&](int z, double (&v)[16]) {
+        const double* src = c + size_t(mirror_index(z, gi.d)) * ip;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = *elem(src, ay[k >> 2] + ax[k & 3]);
+    };
+    int base = __builtin_amdgcn_readfirstlane(int(floor(double(z0) * sp2)));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) load(base - 1 + k, p[k]);
+    for (int oz = z0; oz < z1; ++oz) {
+        const double z = double(oz) * sp2;
+        int i1;
+        double wz[4];
+        spline3_weights(z, i1, wz);
+        i1 = __builtin_amdgcn_readfirstlane(i1);
+        while (base < i1) {
+            ++base;
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                p[0][k] = p[1][k];
+                p[1][k] = p[2][k];
+                p[2][k] = p[3][k];
+            }
+            load(base + 2, p[3]);
+        }
+        double acc = 0.0;
+#pragma unroll
+        for (int k2 = 0; k2 < 4; ++k2)
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                acc += wxy[k] * wz[k2] * p[k2][k];
+                if (k % 4 == 3) __builtin_amdgcn_sched_barrier(0);   // few products in flight
+            }
+        const bool in = inside && z >= -0.5 && z < double(gi.d) - 0.5;
+        out[size_t(oz) * plane + t] = in ? float(acc) : 0.0f;
+    }
+}
+
 // TGVKDeshadeDownsampledProcessor.cpp:107-126 (masked_variant) and
 // TGVKDeshadeDownsampledNotMaskedProcessor.cpp:103-116: r = f' - l with f' the
 // masked input (masked variant) or the input; with a mask l (masked variant)
@@ -294,27 +478,40 @@ inline int grid_for(size_t n) {
 hipError_t launch_resize_spline3(hipStream_t s, const float* in, Geometry gi, double* coef,
                                  float* out, Geometry go) {
     const size_t n = gi.n();
-    hipLaunchKernelGGL(to_double_kernel, dim3(grid_for(n)), dim3(256), 0, s, in, coef, n);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
     Spline3Line sp;
     sp.z = std::sqrt(3.0) - 2.0;
     sp.gain = (1.0 - sp.z) * (1.0 - 1.0 / sp.z);
     sp.pole_factor = sp.z / (sp.z * sp.z - 1.0);
     sp.horizon = long(std::ceil(std::log(1e-10) / std::log(std::fabs(sp.z))));
     const long ext[3] = {gi.w, gi.h, gi.d};
+    hipError_t e = hipSuccess;
     for (int axis = 0; axis < 3; ++axis) {
         const long N = ext[axis];
-        if (N == 1) continue;
-        sp.z2n0 = std::pow(sp.z, double(N - 1));
-        const long lines = long(n) / N;
-        if (axis == 0)
-            hipLaunchKernelGGL(spline3_decompose_x_kernel,
-                               dim3(unsigned((lines + XD_LINES - 1) / XD_LINES)), dim3(XD_LINES), 0,
-                               s, coef, N, lines, sp);
-        else
-            hipLaunchKernelGGL(spline3_decompose_kernel, dim3(unsigned((lines + 255) / 256)),
-                               dim3(256), 0, s, coef, gi, axis, lines, sp);
+        const int group = axis == 0 ? 4 : 8;   // lines per block of the resident kernel
+        const size_t lds = size_t(group) * size_t(N | 1) * 8;
+        const bool resident = N > 1 && N <= (axis == 0 ? RESIDENT_ROW : RESIDENT_COLUMN);
+        if (axis == 0 && !resident)
+            hipLaunchKernelGGL(to_double_kernel, dim3(grid_for(n)), dim3(256), 0, s, in, coef, n);
+        if (N > 1) {
+            sp.z2n0 = std::pow(sp.z, double(N - 1));
+            const long lines = long(n) / N;
+            if (resident) {
+                const dim3 grid{unsigned((lines + group - 1) / group), 1, 1};
+                if (axis == 0)
+                    hipLaunchKernelGGL(spline3_decompose_resident_kernel<1>, grid, dim3(64), lds, s,
+                                       in, coef, gi, axis, int(N), uint32_t(lines), sp);
+                else
+                    hipLaunchKernelGGL(spline3_decompose_resident_kernel<0>, grid, dim3(64), lds, s,
+                                       in, coef, gi, axis, int(N), uint32_t(lines), sp);
+            } else if (axis == 0) {
+                hipLaunchKernelGGL(spline3_decompose_x_kernel,
+                                   dim3(unsigned((lines + XD_LINES - 1) / XD_LINES)), dim3(XD_LINES),
+                                   0, s, coef, N, lines, sp);
+            } else {
+                hipLaunchKernelGGL(spline3_decompose_kernel, dim3(unsigned((lines + 255) / 256)),
+                                   dim3(256), 0, s, coef, gi, axis, lines, sp);
+            }
+        }
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -323,6 +520,18 @@ hipError_t launch_resize_spline3(hipStream_t s, const float* in, Geometry gi, do
     const long geo[3] = {long(go.w) + pad, long(go.h) + pad, long(go.d) + pad};
     double spacing[3];
     for (int a = 0; a < 3; ++a) spacing[a] = 1.0 / double(float(geo[a]) / float(ext[a]));
+    if (spacing[2] <= RESAMPLE_MARCH_SPACING && size_t(gi.w) * size_t(gi.h) * 8 < (size_t(1) << 32)) {
+        // z chunks of 64 outputs or fewer (each loads four planes to begin with), for
+        // about 4096 blocks where the volume has them
+        const unsigned blocks = unsigned((size_t(go.w) * size_t(go.h) + 255) / 256);
+        const int want = int(std::min<size_t>(4096 / blocks + 1, 65535));
+        const int zc = std::max((go.d + 65534) / 65535,
+                                std::max(8, std::min(64, (go.d + want - 1) / want)));
+        hipLaunchKernelGGL(spline3_resample_march_kernel,
+                           dim3(blocks, unsigned((go.d + zc - 1) / zc)), dim3(256), 0, s, coef, gi,
+                           out, go, spacing[0], spacing[1], spacing[2], zc);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(spline3_resample_kernel, dim3(grid_for(go.n())), dim3(256), 0, s, coef, gi,
                        out, go, spacing[0], spacing[1], spacing[2]);
     return hipGetLastError();

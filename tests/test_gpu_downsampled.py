@@ -55,6 +55,22 @@ def test_resize_bitwise_against_oracle(ctx, orc, src, dst):
     np.testing.assert_array_equal(got, orc.resize_spline3(a, dst))
 
 
+# the column walk and its limits (output spacings along z of 1/3 .. 2.5 and beyond:
+# 64 outputs per z chunk and one more, one plane, 2.5 exactly), and the lines the
+# prefilter keeps in LDS (rows of up to 1024 samples, columns of up to 512; blocks
+# of 4 rows and of 8 columns, partial ones among them)
+@pytest.mark.parametrize("src,dst", [((22, 9, 10), (65, 20, 21)), ((130, 6, 7), (66, 5, 6)),
+                                     ((10, 5, 6), (4, 5, 6)), ((11, 5, 6), (4, 5, 6)),
+                                     ((40, 6, 5), (8, 3, 3)), ((1, 5, 1024), (1, 5, 513)),
+                                     ((1, 5, 1025), (1, 5, 600)), ((2, 512, 9), (2, 256, 9)),
+                                     ((2, 513, 9), (2, 257, 9)), ((513, 3, 11), (257, 3, 11)),
+                                     ((512, 3, 11), (600, 4, 12)), ((20, 1, 1), (41, 1, 1))])
+def test_resize_walk_and_resident_lines(ctx, orc, src, dst):
+    _say("resize", src, "->", dst)
+    a = (np.random.default_rng(7).standard_normal(src) + 1.0).astype(np.float32)
+    np.testing.assert_array_equal(ctx.resize_bspline3(a, dst), orc.resize_spline3(a, dst))
+
+
 def test_resize_extents_match(orc):
     from ambient_image_processor_amd import native
     for shape, factor in (((256, 256, 256), 0.5), ((1, 100, 101), 0.3), ((3, 10, 10), 0.01),
