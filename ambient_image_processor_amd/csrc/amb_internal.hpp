@@ -288,25 +288,24 @@ hipError_t launch_tgvk_dual(hipStream_t s, float* const* fields_dev, float* cons
 hipError_t launch_tgvk_primal(hipStream_t s, float* const* fields_dev, float* const* levels_dev,
                               const float* f, const uint8_t* active, Geometry g, int levels,
                               float tau, float lambda, float theta, const PlanOverrides& ov);
-// Fused TGV-k sweep for one level (k = 3): primal half of iteration k and
-// dual half of iteration k + 1, reading the 25 fields `src` (order u, vx, vy,
-// vz, px, py, pz, qxx, qyy, qzz, qxy, qxz, qyz, wx, wy, wz, wxy, wxz, wyz, rx,
-// ry, rz, rxy, rxz, ryz) and writing the same fields to `dst`; u_bar, v_bar
-// and w_bar are neither read nor written.  dst[k] - src[k] must be the same
-// for the first 13 fields and the same for the last 12.  alpha: the three
-// weights (host).
+// Fused TGV-k sweep for one or two levels (k = 3, 4): primal half of
+// iteration k and dual half of iteration k + 1, reading one copy of the state and
+// writing the other; u_bar, v_bar and w_bar are neither read nor written.  t: the
+// copy's 17-field block (state layout, field_stride bytes apart); lv: its level
+// block (18 fields per level: w[6], w_bar[6], r[6]); the destination copies lie dt
+// and dl bytes further on.  alpha: the levels + 2 weights (host).
 struct TgvkFusedPlan {
     int tx;       // owned x columns per block (W: whole rows)
     int ty;       // owned y rows per block
     int zchunk;   // planes per block
 };
-constexpr int N_TGVK_FUSED_FIELDS = 25;
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan);
-hipError_t launch_tgvk_fused(hipStream_t s, const float* const* src, float* const* dst,
-                             const float* f, const uint8_t* active, Geometry g, float tau,
-                             float sigma, float lambda, float theta, const float* alpha,
-                             int planar, const TgvkFusedPlan& plan);
+hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_t field_stride,
+                             ptrdiff_t dt, ptrdiff_t dl, const float* f, const uint8_t* active,
+                             Geometry g, int levels, float tau, float sigma, float lambda,
+                             float theta, const float* alpha, int planar,
+                             const TgvkFusedPlan& plan);
 
 // Cubic B-spline resampling (resize.hip): in (gi) to out (go, the kept voxels);
 // coef: gi.n() doubles of scratch.

@@ -154,11 +154,11 @@ struct amb_context {
     std::vector<float*> klv_host;
     std::vector<float> kalpha_host;
     int klevels = 0;
-    // fused TGV-k sweep (one level): second copy of w_0 and r_0 (grow-only),
-    // the launch plan
+    // fused TGV-k sweep (one or two levels): second copy of the w and r fields
+    // (grow-only; level-block layout), the launch plan
     char* kalt_block = nullptr;
     size_t kalt_cap = 0;
-    float* kalt[12] = {};
+    std::vector<float*> kalt;       // 12 per level
     char* kalt13_block = nullptr;   // its own second copy of the 13 TGV2 fields
     size_t kalt13_cap = 0;
     void* kalt13[N_FUSED_FIELDS] = {};
@@ -854,15 +854,17 @@ amb_status tgvk_begin(amb_context* c, amb_memory mem, const float* f, uint32_t w
     return AMB_OK;
 }
 
-// Level-table slots of w_0 (0..5) and r_0 (12..17), the level fields the
-// fused TGV-k sweep ping-pongs; c->kalt[m] is the other copy of slot KLV_PING[m].
+// Level-table slots of a level's w (0..5) and r (12..17), the level fields the
+// fused TGV-k sweep ping-pongs; c->kalt[12 l + m] is the other copy of level l's
+// slot KLV_PING[m].
 constexpr int KLV_PING[12] = {0, 1, 2, 3, 4, 5, 12, 13, 14, 15, 16, 17};
 
-// The fused TGV-k sweep reaches every destination as its source pointer plus
-// one distance per buffer (25 destination pointers would not fit the scalar
-// registers), so its second copies mirror the first copies' layouts: the 13
-// TGV2 fields in a block of the state block's layout (the u_bar and v_bar
-// slots unused), the level fields in a block of the level block's layout.
+// The fused TGV-k sweep reaches every field at a multiple of the field stride
+// from its block and every destination one distance per block further on (up to
+// 37 source and 37 destination pointers would not fit the scalar registers), so
+// its second copies mirror the first copies' layouts: the 13 TGV2 fields in a
+// block of the state block's layout (the u_bar and v_bar slots unused), the level
+// fields in a block of the level block's layout.
 // (Measured on MI355X at 256^3, same box: 808 us per launch this way; 829 us
 // with each field's second copy in the slot of another field, which the TGV2
 // sweep prefers - see ensure_alt.)
@@ -890,11 +892,13 @@ amb_status ensure_kalt13(amb_context* c) {
 
 amb_status ensure_kalt(amb_context* c) {
     const size_t fstride = align_up(c->g.n() * 4, 256);
-    const size_t need = fstride * 18;
-    auto main_at = [&](int j) { return reinterpret_cast<float*>(c->kblock + size_t(j) * fstride); };
+    const size_t need = fstride * 18 * size_t(c->klevels);
+    auto main_at = [&](size_t j) { return reinterpret_cast<float*>(c->kblock + j * fstride); };
+    const size_t np = 12 * size_t(c->klevels);
+    auto slot = [&](size_t m) { return m / 12 * 18 + size_t(KLV_PING[m % 12]); };
     if (need > c->kalt_cap) {
-        for (int m = 0; m < 12; ++m)   // state must be in the level block
-            if (c->klv_host[KLV_PING[m]] != main_at(KLV_PING[m]))
+        for (size_t m = 0; m < np; ++m)   // state must be in the level block
+            if (c->klv_host[slot(m)] != main_at(slot(m)))
                 return fail(AMB_ERR_NOT_SUPPORTED, "fused TGV-k buffers out of step with the state");
         if (c->kalt_block) AMB_HIP(hipFree(c->kalt_block));
         c->kalt_block = nullptr;
@@ -902,9 +906,10 @@ amb_status ensure_kalt(amb_context* c) {
         AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->kalt_block), need));
         c->kalt_cap = need;
     }
-    for (int m = 0; m < 12; ++m) {
-        const int j = KLV_PING[m];
-        float* a = reinterpret_cast<float*>(c->kalt_block + size_t(j) * fstride);
+    c->kalt.resize(np);
+    for (size_t m = 0; m < np; ++m) {
+        const size_t j = slot(m);
+        float* a = reinterpret_cast<float*>(c->kalt_block + j * fstride);
         c->kalt[m] = c->klv_host[j] == main_at(j) ? a : main_at(j);
     }
     return AMB_OK;
@@ -913,31 +918,35 @@ amb_status ensure_kalt(amb_context* c) {
 // Primal half of TGV-k iteration k + dual half of iteration k + 1 into the
 // second copies, then swap the copies in the host tables.
 amb_status tgvk_fused_step(amb_context* c) {
-    const float* src[N_TGVK_FUSED_FIELDS];
-    float* dst[N_TGVK_FUSED_FIELDS];
+    const size_t fstride = align_up(c->g.n() * 4, 256);
+    const size_t np = 12 * size_t(c->klevels);
+    // the copies' blocks, from one field of each; every other field must lie in its
+    // place there (ensure_kalt13, ensure_kalt)
+    const char* t = static_cast<const char*>(c->fields[FUSED_FIELD_MAP[0]]) -
+                    size_t(FUSED_FIELD_MAP[0]) * fstride;
+    const char* td = static_cast<const char*>(c->kalt13[0]) - size_t(FUSED_FIELD_MAP[0]) * fstride;
+    const char* lv = reinterpret_cast<const char*>(c->klv_host[0]);
+    const char* ld = reinterpret_cast<const char*>(c->kalt[0]);
+    bool ok = true;
     for (int k = 0; k < N_FUSED_FIELDS; ++k) {
-        src[k] = static_cast<const float*>(c->fields[FUSED_FIELD_MAP[k]]);
-        dst[k] = static_cast<float*>(c->kalt13[k]);
+        const size_t off = size_t(FUSED_FIELD_MAP[k]) * fstride;
+        ok = ok && c->fields[FUSED_FIELD_MAP[k]] == t + off && c->kalt13[k] == td + off;
     }
-    for (int m = 0; m < 12; ++m) {
-        src[N_FUSED_FIELDS + m] = c->klv_host[KLV_PING[m]];
-        dst[N_FUSED_FIELDS + m] = c->kalt[m];
+    for (size_t m = 0; m < np; ++m) {
+        const size_t j = m / 12 * 18 + size_t(KLV_PING[m % 12]);
+        ok = ok && reinterpret_cast<const char*>(c->klv_host[j]) == lv + j * fstride &&
+             reinterpret_cast<const char*>(c->kalt[m]) == ld + j * fstride;
     }
-    // every field's other copy lies at one distance per block (ensure_kalt13, ensure_kalt)
-    for (int k = 1; k < N_TGVK_FUSED_FIELDS; ++k) {
-        const int k0 = k < N_FUSED_FIELDS ? 0 : N_FUSED_FIELDS;
-        if (reinterpret_cast<const char*>(dst[k]) - reinterpret_cast<const char*>(src[k]) !=
-            reinterpret_cast<const char*>(dst[k0]) - reinterpret_cast<const char*>(src[k0]))
-            return fail(AMB_ERR_NOT_SUPPORTED, "fused TGV-k buffers out of step with the state");
-    }
+    if (!ok) return fail(AMB_ERR_NOT_SUPPORTED, "fused TGV-k buffers out of step with the state");
     {
         ProfScope ps(c, P_TGVK_FUSED);
-        AMB_HIP(launch_tgvk_fused(c->stream, src, dst, c->f, c->sp.active, c->g, c->sp.tau,
-                                  c->sp.sigma, c->sp.lambda, c->sp.theta, c->kalpha_host.data(),
-                                  c->sp.planar, c->kfplan));
+        AMB_HIP(launch_tgvk_fused(c->stream, t, lv, fstride, td - t, ld - lv, c->f, c->sp.active,
+                                  c->g, c->klevels, c->sp.tau, c->sp.sigma, c->sp.lambda,
+                                  c->sp.theta, c->kalpha_host.data(), c->sp.planar, c->kfplan));
     }
     for (int k = 0; k < N_FUSED_FIELDS; ++k) std::swap(c->fields[FUSED_FIELD_MAP[k]], c->kalt13[k]);
-    for (int m = 0; m < 12; ++m) std::swap(c->klv_host[KLV_PING[m]], c->kalt[m]);
+    for (size_t m = 0; m < np; ++m)
+        std::swap(c->klv_host[m / 12 * 18 + size_t(KLV_PING[m % 12])], c->kalt[m]);
     return AMB_OK;
 }
 
@@ -954,7 +963,7 @@ amb_status tgvk_upload_tables(amb_context* c) {
 
 // The TGV-k loop: per iteration one dual launch (p, q, every r_i) and one
 // primal launch (u, v, every w_i); callback rule as in run().  With the fused
-// sweep (one level) the loop runs dual_0, fused(primal_k + dual_k+1) for
+// sweep (one or two levels) the loop runs dual_0, fused(primal_k + dual_k+1) for
 // k = 0 .. N - 2, primal_N-1, and an observed iteration ends with the primal
 // launch alone, exactly as run() does for TGV2.  The dual and primal launches
 // read the state through the device tables, which are brought up to date

@@ -29,6 +29,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace amb {
 namespace {
@@ -638,76 +639,85 @@ __global__ __launch_bounds__(KT) void tgvk_primal_fixed(
 }
 
 // ---------------------------------------------------------------------------
-// Fused sweep for one level (k = 3): the primal half of iteration k (u, v, w)
-// and the dual half of iteration k + 1 (p, q, r) in one z-march, with the
-// per-voxel arithmetic of tgvk_primal_fixed<1> and tgvk_dual_fixed<1> in the
-// same order.
+// Fused sweep for L = 1 or 2 levels (k = L + 2): the primal half of iteration
+// k (u, v, every w) and the dual half of iteration k + 1 (p, q, every r) in one
+// z-march, with the per-voxel arithmetic of tgvk_primal_fixed<L> and
+// tgvk_dual_fixed<L> in the same order.
 //
-// The dual half at a voxel reads u_bar at its +x, +y, +z neighbours and
-// v_bar, w_bar at its -x, -y, -z neighbours, i.e. primal results of
-// neighbouring voxels.  A block owns a tile of `tx` x columns (one voxel per
-// thread; tx = W: whole rows) and `ty` y rows; it computes the primal half
-// also on one column left and right of the tile (tx < W), one row above and
-// below it and one plane before and after its z chunk, and runs the dual half
-// one plane behind the primal half, so u_bar, v_bar and w_bar never leave the
-// CU.  Neighbouring blocks recompute the halo rows from the same
-// inputs, so the iteration state is read from one copy (src) and written to
-// another (dst).  Per voxel-iteration: reads u, f, v x3, p x3, q x6, w x6,
-// r x6 = 26, writes u, v x3, p x3, q x6, w x6, r x6 = 25: 51 element accesses
-// (204 B) instead of the 86 (344 B) of the two launches.
+// The dual half at a voxel reads u_bar and the odd levels' w_bar (G forward) at
+// its +x, +y, +z neighbours, v_bar and the even levels' w_bar (G backward) at its
+// -x, -y, -z neighbours, i.e. primal results of neighbouring voxels.  A block owns
+// a tile of `tx` x columns (one voxel per thread; tx = W: whole rows) and `ty` y
+// rows; it computes the primal half also on one column left and right of the
+// tile (tx < W), one row above and below it and one plane before and after its z
+// chunk, and runs the dual half one plane behind the primal half, so u_bar, v_bar
+// and w_bar never leave the CU.  Neighbouring blocks recompute the halo rows from
+// the same inputs, so the iteration state is read from one copy (src) and written
+// to another (dst).  Per voxel-iteration: reads u, f, v x3, p x3, q x6 and w x6,
+// r x6 per level, writes all of them but f: 27 + 24 L element accesses (204, 300 B)
+// instead of the two launches' 44 + 42 L (344, 512 B).
 //
 // Thread (c, r) holds y = y0 - 1 + r and x = x0 - 1 + c (tiled) or x = c.
-// Rows 1..ty and columns 1..tx are owned; row and column 0 feed only v_bar and
-// w_bar (the dual half's backward differences), row ty + 1 and column tx + 1
-// only u_bar (its forward differences).  Step s computes the primal half at
-// plane s and the dual half at plane s - 1.
+// Rows 1..ty and columns 1..tx are owned; row and column 0 feed only v_bar and the
+// even w_bar (the dual half's backward differences), row ty + 1 and column tx + 1
+// only u_bar and the odd w_bar (its forward differences).  Step s computes the
+// primal half at plane s and the dual half at plane s - 1.
 //
 // LDS arrays (one float per thread each): P region, plane s, the dual fields whose x
 // or y neighbours the primal half reads; D region, plane s - 1, u_bar, v_bar
-// and w_bar.  z neighbours stay in registers: p_z and the dual fields of
-// plane s - 1, q and r z-components of plane s + 1 (loaded one plane ahead),
-// v_bar and w_bar z-components of plane s - 2.
+// and w_bar.  z neighbours stay in registers: the dual fields of plane s - 1
+// (backward differences of p_z and the odd levels), q and even r z-components of
+// plane s + 1 (loaded one plane ahead), v_bar and even w_bar z-components of plane
+// s - 2; u_bar and odd w_bar at plane s are the ones just computed.
+//
+// Bound by HBM (one level moves 4.5 TB/s of its 204 B per voxel at 256^3, two levels
+// 3.4 TB/s of 300 B); both sides measured in tgvk_fused_plan's comment.
 // ---------------------------------------------------------------------------
-enum KFusedField { KF_U = 0, KF_VX, KF_VY, KF_VZ, KF_PX, KF_PY, KF_PZ, KF_QXX, KF_QYY, KF_QZZ,
-                   KF_QXY, KF_QXZ, KF_QYZ, KF_WX, KF_WY, KF_WZ, KF_WXY, KF_WXZ, KF_WYZ, KF_RX,
-                   KF_RY, KF_RZ, KF_RXY, KF_RXZ, KF_RYZ, N_KF };
-static_assert(N_KF == N_TGVK_FUSED_FIELDS, "fused TGV-k field count");
 
-// dst field k = src field k + dt bytes (k < 13) or + dl bytes (k >= 13): the
-// host lays the second copies out so, which keeps the 25 destination pointers
-// out of the scalar registers.
+// The 13 TGV2 fields lie at t + F_* fs, the level fields at lv + slot fs (slot 18
+// l + component for w, + 12 for r), their other copies dt and dl bytes further on:
+// the host lays both copies out so, which keeps up to 37 source and 37 destination
+// pointers out of the scalar registers (with a pointer per source field the
+// one-level form spilled more of them and took 782 us at 256^3, 767 now).
+constexpr int KFUSED_MAX_LEVELS = 2;
 
 struct KFusedFields {
-    const float* src[N_KF];
-    long long dt, dl;
+    const char* t;
+    const char* lv;
+    long long fs, dt, dl;
+    float alpha[KFUSED_MAX_LEVELS + 2];
 };
 
-enum KFusedRow { KR_PX = 0, KR_PY, KR_QXX, KR_QXY, KR_QYY, KR_QXZ, KR_QYZ, KR_RX, KR_RY, KR_RXY,
-                 KR_RXZ, KR_RYZ,                                            // P region
-                 KR_UB, KR_VBX, KR_VBY, KR_VBZ, KR_WBX, KR_WBY, KR_WBZ, KR_WBXY, KR_WBXZ,
-                 KR_WBYZ,                                                   // D region
-                 N_KROWS };
-constexpr int KFUSED_MAX_THREADS = 1024;
-
-template <class I>
-__device__ __forceinline__ float kf_ld(const float* p, I i) {
-    if constexpr (sizeof(I) == 4) return LDO(p, uint32_t(i) * 4u);
-    else return p[i];
-}
-template <class I>
-__device__ __forceinline__ void kf_st(float* p, I i, float v) {
-    if constexpr (sizeof(I) == 4)
-        __builtin_nontemporal_store(v, reinterpret_cast<float*>(reinterpret_cast<char*>(p) +
-                                                                uint32_t(i) * 4u));
-    else
-        __builtin_nontemporal_store(v, p + i);
+// LDS rows: P region p x, y; q xx, xy, yy, xz, yz; per level r x, y, xy, xz, yz;
+// D region u_bar; v_bar x3; per level w_bar x6
+constexpr int KR_PX = 0, KR_PY = 1, KR_QXX = 2, KR_QXY = 3, KR_QYY = 4, KR_QXZ = 5, KR_QYZ = 6;
+constexpr int KR_R = 7;
+template <int L>
+struct KRows {
+    static constexpr int UB = 7 + 5 * L, VB = UB + 1, WB = VB + 3, N = WB + 6 * L;
+};
+// Threads per block (register budgets of 128 and 168 per lane)
+template <int L>
+constexpr int kfused_threads() { return L == 1 ? 1024 : 768; }
+inline int kfused_max_threads(int levels) {
+    return levels == 1 ? kfused_threads<1>() : kfused_threads<2>();
 }
 
-template <class I, int MK>
-__global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
+template <class I>
+__device__ __forceinline__ float kf_ld(const char* p, I i) {
+    return *reinterpret_cast<const float*>(p + uint32_t(i) * 4u);
+}
+template <class I>
+__device__ __forceinline__ void kf_st(const char* p, I i, float v) {
+    __builtin_nontemporal_store(v, reinterpret_cast<float*>(const_cast<char*>(p) + uint32_t(i) * 4u));
+}
+
+template <int L, int MK>
+__global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
     KFusedFields ff, const float* __restrict__ f_, const uint8_t* __restrict__ act, Geometry g,
-    float tau, float sigma, float lambda, float theta, float a_p, float a_q, float a_r, int tx,
-    int ty, int zchunk, int planar) {
+    float tau, float sigma, float lambda, float theta, int tx, int ty, int zchunk, int planar) {
+    typedef uint32_t I;
+    typedef KRows<L> K;
     extern __shared__ __align__(16) float lds[];
     const int W = g.w, H = g.h, D = g.d;
     // tx < W: tiles of tx columns with one halo column on each side
@@ -722,7 +732,7 @@ __global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
     const int z0 = (tb / nb) * zchunk, z1 = min(z0 + zchunk, D);
     const int y = y0 - 1 + r;
     const bool in = y >= 0 && y < H && x >= 0 && x < W;
-    // column 0 feeds only v_bar and w_bar, column tx + 1 only u_bar (tiled)
+    // column 0 feeds only backward differences, column tx + 1 only forward ones (tiled)
     const bool cl = !tiled || c > 0, cr = !tiled || c < TXH - 1;
     const bool own = in && r >= 1 && r <= ty && cl && cr;
     const bool xp = x > 0, xn = x < W - 1, yp = y > 0, yn = y < H - 1;
@@ -731,75 +741,121 @@ __global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
     const float tl = tau * lambda;
     const int me = r * TXH + c;
     auto R = [&](int k) { return lds + k * RW; };
-    const float* const* src = ff.src;
-    auto dst = [&](int k) {
-        return reinterpret_cast<float*>(
-            const_cast<char*>(reinterpret_cast<const char*>(src[k])) +
-            (k < KF_WX ? ff.dt : ff.dl));
-    };
+    auto T = [&](int k) { return ff.t + k * ff.fs; };                       // TGV2 field F_*
+    auto LW = [&](int l, int k) { return ff.lv + (18 * l + k) * ff.fs; };   // w_l, component k
+    auto LR = [&](int l, int k) { return ff.lv + (18 * l + 12 + k) * ff.fs; };
 
     // D region starts at zero (read before its first write only into unused carries)
-    for (int k = int(threadIdx.x); k < (N_KROWS - KR_UB) * RW; k += int(blockDim.x))
-        lds[KR_UB * RW + k] = 0.f;
+    for (int k = int(threadIdx.x); k < (K::N - K::UB) * RW; k += int(blockDim.x))
+        lds[K::UB * RW + k] = 0.f;
 
-    float p_c[3], q_c[6], r_c[6];     // dual fields at plane s - 1
-    float qn[3], rn[3];               // q_zz, q_xz, q_yz and r_z, r_xz, r_yz at plane s
-    float vb_m2[3], wb_m2[3];         // v_bar, and w_bar z, xz, yz at plane s - 2
+    float p_c[3], q_c[6], r_c[L][6];    // dual fields at plane s - 1
+    float qn[3], rn[L][3];              // q_zz, q_xz, q_yz and even r_z, r_xz, r_yz at plane s
+    float vb_m2[3], wb_m2[L][3];        // v_bar, and even w_bar z, xz, yz at plane s - 2
 #pragma unroll
-    for (int k = 0; k < 3; ++k) p_c[k] = qn[k] = rn[k] = vb_m2[k] = wb_m2[k] = 0.f;
+    for (int k = 0; k < 3; ++k) p_c[k] = qn[k] = vb_m2[k] = 0.f;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) q_c[k] = r_c[k] = 0.f;
+    for (int k = 0; k < 6; ++k) q_c[k] = 0.f;
+#pragma unroll
+    for (int l = 0; l < L; ++l) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) r_c[l][k] = 0.f;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) rn[l][k] = wb_m2[l][k] = 0.f;
+    }
     bool act_c = true;
 
     const int zs = z0 > 0 ? z0 - 1 : 0;
     if (in && zs < D) {
         const I i = I(zs) * plane + col;
-        qn[0] = kf_ld(src[KF_QZZ], i); qn[1] = kf_ld(src[KF_QXZ], i); qn[2] = kf_ld(src[KF_QYZ], i);
-        rn[0] = kf_ld(src[KF_RZ], i); rn[1] = kf_ld(src[KF_RXZ], i); rn[2] = kf_ld(src[KF_RYZ], i);
+        qn[0] = kf_ld(T(F_QZZ), i); qn[1] = kf_ld(T(F_QXZ), i); qn[2] = kf_ld(T(F_QYZ), i);
+#pragma unroll
+        for (int l = 0; l < L; l += 2) {
+            rn[l][0] = kf_ld(LR(l, 2), i); rn[l][1] = kf_ld(LR(l, 4), i); rn[l][2] = kf_ld(LR(l, 5), i);
+        }
     }
 
     for (int s = zs; s <= z1; ++s) {
         const bool pin = s < D;
         const bool zn = s < D - 1;
         const I i = I(s) * plane + col;
-        // ---- loads at plane s (q and r z-components at s + 1)
+        // ---- loads at plane s (q and even r z-components at s + 1); r: x, y, xy and,
+        // odd levels, z, xz, yz
         float px = 0.f, py = 0.f, pz = 0.f, qxx = 0.f, qxy = 0.f, qyy = 0.f, u = 0.f, fv = 0.f;
-        float v[3] = {0.f, 0.f, 0.f}, qnn[3] = {0.f, 0.f, 0.f}, rnn[3] = {0.f, 0.f, 0.f};
-        float rx = 0.f, ry = 0.f, rxy = 0.f;
-        float w[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        float v[3] = {0.f, 0.f, 0.f}, qnn[3] = {0.f, 0.f, 0.f}, rnn[L][3];
+        float rl[L][6], w[L][6];   // r_l, w_l at plane s (component order x, y, z, xy, xz, yz)
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) rl[l][k] = w[l][k] = 0.f;
+#pragma unroll
+            for (int k = 0; k < 3; ++k) rnn[l][k] = 0.f;
+        }
         bool actv = true;
         if (in && pin) {
-            px = kf_ld(src[KF_PX], i); py = kf_ld(src[KF_PY], i); pz = kf_ld(src[KF_PZ], i);
-            qxx = kf_ld(src[KF_QXX], i); qxy = kf_ld(src[KF_QXY], i); qyy = kf_ld(src[KF_QYY], i);
-            u = kf_ld(src[KF_U], i); fv = kf_ld(f_, i);
+            px = kf_ld(T(F_PX), i); py = kf_ld(T(F_PY), i); pz = kf_ld(T(F_PZ), i);
+            qxx = kf_ld(T(F_QXX), i); qxy = kf_ld(T(F_QXY), i); qyy = kf_ld(T(F_QYY), i);
+            u = kf_ld(T(F_U), i);
+            fv = kf_ld(reinterpret_cast<const char*>(f_), i);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) v[k] = kf_ld(src[KF_VX + k], i);
-            rx = kf_ld(src[KF_RX], i); ry = kf_ld(src[KF_RY], i); rxy = kf_ld(src[KF_RXY], i);
+            for (int k = 0; k < 3; ++k) v[k] = kf_ld(T(F_VX + k), i);
 #pragma unroll
-            for (int k = 0; k < 6; ++k) w[k] = kf_ld(src[KF_WX + k], i);
+            for (int l = 0; l < L; ++l) {
+                rl[l][0] = kf_ld(LR(l, 0), i); rl[l][1] = kf_ld(LR(l, 1), i); rl[l][3] = kf_ld(LR(l, 3), i);
+                if (l & 1) {
+                    rl[l][2] = kf_ld(LR(l, 2), i); rl[l][4] = kf_ld(LR(l, 4), i);
+                    rl[l][5] = kf_ld(LR(l, 5), i);
+                }
+#pragma unroll
+                for (int k = 0; k < 6; ++k) w[l][k] = kf_ld(LW(l, k), i);
+            }
             if (zn) {
                 const I j = i + plane;
-                qnn[0] = kf_ld(src[KF_QZZ], j); qnn[1] = kf_ld(src[KF_QXZ], j);
-                qnn[2] = kf_ld(src[KF_QYZ], j);
-                rnn[0] = kf_ld(src[KF_RZ], j); rnn[1] = kf_ld(src[KF_RXZ], j);
-                rnn[2] = kf_ld(src[KF_RYZ], j);
+                qnn[0] = kf_ld(T(F_QZZ), j); qnn[1] = kf_ld(T(F_QXZ), j);
+                qnn[2] = kf_ld(T(F_QYZ), j);
+#pragma unroll
+                for (int l = 0; l < L; l += 2) {
+                    rnn[l][0] = kf_ld(LR(l, 2), j); rnn[l][1] = kf_ld(LR(l, 4), j);
+                    rnn[l][2] = kf_ld(LR(l, 5), j);
+                }
             }
             if (MK) actv = act[i] != 0;
         }
+#pragma unroll
+        for (int l = 0; l < L; l += 2) { rl[l][2] = rn[l][0]; rl[l][4] = rn[l][1]; rl[l][5] = rn[l][2]; }
 
         // ---- P region: plane s
         R(KR_PX)[me] = px; R(KR_PY)[me] = py;
         R(KR_QXX)[me] = qxx; R(KR_QXY)[me] = qxy; R(KR_QYY)[me] = qyy;
         R(KR_QXZ)[me] = qn[1]; R(KR_QYZ)[me] = qn[2];
-        R(KR_RX)[me] = rx; R(KR_RY)[me] = ry; R(KR_RXY)[me] = rxy;
-        R(KR_RXZ)[me] = rn[1]; R(KR_RYZ)[me] = rn[2];
+#pragma unroll
+        for (int l = 0; l < L; ++l) {
+            R(KR_R + 5 * l)[me] = rl[l][0]; R(KR_R + 5 * l + 1)[me] = rl[l][1];
+            R(KR_R + 5 * l + 2)[me] = rl[l][3]; R(KR_R + 5 * l + 3)[me] = rl[l][4];
+            R(KR_R + 5 * l + 4)[me] = rl[l][5];
+        }
         __syncthreads();
 
         // ---- primal half at plane s
-        const bool need_u = in && pin && r > 0 && cl && s >= z0;
-        const bool need_v = in && pin && r < RT - 1 && cr && s < z1;
-        float ubn = 0.f, vbn[3] = {0.f, 0.f, 0.f}, wbn[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        float uo = 0.f, vo[3], wo[6];
+        const bool need_u = in && pin && r > 0 && cl && s >= z0;        // u_bar, odd w_bar
+        const bool need_v = in && pin && r < RT - 1 && cr && s < z1;    // v_bar, even w_bar
+        float ubn = 0.f, vbn[3] = {0.f, 0.f, 0.f}, wbn[L][6];
+        float uo = 0.f, vo[3], wo[L][6];
+#pragma unroll
+        for (int l = 0; l < L; ++l)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) wbn[l][k] = 0.f;
+        const float q0[6] = {qxx, qyy, qn[0], qxy, qn[1], qn[2]};
+        // w_l from H(r_l) - q~ (tgv3_common.cu:362-405; q~ = q or r_{l-1})
+        auto update_w = [&](int l, const float (&h)[6]) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) {
+                float wn = fmaf(-tau, h[k] - (l == 0 ? q0[k] : rl[l > 0 ? l - 1 : 0][k]), w[l][k]);
+                if (MK && !actv) wn = w[l][k];
+                wo[l][k] = wn;
+                wbn[l][k] = fmaf(theta, wn - w[l][k], wn);
+            }
+        };
         if (need_u) {
             // u update, L1 prox, over-relaxation (tgv2_l1.cu:27-60)
             const float pxm = xp ? R(KR_PX)[me - 1] : 0.f;
@@ -816,6 +872,23 @@ __global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
             if (MK && !actv) un = u;
             uo = un;
             ubn = fmaf(theta, un - u, un);
+            // odd levels: H backward (tgv3_common.cu:265-309)
+#pragma unroll
+            for (int l = 1; l < L; l += 2) {
+                const int P = KR_R + 5 * l;
+                const float (&a)[6] = rl[l];
+                auto bwx = [&](int row, float o) { return xp ? -o + R(row)[me - 1] : -o; };
+                auto bwy = [&](int row, float o) { return yp ? -o + R(row)[me - TXH] : -o; };
+                auto bwz = [&](int k) { return s > 0 ? -a[k] + r_c[l][k] : -a[k]; };
+                float h[6];
+                h[0] = bwx(P, a[0]);
+                h[1] = bwy(P + 1, a[1]);
+                h[2] = bwz(2);
+                h[3] = bwx(P + 2, a[3]) + bwy(P + 2, a[3]);
+                h[4] = bwx(P + 3, a[4]) + bwz(4);
+                h[5] = bwy(P + 4, a[5]) + bwz(5);
+                update_w(l, h);
+            }
         }
         if (need_v) {
             // div2(q) with forward differences, v update (tgv2_common.cu:279-354)
@@ -843,50 +916,49 @@ __global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
                 vo[k] = vn;
                 vbn[k] = fmaf(theta, vn - v[k], vn);
             }
-            // w from H(r) (forward differences) - q (tgv3_common.cu:362-405,
-            // tgvk_common.cu:138-182)
-            const float rx_x = xn ? R(KR_RX)[me + 1] : 0.f;
-            const float rxy_x = xn ? R(KR_RXY)[me + 1] : 0.f;
-            const float rxz_x = xn ? R(KR_RXZ)[me + 1] : 0.f;
-            const float ry_y = yn ? R(KR_RY)[me + TXH] : 0.f;
-            const float rxy_y = yn ? R(KR_RXY)[me + TXH] : 0.f;
-            const float ryz_y = yn ? R(KR_RYZ)[me + TXH] : 0.f;
-            float h[6];
-            h[0] = xn ? rx_x - rx : 0.0f;
-            h[1] = yn ? ry_y - ry : 0.0f;
-            h[2] = zn ? rnn[0] - rn[0] : 0.0f;
-            h[3] = (xn ? rxy_x - rxy : 0.0f) + (yn ? rxy_y - rxy : 0.0f);
-            h[4] = (xn ? rxz_x - rn[1] : 0.0f) + (zn ? rnn[1] - rn[1] : 0.0f);
-            h[5] = (yn ? ryz_y - rn[2] : 0.0f) + (zn ? rnn[2] - rn[2] : 0.0f);
-            const float q0[6] = {qxx, qyy, qn[0], qxy, qn[1], qn[2]};
+            // even levels: H forward (tgvk_common.cu:138-182)
 #pragma unroll
-            for (int k = 0; k < 6; ++k) {
-                float wn = fmaf(-tau, h[k] - q0[k], w[k]);
-                if (MK && !actv) wn = w[k];
-                wo[k] = wn;
-                wbn[k] = fmaf(theta, wn - w[k], wn);
+            for (int l = 0; l < L; l += 2) {
+                const int P = KR_R + 5 * l;
+                const float (&a)[6] = rl[l];
+                auto fwx = [&](int row, float o) { return xn ? R(row)[me + 1] - o : 0.0f; };
+                auto fwy = [&](int row, float o) { return yn ? R(row)[me + TXH] - o : 0.0f; };
+                float h[6];
+                h[0] = fwx(P, a[0]);
+                h[1] = fwy(P + 1, a[1]);
+                h[2] = zn ? rnn[l][0] - a[2] : 0.0f;
+                h[3] = fwx(P + 2, a[3]) + fwy(P + 2, a[3]);
+                h[4] = fwx(P + 3, a[4]) + (zn ? rnn[l][1] - a[4] : 0.0f);
+                h[5] = fwy(P + 4, a[5]) + (zn ? rnn[l][2] - a[5] : 0.0f);
+                update_w(l, h);
             }
         }
         if (own && pin && s >= z0 && s < z1) {
-            kf_st(dst(KF_U), i, uo);
+            kf_st(T(F_U) + ff.dt, i, uo);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) kf_st(dst(KF_VX + k), i, vo[k]);
+            for (int k = 0; k < 3; ++k) kf_st(T(F_VX + k) + ff.dt, i, vo[k]);
 #pragma unroll
-            for (int k = 0; k < 6; ++k) kf_st(dst(KF_WX + k), i, wo[k]);
+            for (int l = 0; l < L; ++l)
+#pragma unroll
+                for (int k = 0; k < 6; ++k) kf_st(LW(l, k) + ff.dl, i, wo[l][k]);
         }
 
         // ---- dual half at plane zd = s - 1 (D region holds its u_bar, v_bar, w_bar)
         const int zd = s - 1;
-        float vbc[3], wbc[6];
+        float vbc[3], wbc[L][6];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) vbc[k] = R(KR_VBX + k)[me];
+        for (int k = 0; k < 3; ++k) vbc[k] = R(K::VB + k)[me];
 #pragma unroll
-        for (int k = 0; k < 6; ++k) wbc[k] = R(KR_WBX + k)[me];
+        for (int l = 0; l < L; ++l)
+#pragma unroll
+            for (int k = 0; k < 6; ++k) wbc[l][k] = R(K::WB + 6 * l + k)[me];
         if (own && zd >= z0) {
+            const I id = I(zd) * plane + col;
+            const bool keep = MK && !act_c;   // masked loop: out-of-mask voxels keep their values
             // p update + projection onto |p| <= alpha[0] (tgv2_common.cu:96-131)
-            const float ubc = R(KR_UB)[me];
-            const float uxn = xn ? R(KR_UB)[me + 1] : 0.f;
-            const float uyn = yn ? R(KR_UB)[me + TXH] : 0.f;
+            const float ubc = R(K::UB)[me];
+            const float uxn = xn ? R(K::UB)[me + 1] : 0.f;
+            const float uyn = yn ? R(K::UB)[me + TXH] : 0.f;
             const float dx = xn ? uxn - ubc : 0.0f;
             const float dy = yn ? uyn - ubc : 0.0f;
             const float dz = zd < D - 1 ? ubn - ubc : 0.0f;
@@ -897,18 +969,35 @@ __global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
             float n2 = a3[0] * a3[0];
             n2 = fmaf(a3[1], a3[1], n2);
             n2 = fmaf(a3[2], a3[2], n2);
-            const float tp = sqrtf(n2) / a_p;
+            const float tp = sqrtf(n2) / ff.alpha[0];
             if (tp > 1.0f) {   // wave-uniform branch: the divisions only where a lane projects
 #pragma unroll
                 for (int k = 0; k < 3; ++k) a3[k] = a3[k] / tp;
             }
+#pragma unroll
+            for (int k = 0; k < 3; ++k) kf_st(T(F_PX + k) + ff.dt, id, keep ? p_c[k] : a3[k]);
 
-            // q update with eps_B(v_bar) - w_bar (tgv2_common.cu:174-219, tgv3_common.cu:28-86)
+            // projection of a tensor onto its ball (tgv2_common.cu:222-276)
+            auto project = [&](float (&b)[6], float alpha) {
+                float m2 = b[0] * b[0];
+                m2 = fmaf(b[1], b[1], m2);
+                m2 = fmaf(2.0f * b[3], b[3], m2);
+                m2 = fmaf(b[2], b[2], m2);
+                m2 = fmaf(2.0f * b[4], b[4], m2);
+                m2 = fmaf(2.0f * b[5], b[5], m2);
+                const float tq = sqrtf(m2) / alpha;
+                if (tq > 1.0f) {
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) b[k] = b[k] / tq;
+                }
+            };
+
+            // q update with eps_B(v_bar) - w_bar_0 (tgv2_common.cu:174-219, tgv3_common.cu:28-86)
             float bxv[3], byv[3], bzv[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                bxv[k] = xp ? -vbc[k] + R(KR_VBX + k)[me - 1] : -vbc[k];
-                byv[k] = yp ? -vbc[k] + R(KR_VBX + k)[me - TXH] : -vbc[k];
+                bxv[k] = xp ? -vbc[k] + R(K::VB + k)[me - 1] : -vbc[k];
+                byv[k] = yp ? -vbc[k] + R(K::VB + k)[me - TXH] : -vbc[k];
                 bzv[k] = planar ? 0.0f : (zd > 0 ? -vbc[k] + vb_m2[k] : -vbc[k]);
             }
             float e[6];
@@ -920,98 +1009,88 @@ __global__ __launch_bounds__(KFUSED_MAX_THREADS) void tgvk_fused_kernel(
             e[5] = (byv[2] + bzv[1]) * 0.5f;
             float b6[6];
 #pragma unroll
-            for (int k = 0; k < 6; ++k) b6[k] = fmaf(sigma, e[k] - wbc[k], q_c[k]);
-            float m2 = b6[0] * b6[0];
-            m2 = fmaf(b6[1], b6[1], m2);
-            m2 = fmaf(2.0f * b6[3], b6[3], m2);
-            m2 = fmaf(b6[2], b6[2], m2);
-            m2 = fmaf(2.0f * b6[4], b6[4], m2);
-            m2 = fmaf(2.0f * b6[5], b6[5], m2);
-            const float tq = sqrtf(m2) / a_q;
-            if (tq > 1.0f) {
+            for (int k = 0; k < 6; ++k) b6[k] = fmaf(sigma, e[k] - wbc[0][k], q_c[k]);
+            project(b6, ff.alpha[1]);
 #pragma unroll
-                for (int k = 0; k < 6; ++k) b6[k] = b6[k] / tq;
-            }
+            for (int k = 0; k < 6; ++k) kf_st(T(F_QXX + k) + ff.dt, id, keep ? q_c[k] : b6[k]);
 
-            // r update from G(w_bar) (backward differences), projection with
-            // alpha[2] (tgv3_common.cu:214-262, 311-360)
-            float gg[6];
-            gg[0] = xp ? -wbc[0] + R(KR_WBX)[me - 1] : -wbc[0];
-            gg[1] = yp ? -wbc[1] + R(KR_WBY)[me - TXH] : -wbc[1];
-            gg[2] = zd > 0 ? -wbc[2] + wb_m2[0] : -wbc[2];
-            {
-                const float d = xp ? -wbc[3] + R(KR_WBXY)[me - 1] : -wbc[3];
-                const float d2 = yp ? -wbc[3] + R(KR_WBXY)[me - TXH] : -wbc[3];
-                gg[3] = (d + d2) * 0.5f;
+            // r_l update from G(w_bar_l) - w_bar_{l+1} (even: backward, tgv3_common.cu:214-262;
+            // odd: forward, tgvk_common.cu:89-135), projection with alpha[l + 2]
+            // (tgv3_common.cu:311-360, tgvk_common.cu:28-86)
+#pragma unroll
+            for (int l = 0; l < L; ++l) {
+                const int Wb = K::WB + 6 * l;
+                const float (&o)[6] = wbc[l];
+                auto gx = [&](int k) {
+                    return (l & 1) ? (xn ? R(Wb + k)[me + 1] - o[k] : 0.0f)
+                                   : (xp ? -o[k] + R(Wb + k)[me - 1] : -o[k]);
+                };
+                auto gy = [&](int k) {
+                    return (l & 1) ? (yn ? R(Wb + k)[me + TXH] - o[k] : 0.0f)
+                                   : (yp ? -o[k] + R(Wb + k)[me - TXH] : -o[k]);
+                };
+                auto gz = [&](int k, int m) {
+                    return (l & 1) ? (zd < D - 1 ? wbn[l][k] - o[k] : 0.0f)
+                                   : (zd > 0 ? -o[k] + wb_m2[l][m] : -o[k]);
+                };
+                float gg[6];
+                gg[0] = gx(0);
+                gg[1] = gy(1);
+                gg[2] = gz(2, 0);
+                gg[3] = (gx(3) + gy(3)) * 0.5f;
+                gg[4] = (gx(4) + gz(4, 1)) * 0.5f;
+                gg[5] = (gy(5) + gz(5, 2)) * 0.5f;
+                float rc[6];
+#pragma unroll
+                for (int k = 0; k < 6; ++k)
+                    rc[k] = fmaf(sigma, l + 1 < L ? gg[k] - wbc[l + 1 < L ? l + 1 : l][k] : gg[k],
+                                 r_c[l][k]);
+                project(rc, ff.alpha[l + 2]);
+#pragma unroll
+                for (int k = 0; k < 6; ++k) kf_st(LR(l, k) + ff.dl, id, keep ? r_c[l][k] : rc[k]);
             }
-            {
-                const float d = xp ? -wbc[4] + R(KR_WBXZ)[me - 1] : -wbc[4];
-                const float d2 = zd > 0 ? -wbc[4] + wb_m2[1] : -wbc[4];
-                gg[4] = (d + d2) * 0.5f;
-            }
-            {
-                const float d = yp ? -wbc[5] + R(KR_WBYZ)[me - TXH] : -wbc[5];
-                const float d2 = zd > 0 ? -wbc[5] + wb_m2[2] : -wbc[5];
-                gg[5] = (d + d2) * 0.5f;
-            }
-            float rc[6];
-#pragma unroll
-            for (int k = 0; k < 6; ++k) rc[k] = fmaf(sigma, gg[k], r_c[k]);
-            float r2 = rc[0] * rc[0];
-            r2 = fmaf(rc[1], rc[1], r2);
-            r2 = fmaf(2.0f * rc[3], rc[3], r2);
-            r2 = fmaf(rc[2], rc[2], r2);
-            r2 = fmaf(2.0f * rc[4], rc[4], r2);
-            r2 = fmaf(2.0f * rc[5], rc[5], r2);
-            const float tr = sqrtf(r2) / a_r;
-            if (tr > 1.0f) {
-#pragma unroll
-                for (int k = 0; k < 6; ++k) rc[k] = rc[k] / tr;
-            }
-
-            const I id = I(zd) * plane + col;
-            const bool keep = MK && !act_c;   // masked loop: out-of-mask voxels keep their values
-#pragma unroll
-            for (int k = 0; k < 3; ++k) kf_st(dst(KF_PX + k), id, keep ? p_c[k] : a3[k]);
-#pragma unroll
-            for (int k = 0; k < 6; ++k) kf_st(dst(KF_QXX + k), id, keep ? q_c[k] : b6[k]);
-#pragma unroll
-            for (int k = 0; k < 6; ++k) kf_st(dst(KF_RX + k), id, keep ? r_c[k] : rc[k]);
         }
         __syncthreads();
 
         // ---- D region <- plane s; carry plane s to the next step
-        R(KR_UB)[me] = ubn;
+        R(K::UB)[me] = ubn;
 #pragma unroll
-        for (int k = 0; k < 3; ++k) R(KR_VBX + k)[me] = vbn[k];
-#pragma unroll
-        for (int k = 0; k < 6; ++k) R(KR_WBX + k)[me] = wbn[k];
+        for (int k = 0; k < 3; ++k) R(K::VB + k)[me] = vbn[k];
 #pragma unroll
         for (int k = 0; k < 3; ++k) vb_m2[k] = vbc[k];
-        wb_m2[0] = wbc[2]; wb_m2[1] = wbc[4]; wb_m2[2] = wbc[5];
-        p_c[0] = px; p_c[1] = py; p_c[2] = pz;
-        q_c[0] = qxx; q_c[1] = qyy; q_c[2] = qn[0]; q_c[3] = qxy; q_c[4] = qn[1]; q_c[5] = qn[2];
-        r_c[0] = rx; r_c[1] = ry; r_c[2] = rn[0]; r_c[3] = rxy; r_c[4] = rn[1]; r_c[5] = rn[2];
 #pragma unroll
-        for (int k = 0; k < 3; ++k) { qn[k] = qnn[k]; rn[k] = rnn[k]; }
+        for (int l = 0; l < L; ++l) {
+#pragma unroll
+            for (int k = 0; k < 6; ++k) R(K::WB + 6 * l + k)[me] = wbn[l][k];
+            wb_m2[l][0] = wbc[l][2]; wb_m2[l][1] = wbc[l][4]; wb_m2[l][2] = wbc[l][5];
+#pragma unroll
+            for (int k = 0; k < 6; ++k) r_c[l][k] = rl[l][k];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) rn[l][k] = rnn[l][k];
+        }
+        p_c[0] = px; p_c[1] = py; p_c[2] = pz;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) q_c[k] = q0[k];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) qn[k] = qnn[k];
         act_c = actv;
     }
 }
 
-template <class I, int MK>
+template <int L, int MK>
 hipError_t tgvk_fused_launch(hipStream_t s, const KFusedFields& ff, const float* f,
                              const uint8_t* act, Geometry g, float tau, float sigma, float lambda,
-                             float theta, const float* alpha, int planar, const TgvkFusedPlan& plan) {
+                             float theta, int planar, const TgvkFusedPlan& plan) {
     const int RT = plan.ty + 2, TXH = plan.tx < g.w ? plan.tx + 2 : g.w;
+    if (TXH * RT > kfused_threads<L>()) return hipErrorInvalidConfiguration;
     const int nbx = (g.w + plan.tx - 1) / plan.tx;
     const int nb = (g.h + plan.ty - 1) / plan.ty, nc = (g.d + plan.zchunk - 1) / plan.zchunk;
-    const size_t lds = size_t(N_KROWS) * RT * TXH * sizeof(float);
-    auto kern = tgvk_fused_kernel<I, MK>;
+    const size_t lds = size_t(KRows<L>::N) * RT * TXH * sizeof(float);
+    auto kern = tgvk_fused_kernel<L, MK>;
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3(nbx * nb * nc), dim3(TXH * RT), lds, s, ff, f, act, g, tau,
-                       sigma, lambda, theta, alpha[0], alpha[1], alpha[2], plan.tx, plan.ty,
-                       plan.zchunk, planar);
+                       sigma, lambda, theta, plan.tx, plan.ty, plan.zchunk, planar);
     return hipGetLastError();
 }
 
@@ -1031,22 +1110,35 @@ int tgvk_blocks(const Geometry& g, const PlanOverrides& ov, int* zchunk) {
 
 }  // namespace
 
-// Plan of the fused TGV-k sweep (one level): blocks of up to 1024 threads
-// (one per CU: they hold all its registers), all 22 LDS arrays within the
+// Plan of the fused TGV-k sweep (one or two levels): blocks of up to 1024 or 768
+// threads (one per CU: they hold all its registers), all LDS arrays within the
 // device's limit.  Whole rows (tx = W) whenever a band of at least one row
-// fits (W <= 341), with the tallest band that fits: rows then start on cache
+// fits (W <= 341 or 256), with the tallest band that fits: rows then start on cache
 // lines and halo rows fall on whole waves, which skip the dual half.  Wider
 // rows run in tiles of at most 128 columns plus a halo column on each side.
-// Measured on MI355X at 256^3: whole rows, band 2, 803 us per launch; 64- and
+// Measured on MI355X at 256^3, one level: whole rows, band 2, 767 us per launch; 64- and
 // 128-column tiles with bands of 4 to 13 rows, 1027-1385 us (their rows are
 // 264- or 520-B pieces off cache-line boundaries, and every wave then holds
 // owned lanes and runs the dual half).  The z chunk minimises rounds of
-// resident blocks x (planes + 1).  The overrides tgvk_fused = 0 disable the
+// resident blocks x (planes + 1).
+//
+// Fused against the two launches (us per iteration, one / two levels): 256^3 767 /
+// 1494 against 1330 / 1967, 128^3 102 / 144 against 142 / 228, 96x100x90 50 / 77
+// against 62 / 93, 90x60x66 25 / 38 against 41 / 58.  Volumes of up to
+// KFUSED_SMALL voxels live in the L2s, where a block's chain of plane steps costs
+// more than the second pass over the state (64^3 20.2 / 25.3 against 14.7 / 22.1,
+// 32x30x24 11.8 / 13.6 against 7.0 / 9.1), whatever the band and chunk: they run
+// the two launches, except that one level stays fused up to KFUSED_TINY voxels,
+// where both take the launches' own time (14x12x10: 7.7 against 7.8).  Three
+// levels (217 registers, 512 threads) gained 1.1x at 300x200x40 and lost 0.73x at
+// 256^3: two launches.  The overrides tgvk_fused = 0 disable the
 // fused sweep, tgvk_fused_tx, _ty and _zchunk set the plan.
+constexpr size_t KFUSED_SMALL = 300000, KFUSED_TINY = 16384;
+
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan) {
     // 32-bit offsets only (volumes under 2^30 voxels): the 64-bit form spills
-    if (levels != 1 || needs_index64(g, ov)) return false;
+    if (levels < 1 || levels > KFUSED_MAX_LEVELS || needs_index64(g, ov)) return false;
     if (ov.tgvk_fused == 0) return false;
     int max_lds = 0, cus = 0;
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
@@ -1055,12 +1147,15 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
         return false;
     const int want_tx = std::max(0, ov.tgvk_fused_tx), want_ty = std::max(0, ov.tgvk_fused_ty);
     const int want_zc = std::max(0, ov.tgvk_fused_zchunk);
+    if (!want_tx && !want_ty && !want_zc && g.n() <= KFUSED_SMALL && (levels > 1 || g.n() > KFUSED_TINY))
+        return false;
+    const int max_threads = kfused_max_threads(levels), rows = 11 + 11 * levels;
     int tx = g.w;
     if (want_tx > 0) tx = std::min(want_tx, g.w);
-    else if (3 * g.w > KFUSED_MAX_THREADS) tx = (g.w + (g.w + 127) / 128 - 1) / ((g.w + 127) / 128);
+    else if (3 * g.w > max_threads) tx = (g.w + (g.w + 127) / 128 - 1) / ((g.w + 127) / 128);
     const int txh = tx < g.w ? tx + 2 : g.w;
-    int ty = std::min(KFUSED_MAX_THREADS / txh - 2, g.h);
-    while (ty >= 1 && size_t(N_KROWS) * (ty + 2) * txh * sizeof(float) > size_t(max_lds)) --ty;
+    int ty = std::min(max_threads / txh - 2, g.h);
+    while (ty >= 1 && size_t(rows) * (ty + 2) * txh * sizeof(float) > size_t(max_lds)) --ty;
     if (want_ty > 0) {
         if (want_ty > ty) return false;   // does not fit
         ty = want_ty;
@@ -1080,20 +1175,26 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     return true;
 }
 
-hipError_t launch_tgvk_fused(hipStream_t s, const float* const* src, float* const* dst,
-                             const float* f, const uint8_t* active, Geometry g, float tau,
-                             float sigma, float lambda, float theta, const float* alpha,
-                             int planar, const TgvkFusedPlan& plan) {
-    KFusedFields ff;
-    for (int k = 0; k < N_KF; ++k) ff.src[k] = src[k];
-    ff.dt = reinterpret_cast<const char*>(dst[0]) - reinterpret_cast<const char*>(src[0]);
-    ff.dl = reinterpret_cast<const char*>(dst[KF_WX]) - reinterpret_cast<const char*>(src[KF_WX]);
-    if (g.n() * 4 >= (size_t(1) << 32)) return hipErrorInvalidValue;   // see tgvk_fused_plan
-    if (active)
-        return tgvk_fused_launch<uint32_t, 1>(s, ff, f, active, g, tau, sigma, lambda, theta, alpha,
-                                              planar, plan);
-    return tgvk_fused_launch<uint32_t, 0>(s, ff, f, active, g, tau, sigma, lambda, theta, alpha,
-                                          planar, plan);
+hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_t field_stride,
+                             ptrdiff_t dt, ptrdiff_t dl, const float* f, const uint8_t* active,
+                             Geometry g, int levels, float tau, float sigma, float lambda,
+                             float theta, const float* alpha, int planar,
+                             const TgvkFusedPlan& plan) {
+    if (g.n() * 4 >= (size_t(1) << 32) || levels < 1 || levels > KFUSED_MAX_LEVELS)
+        return hipErrorInvalidValue;   // see tgvk_fused_plan
+    KFusedFields ff{};
+    ff.t = static_cast<const char*>(t);
+    ff.lv = static_cast<const char*>(lv);
+    ff.fs = static_cast<long long>(field_stride);
+    ff.dt = dt;
+    ff.dl = dl;
+    for (int k = 0; k < levels + 2; ++k) ff.alpha[k] = alpha[k];
+    auto go = [&](auto LC) {
+        constexpr int L = decltype(LC)::value;
+        return active ? tgvk_fused_launch<L, 1>(s, ff, f, active, g, tau, sigma, lambda, theta, planar, plan)
+                      : tgvk_fused_launch<L, 0>(s, ff, f, active, g, tau, sigma, lambda, theta, planar, plan);
+    };
+    return levels == 1 ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 2>{});
 }
 
 hipError_t launch_tgvk_dual(hipStream_t s, float* const* fields_dev, float* const* levels_dev,

@@ -161,6 +161,59 @@ def test_tgvk_fused_bitwise_against_oracle(ctx, orc, monkeypatch, shape, tile, b
     np.testing.assert_array_equal(vz, st.v[2])
 
 
+@pytest.mark.parametrize("shape", FUSED_SHAPES)
+@pytest.mark.parametrize("tile,band,zchunk", [(1000, 1, 1), (1000, 2, 3), (8, 1, 1), (16, 2, 3),
+                                              (64, 5, 7), (30, 13, 2)])
+def test_tgvk_fused_two_levels(ctx, orc, shape, tile, band, zchunk):
+    """k = 4: the odd level reads w_bar ahead and r behind.  The same edges as
+    above under its 768 threads, a mask among them."""
+    from ambient_image_processor_amd import native
+    _say("fused tgvk 4", shape, "tile", tile, "band", band, "zchunk", zchunk)
+    d, h, w = shape
+    tx = min(tile, w)
+    fits = band <= h and (band + 2) * (tx + 2 if tx < w else w) <= 768
+    ctx.set_override("tgvk_fused_tx", tile)
+    ctx.set_override("tgvk_fused_ty", band)
+    ctx.set_override("tgvk_fused_zchunk", zchunk)
+    f = _f(shape, 35)
+    alpha = (1.0, 2.0, 0.3, 0.2)
+    ctx.profile(True)
+    ctx.profile_reset()
+    out = ctx.tgvk_deshade(f, _params(native, 12), alpha)
+    prof = ctx.profile_read()
+    ctx.profile(False)
+    assert prof["tgvk_fused"][1] == (11 if fits else 0), prof
+    st = orc.tgvk(f, 12, alpha=alpha, dtype=np.float32, **KPRM)
+    np.testing.assert_array_equal(out[0], st.u)
+    for c in range(3):
+        np.testing.assert_array_equal(out[1 + c], st.v[c])
+    act = (np.random.default_rng(6).random(shape) < 0.5).astype(np.float32)
+    out = ctx.tgvk_deshade_masked(f, _params(native, 7), alpha, act)
+    st = orc.tgvk(f, 7, alpha=alpha, dtype=np.float32, mask=act, **KPRM)
+    np.testing.assert_array_equal(out[0], st.u)
+    np.testing.assert_array_equal(out[3], st.v[2])
+
+
+# the default plans on both sides of the limits (16384 and 300000 voxels)
+@pytest.mark.parametrize("shape,order,fused", [((16, 32, 32), 3, True), ((16, 32, 33), 3, False),
+                                               ((60, 50, 100), 3, False), ((60, 50, 101), 3, True),
+                                               ((60, 50, 100), 4, False), ((60, 50, 101), 4, True),
+                                               ((4, 5, 6), 4, False)])
+def test_tgvk_fused_limits(ctx, orc, shape, order, fused):
+    from ambient_image_processor_amd import native
+    f = _f(shape, 36)
+    alpha = (1.0, 2.0, 0.3, 0.2)[:order]
+    ctx.profile(True)
+    ctx.profile_reset()
+    out = ctx.tgvk_deshade(f, _params(native, 4), alpha)
+    prof = ctx.profile_read()
+    ctx.profile(False)
+    assert prof["tgvk_fused"][1] == (3 if fused else 0), prof
+    st = orc.tgvk(f, 4, alpha=alpha, dtype=np.float32, **KPRM)
+    np.testing.assert_array_equal(out[0], st.u)
+    np.testing.assert_array_equal(out[2], st.v[1])
+
+
 @pytest.mark.parametrize("shape", [(7, 11, 48), (1, 24, 36)])
 def test_tgvk_fused_equals_two_launches(ctx, monkeypatch, shape):
     """u and v after the fused loop equal the two-launch loop's, with the
