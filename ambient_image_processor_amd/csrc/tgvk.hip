@@ -1112,10 +1112,14 @@ int tgvk_blocks(const Geometry& g, const PlanOverrides& ov, int* zchunk) {
 
 // Plan of the fused TGV-k sweep (one or two levels): blocks of up to 1024 or 768
 // threads (one per CU: they hold all its registers), all LDS arrays within the
-// device's limit.  Whole rows (tx = W) whenever a band of at least one row
-// fits (W <= 341 or 256), with the tallest band that fits: rows then start on cache
-// lines and halo rows fall on whole waves, which skip the dual half.  Wider
-// rows run in tiles of at most 128 columns plus a halo column on each side.
+// device's limit.  Whole rows (tx = W), with the tallest band that fits, while a
+// band of two rows fits, or one of one row that fills the block (W = 256, two
+// levels): rows then start on cache lines and halo rows fall on whole waves,
+// which skip the dual half.  Other rows run in equal tiles of at most 128 columns
+// plus a halo column on each side; a band of one whole row would run the dual half
+// three times per voxel (us, one row / tiles: two levels 100x200x200 489 / 409,
+// 120x100x250 383 / 291, 256^3 1489 / 1623; one level 100x300x300 755 / 573,
+// 40x320x320 287 / 250).
 // Measured on MI355X at 256^3, one level: whole rows, band 2, 767 us per launch; 64- and
 // 128-column tiles with bands of 4 to 13 rows, 1027-1385 us (their rows are
 // 264- or 520-B pieces off cache-line boundaries, and every wave then holds
@@ -1129,11 +1133,14 @@ int tgvk_blocks(const Geometry& g, const PlanOverrides& ov, int* zchunk) {
 // more than the second pass over the state (64^3 20.2 / 25.3 against 14.7 / 22.1,
 // 32x30x24 11.8 / 13.6 against 7.0 / 9.1), whatever the band and chunk: they run
 // the two launches, except that one level stays fused up to KFUSED_TINY voxels,
-// where both take the launches' own time (14x12x10: 7.7 against 7.8).  Three
+// where both take the launches' own time (14x12x10: 7.7 against 7.8).  Two levels
+// in tiles start to win above KFUSED_TILED_SMALL (60x70x250 100 against 93, 120x100x250
+// 291 against 379), and volumes of under four planes have no plane to carry
+// (1x1200x256 43 against 27): two launches.  Three
 // levels (217 registers, 512 threads) gained 1.1x at 300x200x40 and lost 0.73x at
 // 256^3: two launches.  The overrides tgvk_fused = 0 disable the
 // fused sweep, tgvk_fused_tx, _ty and _zchunk set the plan.
-constexpr size_t KFUSED_SMALL = 300000, KFUSED_TINY = 16384;
+constexpr size_t KFUSED_SMALL = 300000, KFUSED_TINY = 16384, KFUSED_TILED_SMALL = 1200000;
 
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan) {
@@ -1152,7 +1159,11 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     const int max_threads = kfused_max_threads(levels), rows = 11 + 11 * levels;
     int tx = g.w;
     if (want_tx > 0) tx = std::min(want_tx, g.w);
-    else if (3 * g.w > max_threads) tx = (g.w + (g.w + 127) / 128 - 1) / ((g.w + 127) / 128);
+    else if (4 * g.w > max_threads && 3 * g.w != max_threads)
+        tx = (g.w + (g.w + 127) / 128 - 1) / ((g.w + 127) / 128);
+    if (!want_tx && !want_ty && !want_zc && levels > 1 &&
+        (g.d < 4 || (tx < g.w && g.n() <= KFUSED_TILED_SMALL)))
+        return false;
     const int txh = tx < g.w ? tx + 2 : g.w;
     int ty = std::min(max_threads / txh - 2, g.h);
     while (ty >= 1 && size_t(rows) * (ty + 2) * txh * sizeof(float) > size_t(max_lds)) --ty;

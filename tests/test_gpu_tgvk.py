@@ -194,11 +194,14 @@ def test_tgvk_fused_two_levels(ctx, orc, shape, tile, band, zchunk):
     np.testing.assert_array_equal(out[3], st.v[2])
 
 
-# the default plans on both sides of the limits (16384 and 300000 voxels)
+# the default plans on both sides of the limits (16384 and 300000 voxels; two levels: tiled
+# rows under 1.2 million voxels, under four planes)
 @pytest.mark.parametrize("shape,order,fused", [((16, 32, 32), 3, True), ((16, 32, 33), 3, False),
                                                ((60, 50, 100), 3, False), ((60, 50, 101), 3, True),
                                                ((60, 50, 100), 4, False), ((60, 50, 101), 4, True),
-                                               ((4, 5, 6), 4, False)])
+                                               ((4, 5, 6), 4, False), ((3, 1200, 90), 4, False),
+                                               ((4, 900, 90), 4, True), ((8, 200, 201), 4, False),
+                                               ((20, 300, 201), 4, True), ((4, 400, 257), 3, True)])
 def test_tgvk_fused_limits(ctx, orc, shape, order, fused):
     from ambient_image_processor_amd import native
     f = _f(shape, 36)
