@@ -2,6 +2,7 @@
 // Written for gfx950 (MI355X): wave64, 256 CUs in 8 XCDs, 160 KB LDS per CU.
 #pragma once
 
+#include <vector>
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <cstddef>
@@ -132,6 +133,11 @@ inline bool needs_index64(const Geometry& g, const PlanOverrides& ov) {
     return g.n() * 4 >= (size_t(1) << 32) || ov.index64 > 0;
 }
 
+// A tile of the fused sweep's grid and the planes [z0, z1) it marches.
+struct FusedTile {
+    int tile, z0, z1;
+};
+
 struct SweepParams {
     float lambda, alpha0, alpha1, tau, sigma, theta;
     int data_term;   // 0 L1, 1 L2
@@ -153,10 +159,13 @@ struct SweepParams {
     // vector sweeps' next-plane prefetch (-1: the storage's default)
     int index64;
     int sweep_pf;
-    // masked fused sweep only: one byte per tile of its plan, 0 = no voxel the
-    // tile owns is active, so the tile skips (valid once both copies of the
-    // state agree outside the active set); nullptr = no skipping
-    const uint8_t* tile_active;
+    // masked fused sweep only (non-null with active): launch_fused_active's bytes
+    const uint8_t* fused_active;
+    // masked fused sweep only: the ntiles tiles of its plan that own an active voxel
+    // (valid once both copies of the state agree outside the active set);
+    // nullptr = every tile
+    const FusedTile* tiles;
+    size_t ntiles;
 };
 
 // Column-tile shapes of the sweep kernels: TX x TY threads, each thread owning
@@ -207,9 +216,16 @@ bool fused_energy_plan(const Geometry& g, int device, const PlanOverrides& ov,
                        const FusedPlan& base, FusedPlan* plan);
 // blocks of a fused launch with this plan (= rows of energy partials)
 size_t fused_grid_blocks(const Geometry& g, const FusedPlan& plan);
-// out[t] = 1 if tile t of the fused plan owns an active voxel (fused_grid_blocks bytes)
-hipError_t launch_tile_activity(hipStream_t s, const uint8_t* act, Geometry g,
-                                const FusedPlan& plan, uint8_t* out);
+// Masked fused sweep: which rows (pieces of the plan's tile width) hold active voxels
+// (row_activity_bytes), and from a host copy of that the plan and its tiles
+size_t row_activity_bytes(const Geometry& g, const FusedPlan& plan);
+hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g,
+                               const FusedPlan& plan, uint8_t* out);
+bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
+                        const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
+                        std::vector<FusedTile>* tiles);
+// out[i] = 1 at active voxels, 2 at their x, y and z neighbours, 0 elsewhere (n bytes)
+hipError_t launch_fused_active(hipStream_t s, const uint8_t* act, Geometry g, uint8_t* out);
 hipError_t launch_fused_sweep(hipStream_t s, int storage, void* const* src, void* const* dst13,
                               const float* f, Geometry g, const SweepParams& p,
                               const FusedPlan& plan);

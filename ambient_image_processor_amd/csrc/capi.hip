@@ -117,13 +117,15 @@ struct amb_context {
     // A*, W*, dL/df, partials, scalar accumulators
     char* adj_block = nullptr;
     size_t adj_cap = 0;
-    // masked iteration: one byte per voxel, nonzero = update (grow-only), and
-    // one byte per tile of the fused plan, nonzero = the tile owns an active voxel
+    // masked iteration: one byte per voxel, nonzero = update, the fused sweep's bytes
+    // (launch_fused_active) and its tiles that own an active voxel (grow-only)
     uint8_t* act = nullptr;
     size_t act_cap = 0;
-    uint8_t* tact = nullptr;
-    size_t tact_cap = 0;
-    size_t tact_active = 0;   // active tiles of the masked run's plan
+    uint8_t* fact = nullptr;
+    size_t fact_cap = 0;
+    char* tiles = nullptr;             // row activity, then the tiles
+    size_t tiles_cap = 0;
+    std::vector<FusedTile> tiles_host;
     // fused sweep: second copy of u, v, p, q (grow-only) and the launch plan
     char* alt_block = nullptr;
     size_t alt_cap = 0;
@@ -501,8 +503,10 @@ amb_status begin(amb_context* c, amb_memory mem, const float* f, uint32_t w, uin
     c->sp.index64 = needs_index64(g, c->ov) ? 1 : 0;
     c->sp.sweep_pf = c->ov.sweep_pf;
     c->sp.energy_partials = nullptr;
-    c->sp.tile_active = nullptr;
     c->sp.active = nullptr;
+    c->sp.fused_active = nullptr;
+    c->sp.tiles = nullptr;
+    c->sp.ntiles = 0;
     c->sp.planar = (p->flags & AMB_FLAG_PLANAR) ? 1 : 0;
     const bool fdiv = fused_divisors_ok(c->sp.alpha0, c->sp.alpha1);
     c->fused_ok = fdiv && fused_plan(g, c->storage, c->device, c->ov, &c->fplan);
@@ -568,7 +572,7 @@ amb_status fused_step(amb_context* c, double* energy_out = nullptr) {
             if (c->prof_on) {
                 const size_t nt = fused_grid_blocks(c->g, c->fplan_run);
                 c->prof_tiles_total += nt;
-                c->prof_tiles_swept += c->sp.tile_active ? c->tact_active : nt;
+                c->prof_tiles_swept += c->sp.tiles ? c->sp.ntiles : nt;
             }
         }
     }
@@ -637,13 +641,27 @@ amb_status ensure_active(amb_context* c) {
     return AMB_OK;
 }
 
+amb_status ensure_tiles(amb_context* c, size_t need) {
+    if (need > c->tiles_cap) {
+        if (c->tiles) AMB_HIP(hipFree(c->tiles));
+        c->tiles = nullptr;
+        c->tiles_cap = 0;
+        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->tiles), need));
+        c->tiles_cap = need;
+    }
+    return AMB_OK;
+}
+
 // Runs the iteration with updates restricted to c->act; the restriction is
 // dropped again on every exit path.
 amb_status run_masked(amb_context* c, uint32_t iterations, uint32_t interval,
                       amb_iteration_callback cb, void* user) {
     struct Reset {
         amb_context* c;
-        ~Reset() { c->sp.active = nullptr; c->sp.tile_active = nullptr; }
+        ~Reset() {
+            c->sp.active = c->sp.fused_active = nullptr;
+            c->sp.tiles = nullptr;
+        }
     } reset{c};
     c->sp.active = c->act;
     return run(c, iterations, interval, cb, user, true);
@@ -681,61 +699,43 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
         const int zf[5] = {3, 6, 9, 11, 12};   // vz, pz, qzz, qxz, qyz in the fused order
         for (int k : zf) AMB_HIP(launch_zero_fill(c->stream, c->alt[k], c->g.n() * 4));
     }
-    // masked 3-D loop: tiles of the fused plan that own no active voxel skip,
-    // from the second fused launch of the call on (the first one writes every
-    // voxel of the second copy, after which both copies agree outside the
-    // active set: the masked sweeps store only active voxels)
-    uint8_t* tflags = nullptr;
-    c->sp.tile_active = nullptr;
+    // masked loop: the fused sweep's active bytes, and in 3-D the tiles of its plan
+    // that own an active voxel, which alone are launched from the second fused
+    // launch of the call on (the first one writes every voxel of the second
+    // copy, after which both copies agree outside the active set: the masked
+    // sweeps store only active voxels)
+    const FusedTile* tiles = nullptr;
     c->fplan_run = c->fplan;
+    if (fused && c->sp.active) {
+        const size_t bytes = align_up(c->g.n(), 256);
+        if (bytes > c->fact_cap) {
+            if (c->fact) AMB_HIP(hipFree(c->fact));
+            c->fact = nullptr;
+            c->fact_cap = 0;
+            AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->fact), bytes));
+            c->fact_cap = bytes;
+        }
+        AMB_HIP(launch_fused_active(c->stream, c->sp.active, c->g, c->fact));
+        c->sp.fused_active = c->fact;
+    }
     if (fused && c->sp.active && !image && !c->sp.planar_zero_z) {
-        // the z chunk from the mask: the iteration plan's, 16 or 8 planes, whichever
-        // gives the fewest rounds of active tiles (one resident block per CU) x
-        // (planes + 5) (finer chunks isolate more inactive voxels and spread the
-        // active ones over more CUs; each tile also marches one halo plane and
-        // pays a ramp).  Measured at 256^3 per launch: ball of 51% of the voxels
-        // 362 us with 64 planes, 376 with 16; 18%: 318 / 256 us; 6.5%: 276 / 165 us.
-        FusedPlan cand[3] = {c->fplan, c->fplan, c->fplan};
-        cand[1].zchunk = std::min(c->fplan.zchunk, 16);
-        cand[2].zchunk = std::min(c->fplan.zchunk, 8);
-        const int ncand = c->ov.fused_zchunk > 0 ? 1 : 3;   // a forced z chunk stays
-        size_t need = 0;
-        for (int k = 0; k < ncand; ++k) need += align_up(fused_grid_blocks(c->g, cand[k]), 256);
-        if (need > c->tact_cap) {
-            if (c->tact) AMB_HIP(hipFree(c->tact));
-            c->tact = nullptr;
-            c->tact_cap = 0;
-            AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->tact), need));
-            c->tact_cap = need;
-        }
-        size_t off[3] = {0, 0, 0};
-        for (int k = 0; k < ncand; ++k) {
-            off[k] = k ? off[k - 1] + align_up(fused_grid_blocks(c->g, cand[k - 1]), 256) : 0;
-            AMB_HIP(launch_tile_activity(c->stream, c->sp.active, c->g, cand[k], c->tact + off[k]));
-        }
-        std::vector<uint8_t> h(need);
-        AMB_HIP(hipMemcpyAsync(h.data(), c->tact, need, hipMemcpyDeviceToHost, c->stream));
+        const size_t bytes = row_activity_bytes(c->g, c->fplan);
+        AMB_TRY(ensure_tiles(c, bytes));
+        AMB_HIP(launch_row_activity(c->stream, c->sp.active, c->g, c->fplan,
+                                    reinterpret_cast<uint8_t*>(c->tiles)));
+        std::vector<uint8_t> rows(bytes);
+        AMB_HIP(hipMemcpyAsync(rows.data(), c->tiles, bytes, hipMemcpyDeviceToHost, c->stream));
         AMB_HIP(hipStreamSynchronize(c->stream));
-        size_t active[3] = {0, 0, 0};
-        for (int k = 0; k < ncand; ++k) {
-            const size_t nt = fused_grid_blocks(c->g, cand[k]);
-            for (size_t t = 0; t < nt; ++t) active[k] += h[off[k] + t] != 0;
+        if (fused_masked_tiles(c->g, c->device, c->ov, c->fplan, rows.data(),
+                               &c->fplan_run, &c->tiles_host)) {
+            const size_t need = std::max(c->tiles_host.size(), size_t(1)) * sizeof(FusedTile);
+            AMB_TRY(ensure_tiles(c, need));
+            c->sp.ntiles = c->tiles_host.size();
+            if (c->sp.ntiles > 0)
+                AMB_HIP(hipMemcpyAsync(c->tiles, c->tiles_host.data(), need, hipMemcpyHostToDevice,
+                                       c->stream));
+            tiles = reinterpret_cast<const FusedTile*>(c->tiles);
         }
-        int best = 0;
-        int cus = 0;
-        if (ncand > 1 &&
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->device) ==
-                hipSuccess && cus > 0) {
-            double best_cost = 0.0;
-            for (int k = 0; k < ncand; ++k) {
-                const double rounds = double((active[k] + size_t(cus) - 1) / size_t(cus));
-                const double cost = rounds * double(cand[k].zchunk + 5);
-                if (k == 0 || cost < best_cost) { best = k; best_cost = cost; }
-            }
-        }
-        c->tact_active = active[best];
-        c->fplan_run = cand[best];
-        tflags = c->tact + off[best];
     }
     bool need_dual = true, fused_ran = false;
     const uint32_t every = c->energy_interval;
@@ -749,7 +749,7 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
         if (fused && !observed && it + 1 < iterations && (!want_e || en_fused)) {
             double* slot = nullptr;
             if (want_e) AMB_TRY(etrace_slot(c, &slot));
-            c->sp.tile_active = fused_ran ? tflags : nullptr;
+            c->sp.tiles = fused_ran ? tiles : nullptr;
             AMB_TRY(fused_step(c, slot));
             fused_ran = true;
             need_dual = false;
@@ -787,7 +787,7 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
             }
         }
     }
-    c->sp.tile_active = nullptr;
+    c->sp.tiles = nullptr;
     if (every > 0) AMB_TRY(etrace_collect(c));
     return AMB_OK;
 }
@@ -1264,7 +1264,8 @@ AMB_API amb_status amb_context_destroy(amb_context* c) try {
     if (c->etrace_dev) (void)hipFree(c->etrace_dev);
     if (c->adj_block) (void)hipFree(c->adj_block);
     if (c->act) (void)hipFree(c->act);
-    if (c->tact) (void)hipFree(c->tact);
+    if (c->fact) (void)hipFree(c->fact);
+    if (c->tiles) (void)hipFree(c->tiles);
     if (c->alt_block) (void)hipFree(c->alt_block);
     if (c->kblock) (void)hipFree(c->kblock);
     if (c->klv_dev) (void)hipFree(c->klv_dev);

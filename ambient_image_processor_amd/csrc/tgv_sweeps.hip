@@ -43,9 +43,13 @@ namespace amb {
 namespace {
 
 // Block id -> tile id such that each XCD (blocks are dealt round-robin to the
-// 8 XCDs) receives a contiguous range of tiles.
+// 8 XCDs) receives a contiguous range of tiles, the first nblocks % 8 XCDs one more, so
+// that halo rows are found in the L2 (fused sweep with block counts that 8 does not
+// divide, us per launch against the plain order: 161 x 145 x 140 98 -> 92, 301 x 250
+// x 60 BF16 95 -> 82, 384^3 BF16 771 -> 767).
 __device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
-    if ((nblocks & 7) != 0) return bid;
+    if ((nblocks & 7) != 0)
+        return (bid & 7) * (nblocks >> 3) + min(bid & 7, nblocks & 7) + (bid >> 3);
     return (bid & 7) * (nblocks >> 3) + (bid >> 3);
 }
 
@@ -957,7 +961,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     FusedFields ff, const float* __restrict__ f_, const uint8_t* __restrict__ act, Geometry g,
     float tau, float sigma, float lambda, float alpha0, float alpha1, float theta, int ty,
     int zchunk, int planar, int tx, double* __restrict__ epart,
-    const uint8_t* __restrict__ tile_active, DivConsts dc) {
+    const FusedTile* __restrict__ tiles, DivConsts dc) {
     static_assert(!EN || P2 == 0, "the in-sweep energy covers the 3-D loop");
     static_assert(!SB || P2 == 0, "u_bar / v_bar stores cover the 3-D loop");
     typedef typename S::T T;
@@ -972,15 +976,20 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     const int lane = int(threadIdx.x) % L, r = int(threadIdx.x) / L;
     const int nbx = TL ? (W + tx - 1) / tx : 1, nb = (H + ty - 1) / ty;
     const int t = xcd_tile(blockIdx.x, gridDim.x);
-    // masked loop: a tile without an active voxel among the voxels it owns would
-    // store its inputs unchanged; once both copies of the state agree outside
-    // the active set (the host passes tile_active only then), it can skip
-    if (MK && !EN && P2 == 0 && tile_active && !tile_active[t]) return;
-    const int tb = TL ? t / nbx : t;
+    // masked loop: voxels that are not active keep their values, so once both copies
+    // of the state agree outside the active set (the host passes tiles only then)
+    // the grid is the list of tiles that own an active voxel (fused_masked_tiles),
+    // and without the prefetch (whose registers would spill) lanes load and store
+    // only what the active voxels need (act bytes, fused_active_kernel)
+    constexpr bool LISTS = MK && !EN && P2 == 0, SKIPS = LISTS && !PF;
+    const bool listed = LISTS && tiles, skips = SKIPS && tiles;
+    const int tile = listed ? tiles[t].tile : t;
+    const int tb = TL ? tile / nbx : tile;
     const int y0 = (tb % nb) * ty;
-    const int z0 = (tb / nb) * zchunk, z1 = min(z0 + zchunk, D);
+    const int z0 = listed ? tiles[t].z0 : (tb / nb) * zchunk;
+    const int z1 = listed ? tiles[t].z1 : min(z0 + zchunk, D);
     const int y = IMG ? y0 + r : y0 - 1 + r;
-    const int xb = TL ? (t % nbx) * tx - VX + lane * VX : lane * VX;   // global x of element 0
+    const int xb = TL ? (tile % nbx) * tx - VX + lane * VX : lane * VX;   // global x of element 0
     // (W % VX == 0 and x0 % VX == 0: a lane lies wholly inside or outside the volume)
     const bool rowin = y >= 0 && y < H && (!TL || (xb >= 0 && xb < W));
     const bool cl = !TL || lane > 0, cr = !TL || lane < L - 1;
@@ -1026,6 +1035,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     float qn[3][VX];                      // q_zz, q_xz, q_yz at plane s
     float vb_m2[3][VX];                   // v_bar at plane s - 2
     uint32_t act_c = 0xffffffffu;         // active bytes at plane s - 1
+    bool put_c = true;                    // plane s - 1 is stored
     // EN: FP64 sums (slots of the standalone energy pass; 0 and 4 formed at the end)
     double acc[10];
     float vk_m[3][VX];                    // v (stored value) at plane s - 2
@@ -1038,7 +1048,23 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     for (int k = 0; k < 6; ++k) zero(q_c[k]);
 
     const int zs = z0 > 0 ? z0 - 1 : 0;
-    if (!SKZ && rowin && zs < D) {
+    // act bytes of the next plane to load and of the one after it (MK): read ahead,
+    // as they decide which lanes load anything where the grid is the tile list
+    uint32_t act_0 = 0xffffffffu, act_1 = 0xffffffffu;
+    auto load_act = [&](int zz) {
+        if (!MK) return 0xffffffffu;
+        return rowin && zz < D ? load_active<VX>(act, I(zz) * plane + col) : 0u;
+    };
+    // lanes load and store in groups that cover 128 B: stores of single lanes
+    // write parts of cache lines
+    constexpr int GL = std::min(64, 128 / (VX * int(sizeof(T))));
+    const int gs = (int(threadIdx.x) & 63) & ~(GL - 1);
+    auto group = [&](uint32_t a) {
+        return !skips || ((__ballot(a != 0) >> gs) << (64 - GL)) != 0;
+    };
+    if (SKIPS) { act_0 = load_act(zs); act_1 = load_act(zs + 1); }
+    const bool live_z = group(act_0);
+    if (!SKZ && rowin && zs < D && live_z) {
         const I i = I(zs) * plane + col;
         V::ld(src[G_QZZ], i, qn[0]); V::ld(src[G_QXZ], i, qn[1]);
         if (!IMG) V::ld(src[G_QYZ], i, qn[2]);
@@ -1059,13 +1085,13 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     // absent components are +0 constants in both.
     auto load_plane = [&](int zz, FusedPlane<VX>& P) {
         constexpr bool CLAMP = std::is_same<S, StoreBF16>::value;
-        const bool ok = rowin && zz < D;
+        // (act_1: plane zz + 1 takes its q_zz, q_xz, q_yz from here)
+        const bool ok = group(act_0 | act_1) && rowin && zz < D;
         if (!CLAMP) {
             zero(P.px); zero(P.py); zero(P.pz); zero(P.qxx); zero(P.qxy); zero(P.qyy);
             zero(P.u); zero(P.f);
 #pragma unroll
             for (int k = 0; k < 3; ++k) { zero(P.v[k]); zero(P.qnn[k]); }
-            P.act = 0xffffffffu;
         }
         if (CLAMP || ok) {
             const I i = !CLAMP || ok ? I(zz) * plane + col : I(0);
@@ -1090,8 +1116,9 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                 V::ld(src[G_QZZ], j, P.qnn[0]); V::ld(src[G_QXZ], j, P.qnn[1]);
                 if (!IMG) V::ld(src[G_QYZ], j, P.qnn[2]);
             }
-            P.act = MK ? load_active<VX>(act, i) : 0xffffffffu;
         }
+        if (SKIPS) { P.act = act_0; act_0 = act_1; act_1 = load_act(zz + 2); }
+        else P.act = load_act(zz);
     };
 
     FusedPlane<VX> P;
@@ -1129,8 +1156,9 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
         if (PF && s < z1) load_plane(s + 1, Pn);
 
         // ---- primal half at plane s
-        const bool need_u = rowin && pin && (IMG || r > 0) && cl && s >= z0;
-        const bool need_v = rowin && pin && (IMG || r < RT - 1) && cr && s < z1;
+        const bool live = group(actv), put = group(actv & 0x01010101u);
+        const bool need_u = rowin && pin && (IMG || r > 0) && cl && s >= z0 && live;
+        const bool need_v = rowin && pin && (IMG || r < RT - 1) && cr && s < z1 && live;
         float ubn[VX], vbn[3][VX];
         zero(ubn);
 #pragma unroll
@@ -1162,7 +1190,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                     else if (umf < -tl) un = un + tl;
                     else un = fc;
                 }
-                if (MK && !((actv >> (8 * e)) & 0xffu)) un = uc;
+                if (MK && !((actv >> (8 * e)) & 1u)) un = uc;
                 uo[e] = un;
                 ubn[e] = fmaf(theta, un - uc, un);
             }
@@ -1201,7 +1229,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                 float vn0 = fmaf(-tau, w0 - px[e], v[0][e]);
                 float vn1 = fmaf(-tau, w1 - py[e], v[1][e]);
                 float vn2 = fmaf(-tau, w2 - pz[e], v[2][e]);
-                if (MK && !((actv >> (8 * e)) & 0xffu)) { vn0 = v[0][e]; vn1 = v[1][e]; vn2 = v[2][e]; }
+                if (MK && !((actv >> (8 * e)) & 1u)) { vn0 = v[0][e]; vn1 = v[1][e]; vn2 = v[2][e]; }
                 vo[0][e] = vn0; vo[1][e] = vn1; vo[2][e] = vn2;
                 vbn[0][e] = fmaf(theta, vn0 - v[0][e], vn0);
                 vbn[1][e] = fmaf(theta, vn1 - v[1][e], vn1);
@@ -1286,7 +1314,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                 }
             }
         }
-        if (own && pin && s >= z0 && s < z1) {
+        if (own && pin && s >= z0 && s < z1 && put) {
             V::st(dst[G_U], i, uo);
             V::st(dst[G_VX], i, vo[0]);
             if (!IMG) V::st(dst[G_VY], i, vo[1]);
@@ -1309,7 +1337,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
 #pragma unroll
             for (int k = 0; k < 3; ++k) lds_get<VX>(&sVK[k * RW + rw], vkc[k]);
         }
-        if (own && zd >= z0) {
+        if (own && zd >= z0 && put_c) {
             float ubc[VX], uyn[VX], vym[3][VX], vxm[3];
             lds_get<VX>(&sUB[rw], ubc);
             if (IMG) zero(uyn); else lds_get<VX>(&sUB[rw + RWD], uyn);
@@ -1373,7 +1401,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                     qo[0][e] = bxx; qo[1][e] = byy; qo[2][e] = bzz;
                     qo[3][e] = bxy; qo[4][e] = bxz; qo[5][e] = byz;
                 }
-                if (MK && !((act_c >> (8 * e)) & 0xffu)) {
+                if (MK && !((act_c >> (8 * e)) & 1u)) {
 #pragma unroll
                     for (int k = 0; k < 3; ++k) po[k][e] = p_c[k][e];
 #pragma unroll
@@ -1481,6 +1509,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
 #pragma unroll
         for (int k = 0; k < 3; ++k) copyv(qn[k], qnn[k]);
         act_c = actv;
+        put_c = put;
         if (PF && s < z1) P = Pn;
     }
     if constexpr (EN) {
@@ -1675,10 +1704,13 @@ hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Ge
     auto kern = fused_sweep_kernel<S, I, VX, L2, MK, MAXT, PF, TL, P2, EN, SB>;
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(nbx * nb * nc), dim3(L * RT), lds, s, ff, f, p.active, g, p.tau,
+    const bool list = MK && !EN && P2 == 0 && p.tiles;
+    if (list && p.ntiles == 0) return hipSuccess;   // no active voxel
+    hipLaunchKernelGGL(kern, dim3(list ? unsigned(p.ntiles) : unsigned(nbx * nb * nc)), dim3(L * RT), lds, s, ff,
+                       f, MK ? p.fused_active : nullptr, g, p.tau,
                        p.sigma, p.lambda, p.alpha0, p.alpha1, p.theta, plan.ty, plan.zchunk,
                        p.planar, TL ? plan.tx : 0, EN ? p.energy_partials : nullptr,
-                       MK && !EN && P2 == 0 ? p.tile_active : nullptr,
+                       list ? p.tiles : nullptr,
                        div_consts(p.alpha0, p.alpha1));
     return hipGetLastError();
 }
@@ -2115,34 +2147,171 @@ size_t fused_grid_blocks(const Geometry& g, const FusedPlan& plan) {
     return nbx * size_t((g.h + plan.ty - 1) / plan.ty) * size_t((g.d + plan.zchunk - 1) / plan.zchunk);
 }
 
-// Per tile of a fused plan (the kernel's tile index t): 1 if any voxel the
-// tile owns is active.  One block per tile, an OR over its rows and planes.
-__global__ void tile_activity_kernel(const uint8_t* __restrict__ act, Geometry g, int ty,
-                                     int zchunk, int tx, uint8_t* __restrict__ out) {
-    const int t = int(blockIdx.x);
-    const int nbx = tx > 0 ? (g.w + tx - 1) / tx : 1, nb = (g.h + ty - 1) / ty;
-    const int tb = tx > 0 ? t / nbx : t;
-    const int x0 = tx > 0 ? (t % nbx) * tx : 0, x1 = tx > 0 ? min(x0 + tx, g.w) : g.w;
-    const int y0 = (tb % nb) * ty, y1 = min(y0 + ty, g.h);
-    const int z0 = (tb / nb) * zchunk, z1 = min(z0 + zchunk, g.d);
-    const int rw = x1 - x0;
-    const long cnt = long(y1 - y0) * (z1 - z0) * rw;
-    int any = 0;
-    for (long k = threadIdx.x; k < cnt && !any; k += blockDim.x) {
-        const int x = x0 + int(k % rw);
-        const long r = k / rw;
-        const int y = y0 + int(r % (y1 - y0)), z = z0 + int(r / (y1 - y0));
-        any = act[(size_t(z) * g.h + y) * g.w + x] != 0;
+// Active voxels of the row pieces [bx tx, (bx + 1) tx) of every row (tx = 0: whole
+// rows): out[2 ((bx d + z) h + y)] = 1 if the piece holds one, out[.. + 1] = its 64-voxel
+// chunks that do.  One wave per piece.
+__global__ void row_activity_kernel(const uint8_t* __restrict__ act, Geometry g, int tx, int nbx,
+                                    uint8_t* __restrict__ out) {
+    const long pieces = long(g.h) * g.d * nbx;
+    const int step = tx > 0 ? tx : g.w;
+    for (long r = blockIdx.x; r < pieces; r += gridDim.x) {
+        const int y = int(r % g.h), z = int(r / g.h % g.d), bx = int(r / g.h / g.d);
+        const int x1 = min((bx + 1) * step, g.w);
+        int live = 0;
+        for (int x = bx * step; x < x1; x += 64) {
+            const int xl = x + int(threadIdx.x);
+            live += __ballot(xl < x1 && act[(size_t(z) * g.h + y) * g.w + xl]) != 0;
+        }
+        if (threadIdx.x == 0) {
+            out[2 * r] = uint8_t(live > 0);
+            out[2 * r + 1] = uint8_t(min(live, 255));
+        }
     }
-    any = __syncthreads_or(any);
-    if (threadIdx.x == 0) out[t] = uint8_t(any ? 1 : 0);
 }
 
-hipError_t launch_tile_activity(hipStream_t s, const uint8_t* act, Geometry g,
-                                const FusedPlan& plan, uint8_t* out) {
-    const size_t nt = fused_grid_blocks(g, plan);
-    hipLaunchKernelGGL(tile_activity_kernel, dim3(unsigned(nt)), dim3(256), 0, s, act, g, plan.ty,
-                       plan.zchunk, plan.tx, out);
+size_t row_activity_bytes(const Geometry& g, const FusedPlan& plan) {
+    return 2 * size_t(plan.tx > 0 ? (g.w + plan.tx - 1) / plan.tx : 1) * g.h * g.d;
+}
+
+hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g,
+                               const FusedPlan& plan, uint8_t* out) {
+    const size_t pieces = row_activity_bytes(g, plan) / 2;
+    hipLaunchKernelGGL(row_activity_kernel, dim3(unsigned(std::min(pieces, size_t(65536)))), dim3(64), 0,
+                       s, act, g, plan.tx, plan.tx > 0 ? (g.w + plan.tx - 1) / plan.tx : 1, out);
+    return hipGetLastError();
+}
+
+// Plan and tiles of the masked fused sweep from launch_row_activity's bytes, the
+// planes of each tile trimmed to the ones with an active voxel.  The iteration plan
+// where nearly every 64-voxel chunk of the rows holds an active voxel, so that
+// skipping lanes gives less than the prefetch, and up to MASKED_SMALL voxels, which
+// the latency of a plane step bounds.  Otherwise two voxels per lane (one on odd
+// widths, four with 64-bit offsets), no prefetch, the band and z chunk with the least
+//   rounds of active tiles x (planes + 3) x (1 + 0.15 waves on the busiest CU)
+// (a tile's halo planes and ramp; the last factor is small_fused_plan's).
+// Against the iteration plan and its prefetch, tiles skipped inside the full grid
+// (which left the XCDs unevenly loaded) and every lane of the others loading and
+// storing (us per launch, balls of 3, 11, 31 and 50% of the voxels and a random half):
+// 256^3 147 219 332 353 368 -> 45 103 208 290 368; 181 x 217 x 181 49 87 154 196 199 ->
+// 23 49 135 179 199; 160 x 145 x 140 42 48 87 76 81 -> 16 28 50 67 81; 301 x 250 x 60 45
+// 61 126 155 169 -> 16 30 65 110 147; BF16 256^3 94 153 222 225 234 -> 32 68 158 206 247.
+constexpr size_t MASKED_SMALL = 300000;
+
+bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
+                        const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
+                        std::vector<FusedTile>* tiles) {
+    int max_lds = 0, cus = 0;
+    if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return false;
+    FusedPlan p = base;
+    if (p.vx == 4 && !needs_index64(g, ov) && ov.fused_vx <= 0) p.vx = 2;
+    const int row = p.tx > 0 ? p.tx + 2 * p.vx : g.w, L = row / p.vx;
+    const int nbx = p.tx > 0 ? (g.w + p.tx - 1) / p.tx : 1;
+    const int max_threads = p.vx == 4 ? 512 : 1024, max_waves = p.vx == 4 ? 8 : 16;
+    // sum[bx][z][y]: active pieces of rows < y of planes < z
+    const size_t sh = size_t(g.h) + 1, sz = sh * (size_t(g.d) + 1);
+    std::vector<uint32_t> sum(sz * nbx, 0u);
+    uint64_t live = 0;
+    for (int bx = 0; bx < nbx; ++bx)
+        for (int z = 0; z < g.d; ++z) {
+            const uint8_t* r = rows + 2 * (size_t(bx) * g.d + z) * g.h;
+            uint32_t* const a = &sum[bx * sz + z * sh];
+            uint32_t* const b = a + sh;
+            uint32_t acc = 0;
+            for (int y = 0; y < g.h; ++y) {
+                acc += r[2 * y];
+                live += r[2 * y + 1];
+                b[y + 1] = a[y + 1] + acc;
+            }
+        }
+    const uint64_t chunks = uint64_t(g.h) * g.d * nbx *
+                            ((std::min(p.tx > 0 ? p.tx : g.w, g.w) + 63) / 64);
+    const bool keep = ov.fused_pf == 1 || g.n() <= MASKED_SMALL || live * 20 > chunks * 19;
+    auto active = [&](int bx, int y0, int y1, int z0, int z1) {
+        const uint32_t* a = &sum[bx * sz + z0 * sh];
+        const uint32_t* b = &sum[bx * sz + z1 * sh];
+        return b[y1] - b[y0] != a[y1] - a[y0];
+    };
+    static const int ZC[] = {2, 3, 4, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48, 64};
+    double best = 1e300;
+    const int ty_max = std::min(max_threads / L - 2, g.h);
+    const bool fix_ty = ov.fused_ty > 0, fix_zc = ov.fused_zchunk > 0;
+    int ty_last = 0;
+    for (int q = keep ? 0 : 6; q >= 1; --q) {
+        const int ty = fix_ty ? base.ty : std::max(1, ty_max * q / 6);
+        if (L * (ty + 2) > max_threads || ty == ty_last) continue;
+        ty_last = ty;
+        const size_t lds = (p.vx == 4   ? fused_lds_floats<4>(row, ty)
+                            : p.vx == 2 ? fused_lds_floats<2>(row, ty)
+                                        : fused_lds_floats<1>(row, ty)) * sizeof(float);
+        if (lds > size_t(max_lds)) continue;
+        const int waves = (L * (ty + 2) + 63) / 64;
+        const int per_cu = std::max(1, std::min(int(160 * 1024 / lds), max_waves / waves));
+        for (int k = -1; k < int(sizeof(ZC) / sizeof(ZC[0])); ++k) {
+            const int zc = k < 0 ? base.zchunk : ZC[k];
+            if (zc > g.d) break;
+            // (not the finest grids: the search is the host's time)
+            if (k >= 0 && !fix_zc &&
+                long((g.d + zc - 1) / zc) * ((g.h + ty - 1) / ty) * nbx > 12L * cus)
+                continue;
+            size_t n = 0;
+            for (int z = 0; z < g.d; z += zc)
+                for (int y = 0; y < g.h; y += ty)
+                    for (int bx = 0; bx < nbx; ++bx)
+                        n += active(bx, y, std::min(y + ty, g.h), z, std::min(z + zc, g.d));
+            const size_t on_cu = (n + cus - 1) / cus, rounds = (on_cu + per_cu - 1) / per_cu;
+            const double cost = double(rounds) * (zc + 3) *
+                                (1.0 + 0.15 * double(std::min(on_cu, size_t(per_cu)) * waves));
+            if (cost < best) { best = cost; p.ty = ty; p.zchunk = zc; }
+            if (fix_zc) break;
+        }
+        if (fix_ty) break;
+    }
+    if (best < 1e300) p.pf = 0;
+    else p = base;
+    tiles->clear();
+    int t = 0;
+    for (int z = 0; z < g.d; z += p.zchunk)
+        for (int y = 0; y < g.h; y += p.ty)
+            for (int bx = 0; bx < nbx; ++bx, ++t) {
+                const int y1 = std::min(y + p.ty, g.h);
+                int z0 = z, z1 = std::min(z + p.zchunk, g.d);
+                if (!active(bx, y, y1, z0, z1)) continue;
+                while (!active(bx, y, y1, z0, z0 + 1)) ++z0;
+                while (!active(bx, y, y1, z1 - 1, z1)) --z1;
+                tiles->push_back(FusedTile{t, z0, z1});
+            }
+    *plan = p;
+    return true;
+}
+
+// Bytes for the masked fused sweep: 1 at active voxels, 2 at the others that have an active
+// x, y or z neighbour (their values are read), 0 elsewhere.
+// One wave per row.
+__global__ void fused_active_kernel(const uint8_t* __restrict__ act, Geometry g,
+                                    uint8_t* __restrict__ out) {
+    const size_t row = size_t(g.w), plane = row * g.h, rows = size_t(g.h) * g.d;
+    for (size_t r = blockIdx.x; r < rows; r += gridDim.x) {
+        const int y = int(r % g.h), z = int(r / g.h);
+        for (int x = int(threadIdx.x); x < g.w; x += int(blockDim.x)) {
+            const size_t i = r * row + x;
+            uint8_t v = 0;
+            if (act[i]) v = 1;
+            else if ((x > 0 && act[i - 1]) || (x + 1 < g.w && act[i + 1]) ||
+                     (y > 0 && act[i - row]) || (y + 1 < g.h && act[i + row]) ||
+                     (z > 0 && act[i - plane]) || (z + 1 < g.d && act[i + plane]))
+                v = 2;
+            out[i] = v;
+        }
+    }
+}
+
+hipError_t launch_fused_active(hipStream_t s, const uint8_t* act, Geometry g, uint8_t* out) {
+    const size_t rows = size_t(g.h) * g.d;
+    hipLaunchKernelGGL(fused_active_kernel, dim3(unsigned(std::min(rows, size_t(65536)))), dim3(64), 0, s,
+                       act, g, out);
     return hipGetLastError();
 }
 

@@ -307,3 +307,30 @@ def test_unmasked_fused_sweep_counts_every_tile(ctx):
     ctx.profile(False)
     assert launches >= 2 and total > 0 and total % launches == 0
     assert swept == total
+
+
+# over 300000 voxels the fused masked sweep skips lanes: even and odd widths, whole rows
+# and x tiles (700, 515)
+@pytest.mark.parametrize("shape", [(40, 80, 100), (31, 90, 119), (5, 120, 700), (6, 100, 515)])
+@pytest.mark.parametrize("mask", ["ball", "sparse", "slab", "random", "all", "none", "corners"])
+@pytest.mark.parametrize("storage", [0, 1])
+def test_masked_fused_lane_skipping(ctx, shape, mask, storage):
+    """The list of active tiles and the lanes that load and store nothing equal the
+    two-sweep masked loop bit for bit, whatever the mask."""
+    from ambient_image_processor_amd import native
+    _say("lane skip", shape, mask, "storage", storage)
+    d, h, w = shape
+    z, y, x = np.meshgrid(*(np.arange(n) / n - 0.5 for n in shape), indexing="ij")
+    rng = np.random.default_rng(33)
+    act = {"ball": z * z + y * y + x * x <= 0.16, "sparse": rng.random(shape) < 1e-4,
+           "slab": np.abs(x) < 0.13, "random": rng.random(shape) < 0.5,
+           "all": np.ones(shape, bool), "none": np.zeros(shape, bool),
+           "corners": (np.abs(z) > 0.4) & (np.abs(y) > 0.45) & (np.abs(x) > 0.47)}[mask]
+    f = (0.4 + 0.2 * rng.standard_normal(shape)).astype(np.float32)
+    p = _params(native, 6, storage=storage)
+    # any nonzero byte marks a voxel
+    out = ctx.tgv2_deshade_masked(f, p, act.astype(np.uint8) * 2)
+    ctx.set_override("fused", 0)
+    ref = ctx.tgv2_deshade_masked(f, p, act.astype(np.uint8))
+    for a, b in zip(out, ref):
+        np.testing.assert_array_equal(a, b)
