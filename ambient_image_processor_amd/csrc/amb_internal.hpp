@@ -216,11 +216,20 @@ bool fused_energy_plan(const Geometry& g, int device, const PlanOverrides& ov,
                        const FusedPlan& base, FusedPlan* plan);
 // blocks of a fused launch with this plan (= rows of energy partials)
 size_t fused_grid_blocks(const Geometry& g, const FusedPlan& plan);
-// Masked fused sweep: which rows (pieces of the plan's tile width) hold active voxels
-// (row_activity_bytes), and from a host copy of that the plan and its tiles
-size_t row_activity_bytes(const Geometry& g, const FusedPlan& plan);
-hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g,
-                               const FusedPlan& plan, uint8_t* out);
+// Masked fused sweeps: which rows (pieces of tx columns; 0: whole rows) hold active
+// voxels (row_activity_bytes), and from a host copy of that the plan and its tiles
+size_t row_activity_bytes(const Geometry& g, int tx);
+hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g, int tx,
+                               uint8_t* out);
+struct MaskedSearch {
+    int cus;
+    size_t max_lds, lds_row;   // LDS bytes a block may use, and per row of lanes
+    int tx, lanes;             // tile columns (0: whole rows), lanes per row
+    int max_threads, max_waves;   // per block, per CU
+    bool keep, fix_band, fix_zchunk;
+};
+bool masked_tiles(const Geometry& g, const MaskedSearch& m, const uint8_t* rows, int* band,
+                  int* zchunk, std::vector<FusedTile>* tiles);
 bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
                         const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
                         std::vector<FusedTile>* tiles);
@@ -317,9 +326,11 @@ struct TgvkFusedPlan {
 };
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan);
+bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOverrides& ov,
+                       const uint8_t* rows, TgvkFusedPlan* plan, std::vector<FusedTile>* tiles);
 hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_t field_stride,
                              ptrdiff_t dt, ptrdiff_t dl, const float* f, const uint8_t* active,
-                             Geometry g, int levels, float tau, float sigma, float lambda,
+                             const FusedTile* tiles, size_t ntiles, Geometry g, int levels, float tau, float sigma, float lambda,
                              float theta, const float* alpha, int planar,
                              const TgvkFusedPlan& plan);
 

@@ -652,6 +652,43 @@ amb_status ensure_tiles(amb_context* c, size_t need) {
     return AMB_OK;
 }
 
+// The fused sweeps' bytes of the active set (launch_fused_active).
+amb_status fused_active(amb_context* c) {
+    const size_t bytes = align_up(c->g.n(), 256);
+    if (bytes > c->fact_cap) {
+        if (c->fact) AMB_HIP(hipFree(c->fact));
+        c->fact = nullptr;
+        c->fact_cap = 0;
+        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->fact), bytes));
+        c->fact_cap = bytes;
+    }
+    AMB_HIP(launch_fused_active(c->stream, c->sp.active, c->g, c->fact));
+    c->sp.fused_active = c->fact;
+    return AMB_OK;
+}
+
+// Host copy of launch_row_activity's bytes for tiles of tx columns.
+amb_status row_activity(amb_context* c, int tx, std::vector<uint8_t>* rows) {
+    rows->resize(row_activity_bytes(c->g, tx));
+    AMB_TRY(ensure_tiles(c, rows->size()));
+    AMB_HIP(launch_row_activity(c->stream, c->sp.active, c->g, tx,
+                                reinterpret_cast<uint8_t*>(c->tiles)));
+    AMB_HIP(hipMemcpyAsync(rows->data(), c->tiles, rows->size(), hipMemcpyDeviceToHost, c->stream));
+    AMB_HIP(hipStreamSynchronize(c->stream));
+    return AMB_OK;
+}
+
+// c->tiles_host to the device (the host copy stays until the next call's).
+amb_status upload_tiles(amb_context* c) {
+    const size_t need = std::max(c->tiles_host.size(), size_t(1)) * sizeof(FusedTile);
+    AMB_TRY(ensure_tiles(c, need));
+    c->sp.ntiles = c->tiles_host.size();
+    if (c->sp.ntiles > 0)
+        AMB_HIP(hipMemcpyAsync(c->tiles, c->tiles_host.data(), need, hipMemcpyHostToDevice,
+                               c->stream));
+    return AMB_OK;
+}
+
 // Runs the iteration with updates restricted to c->act; the restriction is
 // dropped again on every exit path.
 amb_status run_masked(amb_context* c, uint32_t iterations, uint32_t interval,
@@ -706,34 +743,13 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
     // sweeps store only active voxels)
     const FusedTile* tiles = nullptr;
     c->fplan_run = c->fplan;
-    if (fused && c->sp.active) {
-        const size_t bytes = align_up(c->g.n(), 256);
-        if (bytes > c->fact_cap) {
-            if (c->fact) AMB_HIP(hipFree(c->fact));
-            c->fact = nullptr;
-            c->fact_cap = 0;
-            AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->fact), bytes));
-            c->fact_cap = bytes;
-        }
-        AMB_HIP(launch_fused_active(c->stream, c->sp.active, c->g, c->fact));
-        c->sp.fused_active = c->fact;
-    }
+    if (fused && c->sp.active) AMB_TRY(fused_active(c));
     if (fused && c->sp.active && !image && !c->sp.planar_zero_z) {
-        const size_t bytes = row_activity_bytes(c->g, c->fplan);
-        AMB_TRY(ensure_tiles(c, bytes));
-        AMB_HIP(launch_row_activity(c->stream, c->sp.active, c->g, c->fplan,
-                                    reinterpret_cast<uint8_t*>(c->tiles)));
-        std::vector<uint8_t> rows(bytes);
-        AMB_HIP(hipMemcpyAsync(rows.data(), c->tiles, bytes, hipMemcpyDeviceToHost, c->stream));
-        AMB_HIP(hipStreamSynchronize(c->stream));
-        if (fused_masked_tiles(c->g, c->device, c->ov, c->fplan, rows.data(),
-                               &c->fplan_run, &c->tiles_host)) {
-            const size_t need = std::max(c->tiles_host.size(), size_t(1)) * sizeof(FusedTile);
-            AMB_TRY(ensure_tiles(c, need));
-            c->sp.ntiles = c->tiles_host.size();
-            if (c->sp.ntiles > 0)
-                AMB_HIP(hipMemcpyAsync(c->tiles, c->tiles_host.data(), need, hipMemcpyHostToDevice,
-                                       c->stream));
+        std::vector<uint8_t> rows;
+        AMB_TRY(row_activity(c, c->fplan.tx, &rows));
+        if (fused_masked_tiles(c->g, c->device, c->ov, c->fplan, rows.data(), &c->fplan_run,
+                               &c->tiles_host)) {
+            AMB_TRY(upload_tiles(c));
             tiles = reinterpret_cast<const FusedTile*>(c->tiles);
         }
     }
@@ -940,8 +956,8 @@ amb_status tgvk_fused_step(amb_context* c) {
     if (!ok) return fail(AMB_ERR_NOT_SUPPORTED, "fused TGV-k buffers out of step with the state");
     {
         ProfScope ps(c, P_TGVK_FUSED);
-        AMB_HIP(launch_tgvk_fused(c->stream, t, lv, fstride, td - t, ld - lv, c->f, c->sp.active,
-                                  c->g, c->klevels, c->sp.tau, c->sp.sigma, c->sp.lambda,
+        AMB_HIP(launch_tgvk_fused(c->stream, t, lv, fstride, td - t, ld - lv, c->f,
+                                  c->sp.fused_active, c->sp.tiles, c->sp.ntiles, c->g, c->klevels, c->sp.tau, c->sp.sigma, c->sp.lambda,
                                   c->sp.theta, c->kalpha_host.data(), c->sp.planar, c->kfplan));
     }
     for (int k = 0; k < N_FUSED_FIELDS; ++k) std::swap(c->fields[FUSED_FIELD_MAP[k]], c->kalt13[k]);
@@ -978,6 +994,19 @@ amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
         // earlier uploads from the host tables have run before they change
         AMB_HIP(hipStreamSynchronize(c->stream));
     }
+    // masked loop: as in run()
+    const FusedTile* tiles = nullptr;
+    bool fused_ran = false;
+    if (fused && c->sp.active) {
+        AMB_TRY(fused_active(c));
+        std::vector<uint8_t> rows;
+        AMB_TRY(row_activity(c, c->kfplan.tx < c->g.w ? c->kfplan.tx : 0, &rows));
+        if (tgvk_masked_tiles(c->g, c->klevels, c->device, c->kov, rows.data(), &c->kfplan,
+                              &c->tiles_host)) {
+            AMB_TRY(upload_tiles(c));
+            tiles = reinterpret_cast<const FusedTile*>(c->tiles);
+        }
+    }
     bool need_dual = true, stale = false;
     for (uint32_t it = 0; it < iterations; ++it) {
         const bool observed = cb && interval > 0 && it > 0 && it % interval == 0;
@@ -987,7 +1016,9 @@ amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
                                      c->klevels, c->sp.sigma, c->sp.planar, c->kov));
         }
         if (fused && !observed && it + 1 < iterations) {
+            c->sp.tiles = fused_ran ? tiles : nullptr;
             AMB_TRY(tgvk_fused_step(c));
+            fused_ran = true;
             need_dual = false;
             stale = true;
         } else {
@@ -1021,7 +1052,10 @@ amb_status tgvk_run_masked(amb_context* c, uint32_t iterations, uint32_t interva
                            amb_iteration_callback cb, void* user) {
     struct Reset {
         amb_context* c;
-        ~Reset() { c->sp.active = nullptr; }
+        ~Reset() {
+            c->sp.active = c->sp.fused_active = nullptr;
+            c->sp.tiles = nullptr;
+        }
     } reset{c};
     c->sp.active = c->act;
     return tgvk_run(c, iterations, interval, cb, user);

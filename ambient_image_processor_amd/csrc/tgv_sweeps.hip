@@ -2169,47 +2169,28 @@ __global__ void row_activity_kernel(const uint8_t* __restrict__ act, Geometry g,
     }
 }
 
-size_t row_activity_bytes(const Geometry& g, const FusedPlan& plan) {
-    return 2 * size_t(plan.tx > 0 ? (g.w + plan.tx - 1) / plan.tx : 1) * g.h * g.d;
+size_t row_activity_bytes(const Geometry& g, int tx) {
+    return 2 * size_t(tx > 0 ? (g.w + tx - 1) / tx : 1) * g.h * g.d;
 }
 
-hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g,
-                               const FusedPlan& plan, uint8_t* out) {
-    const size_t pieces = row_activity_bytes(g, plan) / 2;
+hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g, int tx,
+                               uint8_t* out) {
+    const size_t pieces = row_activity_bytes(g, tx) / 2;
     hipLaunchKernelGGL(row_activity_kernel, dim3(unsigned(std::min(pieces, size_t(65536)))), dim3(64), 0,
-                       s, act, g, plan.tx, plan.tx > 0 ? (g.w + plan.tx - 1) / plan.tx : 1, out);
+                       s, act, g, tx, tx > 0 ? (g.w + tx - 1) / tx : 1, out);
     return hipGetLastError();
 }
 
-// Plan and tiles of the masked fused sweep from launch_row_activity's bytes, the
-// planes of each tile trimmed to the ones with an active voxel.  The iteration plan
-// where nearly every 64-voxel chunk of the rows holds an active voxel, so that
-// skipping lanes gives less than the prefetch, and up to MASKED_SMALL voxels, which
-// the latency of a plane step bounds.  Otherwise two voxels per lane (one on odd
-// widths, four with 64-bit offsets), no prefetch, the band and z chunk with the least
+// Band, z chunk and tiles of a masked fused sweep from launch_row_activity's bytes:
+// the band and chunk with the least
 //   rounds of active tiles x (planes + 3) x (1 + 0.15 waves on the busiest CU)
-// (a tile's halo planes and ramp; the last factor is small_fused_plan's).
-// Against the iteration plan and its prefetch, tiles skipped inside the full grid
-// (which left the XCDs unevenly loaded) and every lane of the others loading and
-// storing (us per launch, balls of 3, 11, 31 and 50% of the voxels and a random half):
-// 256^3 147 219 332 353 368 -> 45 103 208 290 368; 181 x 217 x 181 49 87 154 196 199 ->
-// 23 49 135 179 199; 160 x 145 x 140 42 48 87 76 81 -> 16 28 50 67 81; 301 x 250 x 60 45
-// 61 126 155 169 -> 16 30 65 110 147; BF16 256^3 94 153 222 225 234 -> 32 68 158 206 247.
-constexpr size_t MASKED_SMALL = 300000;
-
-bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
-                        const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
-                        std::vector<FusedTile>* tiles) {
-    int max_lds = 0, cus = 0;
-    if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
-            hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
-        return false;
-    FusedPlan p = base;
-    if (p.vx == 4 && !needs_index64(g, ov) && ov.fused_vx <= 0) p.vx = 2;
-    const int row = p.tx > 0 ? p.tx + 2 * p.vx : g.w, L = row / p.vx;
-    const int nbx = p.tx > 0 ? (g.w + p.tx - 1) / p.tx : 1;
-    const int max_threads = p.vx == 4 ? 512 : 1024, max_waves = p.vx == 4 ? 8 : 16;
+// (a tile's halo planes and ramp; the last factor is small_fused_plan's), the planes of
+// each tile trimmed to the ones with an active voxel.  The given band and chunk
+// stay where a caller fixes them and, false then, where nearly every 64-voxel chunk
+// of the rows holds an active voxel.
+bool masked_tiles(const Geometry& g, const MaskedSearch& m, const uint8_t* rows, int* band,
+                  int* zchunk, std::vector<FusedTile>* tiles) {
+    const int nbx = m.tx > 0 ? (g.w + m.tx - 1) / m.tx : 1;
     // sum[bx][z][y]: active pieces of rows < y of planes < z
     const size_t sh = size_t(g.h) + 1, sz = sh * (size_t(g.d) + 1);
     std::vector<uint32_t> sum(sz * nbx, 0u);
@@ -2227,33 +2208,31 @@ bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
             }
         }
     const uint64_t chunks = uint64_t(g.h) * g.d * nbx *
-                            ((std::min(p.tx > 0 ? p.tx : g.w, g.w) + 63) / 64);
-    const bool keep = ov.fused_pf == 1 || g.n() <= MASKED_SMALL || live * 20 > chunks * 19;
+                            ((std::min(m.tx > 0 ? m.tx : g.w, g.w) + 63) / 64);
+    const bool keep = m.keep || live * 20 > chunks * 19;
     auto active = [&](int bx, int y0, int y1, int z0, int z1) {
         const uint32_t* a = &sum[bx * sz + z0 * sh];
         const uint32_t* b = &sum[bx * sz + z1 * sh];
         return b[y1] - b[y0] != a[y1] - a[y0];
     };
     static const int ZC[] = {2, 3, 4, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48, 64};
+    const int base_ty = *band, base_zc = *zchunk, cus = m.cus;
     double best = 1e300;
-    const int ty_max = std::min(max_threads / L - 2, g.h);
-    const bool fix_ty = ov.fused_ty > 0, fix_zc = ov.fused_zchunk > 0;
     int ty_last = 0;
+    const int ty_max = std::min(m.max_threads / m.lanes - 2, g.h);
     for (int q = keep ? 0 : 6; q >= 1; --q) {
-        const int ty = fix_ty ? base.ty : std::max(1, ty_max * q / 6);
-        if (L * (ty + 2) > max_threads || ty == ty_last) continue;
+        const int ty = m.fix_band ? base_ty : std::max(1, ty_max * q / 6);
+        if (m.lanes * (ty + 2) > m.max_threads || ty == ty_last) continue;
         ty_last = ty;
-        const size_t lds = (p.vx == 4   ? fused_lds_floats<4>(row, ty)
-                            : p.vx == 2 ? fused_lds_floats<2>(row, ty)
-                                        : fused_lds_floats<1>(row, ty)) * sizeof(float);
-        if (lds > size_t(max_lds)) continue;
-        const int waves = (L * (ty + 2) + 63) / 64;
-        const int per_cu = std::max(1, std::min(int(160 * 1024 / lds), max_waves / waves));
+        const size_t lds = m.lds_row * (ty + 2);
+        if (lds > m.max_lds) continue;
+        const int waves = (m.lanes * (ty + 2) + 63) / 64;
+        const int per_cu = std::max(1, std::min(int(160 * 1024 / lds), m.max_waves / waves));
         for (int k = -1; k < int(sizeof(ZC) / sizeof(ZC[0])); ++k) {
-            const int zc = k < 0 ? base.zchunk : ZC[k];
+            const int zc = k < 0 ? base_zc : ZC[k];
             if (zc > g.d) break;
             // (not the finest grids: the search is the host's time)
-            if (k >= 0 && !fix_zc &&
+            if (k >= 0 && !m.fix_zchunk &&
                 long((g.d + zc - 1) / zc) * ((g.h + ty - 1) / ty) * nbx > 12L * cus)
                 continue;
             size_t n = 0;
@@ -2264,26 +2243,62 @@ bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
             const size_t on_cu = (n + cus - 1) / cus, rounds = (on_cu + per_cu - 1) / per_cu;
             const double cost = double(rounds) * (zc + 3) *
                                 (1.0 + 0.15 * double(std::min(on_cu, size_t(per_cu)) * waves));
-            if (cost < best) { best = cost; p.ty = ty; p.zchunk = zc; }
-            if (fix_zc) break;
+            if (cost < best) { best = cost; *band = ty; *zchunk = zc; }
+            if (m.fix_zchunk) break;
         }
-        if (fix_ty) break;
+        if (m.fix_band) break;
     }
-    if (best < 1e300) p.pf = 0;
-    else p = base;
     tiles->clear();
     int t = 0;
-    for (int z = 0; z < g.d; z += p.zchunk)
-        for (int y = 0; y < g.h; y += p.ty)
+    for (int z = 0; z < g.d; z += *zchunk)
+        for (int y = 0; y < g.h; y += *band)
             for (int bx = 0; bx < nbx; ++bx, ++t) {
-                const int y1 = std::min(y + p.ty, g.h);
-                int z0 = z, z1 = std::min(z + p.zchunk, g.d);
+                const int y1 = std::min(y + *band, g.h);
+                int z0 = z, z1 = std::min(z + *zchunk, g.d);
                 if (!active(bx, y, y1, z0, z1)) continue;
                 while (!active(bx, y, y1, z0, z0 + 1)) ++z0;
                 while (!active(bx, y, y1, z1 - 1, z1)) --z1;
                 tiles->push_back(FusedTile{t, z0, z1});
             }
-    *plan = p;
+    return best < 1e300;
+}
+
+// Plan and tiles of the masked fused TGV2 sweep.  The iteration plan where
+// skipping lanes gives less than the prefetch (masked_tiles), and up to MASKED_SMALL
+// voxels, which the latency of a plane step bounds; otherwise two voxels per lane
+// (one on odd widths, four with 64-bit offsets), no prefetch.
+// Against the iteration plan and its prefetch, tiles skipped inside the full grid
+// (which left the XCDs unevenly loaded) and every lane of the others loading and
+// storing (us per launch, balls of 3, 11, 31 and 50% of the voxels and a random half):
+// 256^3 147 219 332 353 368 -> 45 103 208 290 368; 181 x 217 x 181 49 87 154 196 199 ->
+// 23 49 135 179 199; 160 x 145 x 140 42 48 87 76 81 -> 16 28 50 67 81; 301 x 250 x 60 45
+// 61 126 155 169 -> 16 30 65 110 147; BF16 256^3 94 153 222 225 234 -> 32 68 158 206 247.
+constexpr size_t MASKED_SMALL = 300000;
+
+bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
+                        const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
+                        std::vector<FusedTile>* tiles) {
+    int max_lds = 0, cus = 0;
+    if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return false;
+    FusedPlan p = base;
+    p.pf = 0;
+    if (p.vx == 4 && !needs_index64(g, ov) && ov.fused_vx <= 0) p.vx = 2;
+    const int row = p.tx > 0 ? p.tx + 2 * p.vx : g.w;
+    MaskedSearch m{};
+    m.cus = cus;
+    m.max_lds = size_t(max_lds);
+    m.tx = p.tx;
+    m.lanes = row / p.vx;
+    m.max_threads = p.vx == 4 ? 512 : 1024;
+    m.max_waves = p.vx == 4 ? 8 : 16;
+    m.lds_row = 8 * size_t(row + m.lanes + 1) * sizeof(float);
+    m.keep = ov.fused_pf == 1 || g.n() <= MASKED_SMALL;
+    m.fix_band = ov.fused_ty > 0;
+    m.fix_zchunk = ov.fused_zchunk > 0;
+    *plan = masked_tiles(g, m, rows, &p.ty, &p.zchunk, tiles) ? p : base;
     return true;
 }
 

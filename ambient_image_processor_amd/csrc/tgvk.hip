@@ -43,7 +43,8 @@ __device__ __forceinline__ int comp_axis_b(int c) { return c < 3 ? -1 : (c == 3 
 // Block id -> tile id such that each XCD (blocks are dealt round-robin to the
 // 8 XCDs) receives a contiguous range of tiles.
 __device__ __forceinline__ int kxcd_tile(int bid, int nblocks) {
-    if ((nblocks & 7) != 0) return bid;
+    if ((nblocks & 7) != 0)
+        return (bid & 7) * (nblocks >> 3) + min(bid & 7, nblocks & 7) + (bid >> 3);
     return (bid & 7) * (nblocks >> 3) + (bid >> 3);
 }
 
@@ -715,7 +716,8 @@ __device__ __forceinline__ void kf_st(const char* p, I i, float v) {
 template <int L, int MK>
 __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
     KFusedFields ff, const float* __restrict__ f_, const uint8_t* __restrict__ act, Geometry g,
-    float tau, float sigma, float lambda, float theta, int tx, int ty, int zchunk, int planar) {
+    float tau, float sigma, float lambda, float theta, int tx, int ty, int zchunk, int planar,
+    const FusedTile* __restrict__ tiles) {
     typedef uint32_t I;
     typedef KRows<L> K;
     extern __shared__ __align__(16) float lds[];
@@ -725,11 +727,16 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
     const int TXH = tiled ? tx + 2 : W, RT = ty + 2, RW = RT * TXH;
     const int c = int(threadIdx.x) % TXH, r = int(threadIdx.x) / TXH;
     const int nbx = (W + tx - 1) / tx, nb = (H + ty - 1) / ty;
-    const int t = kxcd_tile(int(blockIdx.x), int(gridDim.x));
+    const int b = kxcd_tile(int(blockIdx.x), int(gridDim.x));
+    // masked loop, both copies equal outside the active set: the tiles that own an active
+    // voxel, and only lanes that such voxels need (as in the fused TGV2 sweep)
+    const bool skips = MK && tiles;
+    const int t = skips ? tiles[b].tile : b;
     const int tb = t / nbx;
     const int x = tiled ? (t % nbx) * tx - 1 + c : c;
     const int y0 = (tb % nb) * ty;
-    const int z0 = (tb / nb) * zchunk, z1 = min(z0 + zchunk, D);
+    const int z0 = skips ? tiles[b].z0 : (tb / nb) * zchunk;
+    const int z1 = skips ? tiles[b].z1 : min(z0 + zchunk, D);
     const int y = y0 - 1 + r;
     const bool in = y >= 0 && y < H && x >= 0 && x < W;
     // column 0 feeds only backward differences, column tx + 1 only forward ones (tiled)
@@ -763,10 +770,20 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
 #pragma unroll
         for (int k = 0; k < 3; ++k) rn[l][k] = wb_m2[l][k] = 0.f;
     }
-    bool act_c = true;
+    bool act_c = true, put_c = true;
 
     const int zs = z0 > 0 ? z0 - 1 : 0;
-    if (in && zs < D) {
+    // bytes of the next plane and the one after it (MK); lanes load and store in
+    // groups of 32 (128 B)
+    uint32_t act_0 = 1, act_1 = 1;
+    auto load_act = [&](int zz) {
+        return MK && in && zz < D ? uint32_t(act[I(zz) * plane + col]) : 0u;
+    };
+    const int gs = int(threadIdx.x) & 32;
+    auto group = [&](uint32_t a) { return !skips || uint32_t(__ballot(a != 0) >> gs) != 0; };
+    if (MK) { act_0 = load_act(zs); act_1 = load_act(zs + 1); }
+    const bool live_z = group(act_0);
+    if (in && zs < D && live_z) {
         const I i = I(zs) * plane + col;
         qn[0] = kf_ld(T(F_QZZ), i); qn[1] = kf_ld(T(F_QXZ), i); qn[2] = kf_ld(T(F_QYZ), i);
 #pragma unroll
@@ -791,8 +808,16 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
 #pragma unroll
             for (int k = 0; k < 3; ++k) rnn[l][k] = 0.f;
         }
-        bool actv = true;
-        if (in && pin) {
+        bool actv = true, live = true, put = true;
+        bool wanted = true;   // (act_1: plane s + 1 takes its q and r from here)
+        if (MK) {
+            actv = (act_0 & 1u) != 0;
+            live = group(act_0);
+            wanted = group(act_0 | act_1);
+            put = group(act_0 & 1u);
+            act_0 = act_1;
+        }
+        if (in && pin && wanted) {
             px = kf_ld(T(F_PX), i); py = kf_ld(T(F_PY), i); pz = kf_ld(T(F_PZ), i);
             qxx = kf_ld(T(F_QXX), i); qxy = kf_ld(T(F_QXY), i); qyy = kf_ld(T(F_QYY), i);
             u = kf_ld(T(F_U), i);
@@ -819,8 +844,8 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
                     rnn[l][2] = kf_ld(LR(l, 5), j);
                 }
             }
-            if (MK) actv = act[i] != 0;
         }
+        if (MK) act_1 = load_act(s + 2);
 #pragma unroll
         for (int l = 0; l < L; l += 2) { rl[l][2] = rn[l][0]; rl[l][4] = rn[l][1]; rl[l][5] = rn[l][2]; }
 
@@ -837,8 +862,8 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
         __syncthreads();
 
         // ---- primal half at plane s
-        const bool need_u = in && pin && r > 0 && cl && s >= z0;        // u_bar, odd w_bar
-        const bool need_v = in && pin && r < RT - 1 && cr && s < z1;    // v_bar, even w_bar
+        const bool need_u = in && pin && r > 0 && cl && s >= z0 && live;        // u_bar, odd w_bar
+        const bool need_v = in && pin && r < RT - 1 && cr && s < z1 && live;    // v_bar, even w_bar
         float ubn = 0.f, vbn[3] = {0.f, 0.f, 0.f}, wbn[L][6];
         float uo = 0.f, vo[3], wo[L][6];
 #pragma unroll
@@ -933,7 +958,7 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
                 update_w(l, h);
             }
         }
-        if (own && pin && s >= z0 && s < z1) {
+        if (own && pin && s >= z0 && s < z1 && put) {
             kf_st(T(F_U) + ff.dt, i, uo);
 #pragma unroll
             for (int k = 0; k < 3; ++k) kf_st(T(F_VX + k) + ff.dt, i, vo[k]);
@@ -952,7 +977,7 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
         for (int l = 0; l < L; ++l)
 #pragma unroll
             for (int k = 0; k < 6; ++k) wbc[l][k] = R(K::WB + 6 * l + k)[me];
-        if (own && zd >= z0) {
+        if (own && zd >= z0 && put_c) {
             const I id = I(zd) * plane + col;
             const bool keep = MK && !act_c;   // masked loop: out-of-mask voxels keep their values
             // p update + projection onto |p| <= alpha[0] (tgv2_common.cu:96-131)
@@ -1074,12 +1099,14 @@ __global__ __launch_bounds__(kfused_threads<L>()) void tgvk_fused_kernel(
 #pragma unroll
         for (int k = 0; k < 3; ++k) qn[k] = qnn[k];
         act_c = actv;
+        put_c = put;
     }
 }
 
 template <int L, int MK>
 hipError_t tgvk_fused_launch(hipStream_t s, const KFusedFields& ff, const float* f,
-                             const uint8_t* act, Geometry g, float tau, float sigma, float lambda,
+                             const uint8_t* act, const FusedTile* tiles, size_t ntiles,
+                             Geometry g, float tau, float sigma, float lambda,
                              float theta, int planar, const TgvkFusedPlan& plan) {
     const int RT = plan.ty + 2, TXH = plan.tx < g.w ? plan.tx + 2 : g.w;
     if (TXH * RT > kfused_threads<L>()) return hipErrorInvalidConfiguration;
@@ -1089,8 +1116,10 @@ hipError_t tgvk_fused_launch(hipStream_t s, const KFusedFields& ff, const float*
     auto kern = tgvk_fused_kernel<L, MK>;
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3(nbx * nb * nc), dim3(TXH * RT), lds, s, ff, f, act, g, tau,
-                       sigma, lambda, theta, plan.tx, plan.ty, plan.zchunk, planar);
+    if (MK && tiles && ntiles == 0) return hipSuccess;   // no active voxel
+    const size_t nblk = MK && tiles ? ntiles : size_t(nbx) * nb * nc;
+    hipLaunchKernelGGL(kern, dim3(unsigned(nblk)), dim3(TXH * RT), lds, s, ff, f, act, g, tau,
+                       sigma, lambda, theta, plan.tx, plan.ty, plan.zchunk, planar, tiles);
     return hipGetLastError();
 }
 
@@ -1186,9 +1215,36 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     return true;
 }
 
+// The masked loop's band, z chunk and tiles (masked_tiles), the plan's rows or x tiles.
+// Against the whole grid with every lane loading and storing, order 3 (and for
+// order 4 against the two launches), us per iteration, balls of 3, 11, 31 and 50% of the
+// voxels: 256^3 841 847 843 840 -> 95 251 477 709 (1258 1380 1628 1916 -> 244 538 1029
+// 1419); 161 x 145 x 140 199 200 201 202 -> 23 58 103 150; 96 x 120 x 100 61 61 61 61 ->
+// 14 22 36 51; a random half 256^3 823 -> 786.
+bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOverrides& ov,
+                       const uint8_t* rows, TgvkFusedPlan* plan, std::vector<FusedTile>* tiles) {
+    int max_lds = 0, cus = 0;
+    if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
+        return false;
+    MaskedSearch m{};
+    m.cus = cus;
+    m.max_lds = size_t(max_lds);
+    m.tx = plan->tx < g.w ? plan->tx : 0;
+    m.lanes = plan->tx < g.w ? plan->tx + 2 : g.w;
+    m.max_threads = kfused_max_threads(levels);
+    m.max_waves = m.max_threads / 64;
+    m.lds_row = size_t(11 + 11 * levels) * m.lanes * sizeof(float);
+    m.fix_band = ov.tgvk_fused_ty > 0;
+    m.fix_zchunk = ov.tgvk_fused_zchunk > 0;
+    masked_tiles(g, m, rows, &plan->ty, &plan->zchunk, tiles);
+    return true;
+}
+
 hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_t field_stride,
                              ptrdiff_t dt, ptrdiff_t dl, const float* f, const uint8_t* active,
-                             Geometry g, int levels, float tau, float sigma, float lambda,
+                             const FusedTile* tiles, size_t ntiles, Geometry g, int levels, float tau, float sigma, float lambda,
                              float theta, const float* alpha, int planar,
                              const TgvkFusedPlan& plan) {
     if (g.n() * 4 >= (size_t(1) << 32) || levels < 1 || levels > KFUSED_MAX_LEVELS)
@@ -1202,8 +1258,8 @@ hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_
     for (int k = 0; k < levels + 2; ++k) ff.alpha[k] = alpha[k];
     auto go = [&](auto LC) {
         constexpr int L = decltype(LC)::value;
-        return active ? tgvk_fused_launch<L, 1>(s, ff, f, active, g, tau, sigma, lambda, theta, planar, plan)
-                      : tgvk_fused_launch<L, 0>(s, ff, f, active, g, tau, sigma, lambda, theta, planar, plan);
+        return active ? tgvk_fused_launch<L, 1>(s, ff, f, active, tiles, ntiles, g, tau, sigma, lambda, theta, planar, plan)
+                      : tgvk_fused_launch<L, 0>(s, ff, f, nullptr, nullptr, 0, g, tau, sigma, lambda, theta, planar, plan);
     };
     return levels == 1 ? go(std::integral_constant<int, 1>{}) : go(std::integral_constant<int, 2>{});
 }

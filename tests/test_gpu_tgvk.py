@@ -487,3 +487,31 @@ def test_masked_tgvk_depth1_and_launchers(orc):
     st3 = orc.tgvk(f3, 25, alpha=alpha, dtype=np.float32, mask=m3, **KPRM)
     np.testing.assert_array_equal(u3, st3.u)
     np.testing.assert_array_equal(vz3, st3.v[2])
+
+
+# fused masked launches with the list of active tiles and skipping lanes (over the two-launch
+# limits): whole rows, tiles (even and ragged), order 4 over its tiled limit
+@pytest.mark.parametrize("shape,order", [((40, 80, 101), 3), ((12, 90, 400), 3), ((31, 90, 119), 4),
+                                         ((20, 310, 201), 4)])
+@pytest.mark.parametrize("mask", ["ball", "sparse", "slab", "random", "none", "corners"])
+def test_tgvk_fused_masked_lane_skipping(ctx, shape, order, mask):
+    from ambient_image_processor_amd import native
+    _say("tgvk lane skip", shape, "order", order, mask)
+    z, y, x = np.meshgrid(*(np.arange(n) / n - 0.5 for n in shape), indexing="ij")
+    rng = np.random.default_rng(34)
+    act = {"ball": z * z + y * y + x * x <= 0.16, "sparse": rng.random(shape) < 1e-4,
+           "slab": np.abs(x) < 0.13, "random": rng.random(shape) < 0.5,
+           "none": np.zeros(shape, bool),
+           "corners": (np.abs(z) > 0.4) & (np.abs(y) > 0.45) & (np.abs(x) > 0.47)}[mask]
+    f = _f(shape, 37)
+    alpha = (1.0, 2.0, 0.3, 0.2)[:order]
+    ctx.profile(True)
+    ctx.profile_reset()
+    out = ctx.tgvk_deshade_masked(f, _params(native, 6), alpha, act.astype(np.uint8) * 3)
+    prof = ctx.profile_read()
+    ctx.profile(False)
+    assert prof["tgvk_fused"][1] == 5, prof
+    ctx.set_override("tgvk_fused", 0)
+    ref = ctx.tgvk_deshade_masked(f, _params(native, 6), alpha, act.astype(np.uint8))
+    for a, b in zip(out, ref):
+        np.testing.assert_array_equal(a, b)
