@@ -212,7 +212,7 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
 size_t fused_lds_bytes(const Geometry& g, const FusedPlan& plan);
 // Plan of the fused sweep's energy form (SweepParams::energy_partials) derived
 // from the iteration plan; false when the form does not cover the geometry.
-bool fused_energy_plan(const Geometry& g, int device, const PlanOverrides& ov,
+bool fused_energy_plan(const Geometry& g, int storage, int device, const PlanOverrides& ov,
                        const FusedPlan& base, FusedPlan* plan);
 // blocks of a fused launch with this plan (= rows of energy partials)
 size_t fused_grid_blocks(const Geometry& g, const FusedPlan& plan);
@@ -224,13 +224,27 @@ hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g, in
 struct MaskedSearch {
     int cus;
     size_t max_lds, lds_row;   // LDS bytes a block may use, and per row of lanes
-    int tx, lanes;             // tile columns (0: whole rows), lanes per row
+    int lanes;                 // per row
     int max_threads, max_waves;   // per block, per CU
-    bool keep, fix_band, fix_zchunk;
+    bool fix_band, fix_zchunk;
 };
-bool masked_tiles(const Geometry& g, const MaskedSearch& m, const uint8_t* rows, int* band,
-                  int* zchunk, std::vector<FusedTile>* tiles);
-bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
+struct MaskedRows {
+    Geometry g;
+    int tx, nbx;       // tile columns (0: whole rows), tiles per row
+    size_t sh, sz;
+    std::vector<uint32_t> sum;
+    bool dense;        // nearly every 64-voxel chunk of the rows holds an active voxel
+    MaskedRows(const Geometry& g, int tx, const uint8_t* rows);
+    bool active(int bx, int y0, int y1, int z0, int z1) const {
+        const uint32_t* a = &sum[bx * sz + z0 * sh];
+        const uint32_t* b = &sum[bx * sz + z1 * sh];
+        return b[y1] - b[y0] != a[y1] - a[y0];
+    }
+    double search(const MaskedSearch& m, int* band, int* zchunk) const;
+    void tiles(int band, int zchunk, std::vector<FusedTile>* out) const;
+};
+int fused_masked_tx(const Geometry& g, const PlanOverrides& ov, const FusedPlan& base);
+bool fused_masked_tiles(const Geometry& g, int storage, int device, const PlanOverrides& ov,
                         const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
                         std::vector<FusedTile>* tiles);
 // out[i] = 1 at active voxels, 2 at their x, y and z neighbours, 0 elsewhere (n bytes)

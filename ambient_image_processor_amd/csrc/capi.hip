@@ -283,7 +283,7 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
     size_t pn = energy_partials_size(g);
     FusedPlan base{0, 0}, en{0, 0};
     if (fused_plan(g, storage, c->device, c->ov, &base) &&
-        fused_energy_plan(g, c->device, c->ov, base, &en))
+        fused_energy_plan(g, storage, c->device, c->ov, base, &en))
         pn = std::max(pn, fused_grid_blocks(g, en) * 10 + 16);
     if (pn > c->partials_cap) {
         if (c->partials) AMB_HIP(hipFree(c->partials));
@@ -513,7 +513,7 @@ amb_status begin(amb_context* c, amb_memory mem, const float* f, uint32_t w, uin
     c->iplan_ok = fdiv && c->sp.planar && c->storage == 0 &&
                   fused_image_plan(g, c->device, c->ov, &c->iplan);
     c->fen_ok = c->fused_ok && !c->sp.planar &&
-                fused_energy_plan(g, c->device, c->ov, c->fplan, &c->fen_plan) &&
+                fused_energy_plan(g, c->storage, c->device, c->ov, c->fplan, &c->fen_plan) &&
                 fused_grid_blocks(g, c->fen_plan) * 10 + 16 <= c->partials_cap;
     c->have_state = true;
     c->z_zero = true;
@@ -746,9 +746,9 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
     if (fused && c->sp.active) AMB_TRY(fused_active(c));
     if (fused && c->sp.active && !image && !c->sp.planar_zero_z) {
         std::vector<uint8_t> rows;
-        AMB_TRY(row_activity(c, c->fplan.tx, &rows));
-        if (fused_masked_tiles(c->g, c->device, c->ov, c->fplan, rows.data(), &c->fplan_run,
-                               &c->tiles_host)) {
+        AMB_TRY(row_activity(c, fused_masked_tx(c->g, c->ov, c->fplan), &rows));
+        if (fused_masked_tiles(c->g, c->storage, c->device, c->ov, c->fplan, rows.data(),
+                               &c->fplan_run, &c->tiles_host)) {
             AMB_TRY(upload_tiles(c));
             tiles = reinterpret_cast<const FusedTile*>(c->tiles);
         }

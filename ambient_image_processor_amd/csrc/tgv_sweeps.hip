@@ -45,8 +45,8 @@ namespace {
 // Block id -> tile id such that each XCD (blocks are dealt round-robin to the
 // 8 XCDs) receives a contiguous range of tiles, the first nblocks % 8 XCDs one more, so
 // that halo rows are found in the L2 (fused sweep with block counts that 8 does not
-// divide, us per launch against the plain order: 161 x 145 x 140 98 -> 92, 301 x 250
-// x 60 BF16 95 -> 82, 384^3 BF16 771 -> 767).
+// divide, us per launch against the plain order: 161 x 145 x 140 97 -> 90, 301 x 250
+// x 60 BF16 92 -> 78, 291 x 101 x 142 BF16 84 -> 67; 75 of 78 shapes 1.01-1.26x).
 __device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
     if ((nblocks & 7) != 0)
         return (bid & 7) * (nblocks >> 3) + min(bid & 7, nblocks & 7) + (bid >> 3);
@@ -394,12 +394,12 @@ struct VecIO;
 template <>
 struct VecIO<StoreF32, 4> {
     template <class I>
-    static __device__ __forceinline__ void ld(const float* p, I i, float (&o)[4]) {
+    static __device__ __forceinline__ void ld(const float* p, I i, float (&o)[4], int = 0) {
         const float4 t = *reinterpret_cast<const float4*>(elem(p, i));
         o[0] = t.x; o[1] = t.y; o[2] = t.z; o[3] = t.w;
     }
     template <class I>
-    static __device__ __forceinline__ void st(float* p, I i, const float (&v)[4]) {
+    static __device__ __forceinline__ void st(float* p, I i, const float (&v)[4], int = 0) {
         // written once per launch and not read back in it: a streaming store
         typedef float f4 __attribute__((ext_vector_type(4)));
         const f4 t = {v[0], v[1], v[2], v[3]};
@@ -410,13 +410,13 @@ struct VecIO<StoreF32, 4> {
 template <>
 struct VecIO<StoreBF16, 4> {
     template <class I>
-    static __device__ __forceinline__ void ld(const uint16_t* p, I i, float (&o)[4]) {
+    static __device__ __forceinline__ void ld(const uint16_t* p, I i, float (&o)[4], int = 0) {
         const uint2 t = *reinterpret_cast<const uint2*>(elem(p, i));
         o[0] = __uint_as_float(t.x << 16); o[1] = __uint_as_float(t.x & 0xffff0000u);
         o[2] = __uint_as_float(t.y << 16); o[3] = __uint_as_float(t.y & 0xffff0000u);
     }
     template <class I>
-    static __device__ __forceinline__ void st(uint16_t* p, I i, const float (&v)[4]) {
+    static __device__ __forceinline__ void st(uint16_t* p, I i, const float (&v)[4], int = 0) {
         uint2 t;
         t.x = StoreBF16::rne2(v[0], v[1]);
         t.y = StoreBF16::rne2(v[2], v[3]);
@@ -427,11 +427,11 @@ struct VecIO<StoreBF16, 4> {
 template <class S>
 struct VecIO<S, 1> {   // one voxel per lane (odd widths)
     template <class I>
-    static __device__ __forceinline__ void ld(const typename S::T* p, I i, float (&o)[1]) {
+    static __device__ __forceinline__ void ld(const typename S::T* p, I i, float (&o)[1], int = 0) {
         o[0] = S::ld(p, i);
     }
     template <class I>
-    static __device__ __forceinline__ void st(typename S::T* p, I i, const float (&v)[1]) {
+    static __device__ __forceinline__ void st(typename S::T* p, I i, const float (&v)[1], int = 0) {
         S::st(p, i, v[0]);
     }
 };
@@ -439,12 +439,12 @@ struct VecIO<S, 1> {   // one voxel per lane (odd widths)
 template <>
 struct VecIO<StoreF32, 2> {
     template <class I>
-    static __device__ __forceinline__ void ld(const float* p, I i, float (&o)[2]) {
+    static __device__ __forceinline__ void ld(const float* p, I i, float (&o)[2], int = 0) {
         const float2 t = *reinterpret_cast<const float2*>(elem(p, i));
         o[0] = t.x; o[1] = t.y;
     }
     template <class I>
-    static __device__ __forceinline__ void st(float* p, I i, const float (&v)[2]) {
+    static __device__ __forceinline__ void st(float* p, I i, const float (&v)[2], int = 0) {
         typedef float f2 __attribute__((ext_vector_type(2)));
         const f2 t = {v[0], v[1]};
         __builtin_nontemporal_store(t, reinterpret_cast<f2*>(elem(p, i)));
@@ -454,21 +454,40 @@ struct VecIO<StoreF32, 2> {
 template <>
 struct VecIO<StoreBF16, 2> {
     template <class I>
-    static __device__ __forceinline__ void ld(const uint16_t* p, I i, float (&o)[2]) {
+    static __device__ __forceinline__ void ld(const uint16_t* p, I i, float (&o)[2], int = 0) {
         const uint32_t t = *reinterpret_cast<const uint32_t*>(elem(p, i));
         o[0] = __uint_as_float(t << 16); o[1] = __uint_as_float(t & 0xffff0000u);
     }
     template <class I>
-    static __device__ __forceinline__ void st(uint16_t* p, I i, const float (&v)[2]) {
+    static __device__ __forceinline__ void st(uint16_t* p, I i, const float (&v)[2], int = 0) {
         *reinterpret_cast<uint32_t*>(elem(p, i)) = StoreBF16::rne2(v[0], v[1]);
     }
 };
 
-// Active bytes of VX consecutive voxels (byte e of the result = voxel e).
+// Two voxels per lane of rows of odd width (FP32): the accesses are aligned to 4 bytes,
+// and the row's last lane (odd = 1) holds one voxel.  It loads the pair that ends
+// with it, so that nothing beyond the volume is read, and stores that voxel alone.
+struct OddIO {
+    typedef float f2 __attribute__((ext_vector_type(2), aligned(4)));
+    template <class I>
+    static __device__ __forceinline__ void ld(const float* p, I i, float (&o)[2], int odd) {
+        const f2 t = *reinterpret_cast<const f2*>(elem(p, I(i - I(odd))));
+        o[0] = odd ? t.y : t.x; o[1] = t.y;
+    }
+    template <class I>
+    static __device__ __forceinline__ void st(float* p, I i, const float (&v)[2], int odd) {
+        const f2 t = {v[0], v[1]};
+        if (odd) __builtin_nontemporal_store(v[0], elem(p, i));
+        else __builtin_nontemporal_store(t, reinterpret_cast<f2*>(elem(p, i)));
+    }
+};
+
+// Active bytes of VX consecutive voxels (byte e of the result = voxel e); odd: see OddIO.
 template <int VX, class I>
-__device__ __forceinline__ uint32_t load_active(const uint8_t* act, I i) {
+__device__ __forceinline__ uint32_t load_active(const uint8_t* act, I i, int odd = 0) {
     if constexpr (VX == 4) return *reinterpret_cast<const uint32_t*>(elem(act, i));
-    else if constexpr (VX == 2) return uint32_t(*reinterpret_cast<const uint16_t*>(elem(act, i)));
+    else if constexpr (VX == 2)
+        return uint32_t(*reinterpret_cast<const uint16_t*>(elem(act, I(i - I(odd))))) >> (8 * odd);
     else return uint32_t(*elem(act, i));
 }
 
@@ -956,26 +975,31 @@ struct FusedPlane {
 // then holds the whole state after the primal half with p and q one dual half
 // ahead (the adjoint's recompute of a segment, one launch per iteration).
 template <class S, class I, int VX, int L2, int MK, int MAXT, int PF, int TL, int P2, int EN = 0,
-          int SB = 0>
+          int SB = 0, int OD = 0>
 __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     FusedFields ff, const float* __restrict__ f_, const uint8_t* __restrict__ act, Geometry g,
     float tau, float sigma, float lambda, float alpha0, float alpha1, float theta, int ty,
     int zchunk, int planar, int tx, double* __restrict__ epart,
     const FusedTile* __restrict__ tiles, DivConsts dc) {
     static_assert(!EN || P2 == 0, "the in-sweep energy covers the 3-D loop");
+    static_assert(!OD || (VX == 2 && P2 == 0 && std::is_same<S, StoreF32>::value), "odd rows");
     static_assert(!SB || P2 == 0, "u_bar / v_bar stores cover the 3-D loop");
     typedef typename S::T T;
-    typedef VecIO<S, VX> V;
-    typedef VecIO<StoreF32, VX> VF;
+    typedef typename std::conditional<OD != 0, OddIO, VecIO<S, VX>>::type V;
+    typedef typename std::conditional<OD != 0, OddIO, VecIO<StoreF32, VX>>::type VF;
     extern __shared__ __align__(16) float lds[];
 
     const int W = g.w, H = g.h, D = g.d;
     constexpr bool SKZ = P2 == 1, IMG = P2 == 2;
-    const int L = TL ? tx / VX + 2 : W / VX, RT = IMG ? ty : ty + 2;
+    const int L = TL ? tx / VX + 2 : (W + OD) / VX, RT = IMG ? ty : ty + 2;
     const int RWD = L * VX;               // floats per LDS row
     const int lane = int(threadIdx.x) % L, r = int(threadIdx.x) / L;
     const int nbx = TL ? (W + tx - 1) / tx : 1, nb = (H + ty - 1) / ty;
-    const int t = xcd_tile(blockIdx.x, gridDim.x);
+    // (FP32 with the prefetch and more blocks than CUs, not a multiple of 8: the plain
+    // order; 50 x 139 x 110 in 481 blocks 29.7 us, contiguous 32.6; 142 x 232 x 297 in 507
+    // 250 / 257)
+    const bool plain = PF && (gridDim.x & 7) != 0 && gridDim.x > 256 && !(MK && tiles);
+    const int t = plain ? int(blockIdx.x) : xcd_tile(blockIdx.x, gridDim.x);
     // masked loop: voxels that are not active keep their values, so once both copies
     // of the state agree outside the active set (the host passes tiles only then)
     // the grid is the list of tiles that own an active voxel (fused_masked_tiles),
@@ -990,7 +1014,9 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     const int z1 = listed ? tiles[t].z1 : min(z0 + zchunk, D);
     const int y = IMG ? y0 + r : y0 - 1 + r;
     const int xb = TL ? (tile % nbx) * tx - VX + lane * VX : lane * VX;   // global x of element 0
-    // (W % VX == 0 and x0 % VX == 0: a lane lies wholly inside or outside the volume)
+    // (W % VX == 0 and x0 % VX == 0: a lane lies wholly inside or outside the volume;
+    // OD: or holds the row's last voxel and one that does not exist)
+    const int odd = OD && xb == W - 1;
     const bool rowin = y >= 0 && y < H && (!TL || (xb >= 0 && xb < W));
     const bool cl = !TL || lane > 0, cr = !TL || lane < L - 1;
     const bool own = rowin && (IMG || (r >= 1 && r <= ty)) && cl && cr;
@@ -1053,7 +1079,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     uint32_t act_0 = 0xffffffffu, act_1 = 0xffffffffu;
     auto load_act = [&](int zz) {
         if (!MK) return 0xffffffffu;
-        return rowin && zz < D ? load_active<VX>(act, I(zz) * plane + col) : 0u;
+        return rowin && zz < D ? load_active<VX>(act, I(zz) * plane + col, odd) : 0u;
     };
     // lanes load and store in groups that cover 128 B: stores of single lanes
     // write parts of cache lines
@@ -1066,8 +1092,8 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     const bool live_z = group(act_0);
     if (!SKZ && rowin && zs < D && live_z) {
         const I i = I(zs) * plane + col;
-        V::ld(src[G_QZZ], i, qn[0]); V::ld(src[G_QXZ], i, qn[1]);
-        if (!IMG) V::ld(src[G_QYZ], i, qn[2]);
+        V::ld(src[G_QZZ], i, qn[0], odd); V::ld(src[G_QXZ], i, qn[1], odd);
+        if (!IMG) V::ld(src[G_QYZ], i, qn[2], odd);
     }
 
     // BF16 fields (the sweep is bound by instruction issue there): lanes outside
@@ -1095,26 +1121,26 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
         }
         if (CLAMP || ok) {
             const I i = !CLAMP || ok ? I(zz) * plane + col : I(0);
-            V::ld(src[G_PX], i, P.px);
-            if (IMG) zero(P.py); else V::ld(src[G_PY], i, P.py);
-            if (SKZ) zero(P.pz); else V::ld(src[G_PZ], i, P.pz);
-            V::ld(src[G_QXX], i, P.qxx);
+            V::ld(src[G_PX], i, P.px, odd);
+            if (IMG) zero(P.py); else V::ld(src[G_PY], i, P.py, odd);
+            if (SKZ) zero(P.pz); else V::ld(src[G_PZ], i, P.pz, odd);
+            V::ld(src[G_QXX], i, P.qxx, odd);
             if (IMG) { zero(P.qxy); zero(P.qyy); }
-            else { V::ld(src[G_QXY], i, P.qxy); V::ld(src[G_QYY], i, P.qyy); }
-            V::ld(src[G_U], i, P.u); VF::ld(f_, i, P.f);
-            V::ld(src[G_VX], i, P.v[0]);
-            if (IMG) zero(P.v[1]); else V::ld(src[G_VY], i, P.v[1]);
-            if (SKZ) zero(P.v[2]); else V::ld(src[G_VZ], i, P.v[2]);
+            else { V::ld(src[G_QXY], i, P.qxy, odd); V::ld(src[G_QYY], i, P.qyy, odd); }
+            V::ld(src[G_U], i, P.u, odd); VF::ld(f_, i, P.f, odd);
+            V::ld(src[G_VX], i, P.v[0], odd);
+            if (IMG) zero(P.v[1]); else V::ld(src[G_VY], i, P.v[1], odd);
+            if (SKZ) zero(P.v[2]); else V::ld(src[G_VZ], i, P.v[2], odd);
             if (SKZ) {
                 zero(P.qnn[0]); zero(P.qnn[1]); zero(P.qnn[2]);
             } else if (CLAMP) {
                 const I j = ok && zz + 1 < D ? i + plane : i;
-                V::ld(src[G_QZZ], j, P.qnn[0]); V::ld(src[G_QXZ], j, P.qnn[1]);
-                if (IMG) zero(P.qnn[2]); else V::ld(src[G_QYZ], j, P.qnn[2]);
+                V::ld(src[G_QZZ], j, P.qnn[0], odd); V::ld(src[G_QXZ], j, P.qnn[1], odd);
+                if (IMG) zero(P.qnn[2]); else V::ld(src[G_QYZ], j, P.qnn[2], odd);
             } else if (zz + 1 < D) {
                 const I j = i + plane;
-                V::ld(src[G_QZZ], j, P.qnn[0]); V::ld(src[G_QXZ], j, P.qnn[1]);
-                if (!IMG) V::ld(src[G_QYZ], j, P.qnn[2]);
+                V::ld(src[G_QZZ], j, P.qnn[0], odd); V::ld(src[G_QXZ], j, P.qnn[1], odd);
+                if (!IMG) V::ld(src[G_QYZ], j, P.qnn[2], odd);
             }
         }
         if (SKIPS) { P.act = act_0; act_0 = act_1; act_1 = load_act(zz + 2); }
@@ -1254,6 +1280,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
 #pragma unroll
                 for (int e = 0; e < VX; ++e) {
                     const int x = xb + e;
+                    if (OD && x >= W) continue;
                     const int en = e + 1 < VX ? e + 1 : e;
                     const bool xl = e < VX - 1;
                     const bool hx = x > 0, hy = y > 0, hz = s > 0;
@@ -1315,15 +1342,15 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
             }
         }
         if (own && pin && s >= z0 && s < z1 && put) {
-            V::st(dst[G_U], i, uo);
-            V::st(dst[G_VX], i, vo[0]);
-            if (!IMG) V::st(dst[G_VY], i, vo[1]);
-            if (!SKZ) V::st(dst[G_VZ], i, vo[2]);
+            V::st(dst[G_U], i, uo, odd);
+            V::st(dst[G_VX], i, vo[0], odd);
+            if (!IMG) V::st(dst[G_VY], i, vo[1], odd);
+            if (!SKZ) V::st(dst[G_VZ], i, vo[2], odd);
             if constexpr (SB) {
                 T* const* bars = reinterpret_cast<T* const*>(ff.bars);
-                V::st(bars[0], i, ubn);
+                V::st(bars[0], i, ubn, odd);
 #pragma unroll
-                for (int k = 0; k < 3; ++k) V::st(bars[1 + k], i, vbn[k]);
+                for (int k = 0; k < 3; ++k) V::st(bars[1 + k], i, vbn[k], odd);
             }
         }
 
@@ -1423,6 +1450,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
 #pragma unroll
                 for (int e = 0; e < VX; ++e) {
                     const int x = xb + e;
+                    if (OD && x >= W) continue;
                     const int en = e + 1 < VX ? e + 1 : e;
                     const bool nx = x < W - 1, ny = y < H - 1, nz = zd < D - 1;
                     const bool hx = x > 0, hy = y > 0, hz = zd > 0;
@@ -1466,16 +1494,16 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                     acc[7] += a0d * enr - eq;
                 }
             }
-            V::st(dst[G_PX], id, po[0]); V::st(dst[G_QXX], id, qo[0]);
+            V::st(dst[G_PX], id, po[0], odd); V::st(dst[G_QXX], id, qo[0], odd);
             if (!IMG) {
-                V::st(dst[G_PY], id, po[1]); V::st(dst[G_QYY], id, qo[1]);
-                V::st(dst[G_QXY], id, qo[3]);
+                V::st(dst[G_PY], id, po[1], odd); V::st(dst[G_QYY], id, qo[1], odd);
+                V::st(dst[G_QXY], id, qo[3], odd);
             }
             if (!SKZ) {
-                V::st(dst[G_PZ], id, po[2]);
-                V::st(dst[G_QZZ], id, qo[2]); V::st(dst[G_QXZ], id, qo[4]);
+                V::st(dst[G_PZ], id, po[2], odd);
+                V::st(dst[G_QZZ], id, qo[2], odd); V::st(dst[G_QXZ], id, qo[4], odd);
             }
-            if (!SKZ && !IMG) V::st(dst[G_QYZ], id, qo[5]);
+            if (!SKZ && !IMG) V::st(dst[G_QYZ], id, qo[5], odd);
         }
         __syncthreads();
 
@@ -1690,10 +1718,10 @@ hipError_t primal_tiles(hipStream_t s, void* const* fv, const float* f, Geometry
 }
 
 template <class S, class I, int VX, int L2, int MK, int MAXT, int PF, int TL = 0, int P2 = 0,
-          int EN = 0, int SB = 0>
+          int EN = 0, int SB = 0, int OD = 0>
 hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Geometry g,
                         const SweepParams& p, const FusedPlan& plan) {
-    const int row = TL ? plan.tx + 2 * VX : g.w;
+    const int row = TL ? plan.tx + 2 * VX : g.w + OD;
     const int L = row / VX, RT = P2 == 2 ? plan.ty : plan.ty + 2;
     if (L * RT > MAXT) return hipErrorInvalidConfiguration;
     if (!fused_divisors_ok(p.alpha0, p.alpha1)) return hipErrorInvalidValue;
@@ -1701,7 +1729,8 @@ hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Ge
     const int nb = (g.h + plan.ty - 1) / plan.ty, nc = (g.d + plan.zchunk - 1) / plan.zchunk;
     size_t lds = (size_t(EN ? 12 : 8) * RT * row + size_t(EN ? 12 : 8) * RT * (L + 1)) * sizeof(float);
     if (EN) lds = std::max(lds, size_t(16 * 10 * sizeof(double)));   // the block reduction
-    auto kern = fused_sweep_kernel<S, I, VX, L2, MK, MAXT, PF, TL, P2, EN, SB>;
+    if (OD && g.w < 3) return hipErrorInvalidValue;
+    auto kern = fused_sweep_kernel<S, I, VX, L2, MK, MAXT, PF, TL, P2, EN, SB, OD>;
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
     const bool list = MK && !EN && P2 == 0 && p.tiles;
@@ -1716,7 +1745,7 @@ hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Ge
 }
 
 // The energy form (EN = 1): 32-bit offsets, the 3-D loop, two voxels per
-// thread, no next-plane prefetch, blocks of at most EN_THREADS threads (two
+// thread (FP32 also on odd widths: 161 x 145 x 140 174 us per launch, one voxel 239), no next-plane prefetch, blocks of at most EN_THREADS threads (two
 // waves per SIMD: the FP64 sums and the carried u, v need the registers); the
 // plan comes from fused_energy_plan.
 constexpr int EN_THREADS = 512;
@@ -1734,6 +1763,18 @@ hipError_t fused_energy_mk(hipStream_t s, const FusedFields& ff, const float* f,
                                 : fused_launch<S, I, 1, 0, MK, T, 0, 0, 0, 1>(s, ff, f, g, p, plan);
     }
     if (plan.vx != 2) return hipErrorInvalidValue;
+    if (g.w % 2 != 0) {
+        if constexpr (std::is_same<S, StoreF32>::value) {
+            if (plan.tx > 0)
+                return p.data_term == 1
+                           ? fused_launch<S, I, 2, 1, MK, T, 0, 1, 0, 1, 0, 1>(s, ff, f, g, p, plan)
+                           : fused_launch<S, I, 2, 0, MK, T, 0, 1, 0, 1, 0, 1>(s, ff, f, g, p, plan);
+            return p.data_term == 1
+                       ? fused_launch<S, I, 2, 1, MK, T, 0, 0, 0, 1, 0, 1>(s, ff, f, g, p, plan)
+                       : fused_launch<S, I, 2, 0, MK, T, 0, 0, 0, 1, 0, 1>(s, ff, f, g, p, plan);
+        }
+        return hipErrorInvalidValue;
+    }
     if (plan.tx > 0)
         return p.data_term == 1 ? fused_launch<S, I, 2, 1, MK, T, 0, 1, 0, 1>(s, ff, f, g, p, plan)
                                 : fused_launch<S, I, 2, 0, MK, T, 0, 1, 0, 1>(s, ff, f, g, p, plan);
@@ -1764,6 +1805,27 @@ hipError_t fused_shape(hipStream_t s, const FusedFields& ff, const float* f, Geo
                              : fused_launch<S, I, 4, 0, MK, 512, PF>(s, ff, f, g, p, plan);
 }
 
+// Odd widths, FP32 fields: two voxels per lane (OddIO).
+template <int MK, int SB = 0>
+hipError_t fused_odd(hipStream_t s, const FusedFields& ff, const float* f, Geometry g,
+                     const SweepParams& p, const FusedPlan& plan) {
+    typedef StoreF32 S;
+    typedef uint32_t I;
+    const int lanes = plan.tx > 0 ? plan.tx / 2 + 2 : (g.w + 1) / 2;
+    const bool pf = plan.pf && lanes * (plan.ty + 2) <= 768;
+    auto go = [&](auto L2C) {
+        constexpr int L2 = decltype(L2C)::value;
+        if (plan.tx > 0)
+            return pf ? fused_launch<S, I, 2, L2, MK, 768, 1, 1, 0, 0, SB, 1>(s, ff, f, g, p, plan)
+                      : fused_launch<S, I, 2, L2, MK, 1024, 0, 1, 0, 0, SB, 1>(s, ff, f, g, p, plan);
+        return pf ? fused_launch<S, I, 2, L2, MK, 768, 1, 0, 0, 0, SB, 1>(s, ff, f, g, p, plan)
+                  : fused_launch<S, I, 2, L2, MK, 1024, 0, 0, 0, 0, SB, 1>(s, ff, f, g, p, plan);
+    };
+    if (SB || p.data_term == 1) return go(std::integral_constant<int, 1>{});
+    if constexpr (!SB) return go(std::integral_constant<int, 0>{});
+    return hipErrorInvalidValue;
+}
+
 template <class S, class I, int MK>
 hipError_t fused_pf(hipStream_t s, const FusedFields& ff, const float* f, Geometry g,
                     const SweepParams& p, const FusedPlan& plan) {
@@ -1773,6 +1835,9 @@ hipError_t fused_pf(hipStream_t s, const FusedFields& ff, const float* f, Geomet
                                     : fused_launch<S, I, 4, 0, MK, 512, 0, 1, 0>(s, ff, f, g, p, plan);
         return fused_shape<S, I, MK, 0>(s, ff, f, g, p, plan);
     } else {
+        if constexpr (std::is_same<S, StoreF32>::value) {
+            if (g.w % 2 != 0 && plan.vx == 2) return fused_odd<MK>(s, ff, f, g, p, plan);
+        }
         if (plan.vx == 1) {   // odd widths: one voxel per thread, 1024-thread blocks
             if (plan.tx > 0)
                 return p.data_term == 1 ? fused_launch<S, I, 1, 1, MK, 1024, 0, 1>(s, ff, f, g, p, plan)
@@ -1839,6 +1904,7 @@ hipError_t fused_bars_dispatch(hipStream_t s, const FusedFields& ff, const float
         return plan.tx > 0 ? fused_launch<S, I, 1, 1, 0, 1024, 0, 1, 0, 0, 1>(s, ff, f, g, p, plan)
                            : fused_launch<S, I, 1, 1, 0, 1024, 0, 0, 0, 0, 1>(s, ff, f, g, p, plan);
     if (plan.vx != 2) return hipErrorInvalidValue;
+    if (g.w % 2 != 0) return fused_odd<0, 1>(s, ff, f, g, p, plan);
     const int lanes = plan.tx > 0 ? plan.tx / 2 + 2 : g.w / 2;
     const bool pf = plan.pf && lanes * (plan.ty + 2) <= 768;
     if (plan.tx > 0)
@@ -1868,6 +1934,11 @@ hipError_t fused_bars_dispatch(hipStream_t s, const FusedFields& ff, const float
 // at 34x32x250), and so do images and slabs of fewer than 8 planes (500^2: 17.1
 // / 11.3).
 constexpr size_t SMALL_VOXELS = 400000, SMALL_VOXELS_ODD = 170000;
+
+// Odd widths whose rows the two-voxel forms can run (OddIO).
+static bool fused_odd_ok(const Geometry& g, int storage, bool index64) {
+    return g.w % 2 != 0 && g.w >= 3 && storage == 0 && !index64 && g.d > 1;
+}
 
 bool small_fused_plan(const Geometry& g, int cus, int max_lds, FusedPlan* plan) {
     const bool even = g.w % 2 == 0;
@@ -1944,20 +2015,28 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
     // rows fit (four rows of lanes): bands of one row read each row three times
     // (257^3 per launch: 755 us, tiles of 126 columns 549 us; 255^3 with bands
     // of two rows 431 us, of one row 662 us, tiles 542 us)
+    // odd widths, FP32: two voxels per lane (OddIO) where whole rows then fit bands of
+    // three rows and one voxel per lane would run tiles, or where the override asks
+    // (per launch, against one voxel: 257^3 472 / 562 us, 301 x 250 x 60 121 / 154;
+    // narrower 181 x 217 x 181 201 / 185, 161 x 145 x 140 89.6 / 90; wider, in tiles 2047 x
+    // 128 x 48 392 / 366: the row's last lane stores by itself)
+    const bool odd2 = fused_odd_ok(g, storage, big_index) &&
+                      (want_vx == 2 || (4 * g.w > 1024 && 5 * ((g.w + 1) / 2) <= 768));
     for (int vx : {1, 2, 4}) {
         if (want_vx && vx != want_vx) continue;
         if (want_tx > 0) break;   // x tiles forced
-        if (g.w % vx != 0 || (vx <= 2 && big_index) || (vx == 1 && g.w % 2 == 0)) continue;
+        const bool od = odd2 && vx == 2;   // (vx = 1 then has no whole-row band)
+        if ((g.w % vx != 0 && !od) || (vx <= 2 && big_index) || (vx == 1 && g.w % 2 == 0)) continue;
         if (vx == 1 && 4 * g.w > 1024 && !want_ty) continue;
-        const int L = g.w / vx;
+        const int wl = g.w + od, L = wl / vx;
         const int max_threads = vx == 4 ? 512 : 1024;
         const int waves_simd_cap = vx == 4 ? 2 : 4;
         for (int rt = 3; rt * L <= max_threads && rt - 2 <= g.h + 1; ++rt) {
             const int ty = rt - 2;
             if (want_ty && ty != want_ty) continue;
-            const size_t lds = (vx == 4   ? fused_lds_floats<4>(g.w, ty)
-                                : vx == 2 ? fused_lds_floats<2>(g.w, ty)
-                                          : fused_lds_floats<1>(g.w, ty)) *
+            const size_t lds = (vx == 4   ? fused_lds_floats<4>(wl, ty)
+                                : vx == 2 ? fused_lds_floats<2>(wl, ty)
+                                          : fused_lds_floats<1>(wl, ty)) *
                                sizeof(float);
             if (lds > size_t(max_lds)) break;
             const int waves_simd = ((rt * L + 63) / 64 + 3) / 4;
@@ -2086,7 +2165,7 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
     // loads issued one step ahead fit the 168 VGPRs of three waves per SIMD
     // (measured at 256^3, band 4: 366.5 vs 373.7 us; with BF16 fields it is
     // slower, 528 vs 316 us)
-    if (storage == 0 && bp.vx == 2 && !big_index && (g.w / 2) * (bp.ty + 2) <= 768) bp.pf = 1;
+    if (storage == 0 && bp.vx == 2 && !big_index && ((g.w + 1) / 2) * (bp.ty + 2) <= 768) bp.pf = 1;
     if (want_pf == 0 || want_pf == 1) bp.pf = want_pf;
     if (bp.vx == 1) bp.pf = 0;   // the one-voxel form has no prefetch variant
     *plan = bp;
@@ -2094,12 +2173,12 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
 }
 
 // The energy form's plan (results do not depend on the plan): two voxels per
-// thread (one on odd widths), no prefetch, the iteration plan's z chunk; whole
+// thread (one on odd widths with BF16 fields), no prefetch, the iteration plan's z chunk; whole
 // rows in bands of up to the iteration plan's height while three rows fit
 // EN_THREADS threads, else x tiles of 124 columns (64 lanes) in bands of up to
-// 6 rows (odd widths: 126 columns, 128 lanes, bands of 2 rows).  None for
+// 6 rows (one voxel per thread: 126 columns, 128 lanes, bands of 2 rows).  None for
 // 64-bit offsets.
-bool fused_energy_plan(const Geometry& g, int device, const PlanOverrides& ov,
+bool fused_energy_plan(const Geometry& g, int storage, int device, const PlanOverrides& ov,
                        const FusedPlan& base, FusedPlan* plan) {
     if (needs_index64(g, ov) || base.ty < 1) return false;
     FusedPlan e = base;
@@ -2108,7 +2187,7 @@ bool fused_energy_plan(const Geometry& g, int device, const PlanOverrides& ov,
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
         hipSuccess)
         return false;
-    if (g.w % 2 != 0) {
+    if (g.w % 2 != 0 && !fused_odd_ok(g, storage, false)) {
         e.vx = 1;
         if (base.tx == 0 && 3 * g.w <= EN_THREADS) {
             e.tx = 0;
@@ -2126,17 +2205,20 @@ bool fused_energy_plan(const Geometry& g, int device, const PlanOverrides& ov,
         return true;
     }
     e.vx = 2;
-    if (base.tx == 0 && 3 * (g.w / 2) <= EN_THREADS) {
+    const int lanes = (g.w + 1) / 2;
+    if (base.tx == 0 && 3 * lanes <= EN_THREADS) {
         e.tx = 0;
-        e.ty = std::min(base.ty, EN_THREADS / (g.w / 2) - 2);
+        e.ty = EN_THREADS / lanes - 2;
+        if (base.vx != 1) e.ty = std::min(base.ty, e.ty);
     } else {
         e.tx = base.tx > 0 && base.vx == 2 ? base.tx : 124;
+        if (base.vx == 1 && e.tx >= g.w) return false;
         if (e.tx >= g.w) e.tx = 124;
         e.ty = std::min(std::min(base.tx > 0 ? base.ty : 6, 6), EN_THREADS / (e.tx / 2 + 2) - 2);
     }
     e.ty = std::min(e.ty, g.h);
     if (e.ty < 1) return false;
-    const int row = e.tx > 0 ? e.tx + 4 : g.w;
+    const int row = e.tx > 0 ? e.tx + 4 : 2 * lanes;
     if (fused_lds_floats<2>(row, e.ty, 1) * sizeof(float) > size_t(max_lds)) return false;
     *plan = e;
     return true;
@@ -2181,19 +2263,13 @@ hipError_t launch_row_activity(hipStream_t s, const uint8_t* act, Geometry g, in
     return hipGetLastError();
 }
 
-// Band, z chunk and tiles of a masked fused sweep from launch_row_activity's bytes:
-// the band and chunk with the least
-//   rounds of active tiles x (planes + 3) x (1 + 0.15 waves on the busiest CU)
-// (a tile's halo planes and ramp; the last factor is small_fused_plan's), the planes of
-// each tile trimmed to the ones with an active voxel.  The given band and chunk
-// stay where a caller fixes them and, false then, where nearly every 64-voxel chunk
-// of the rows holds an active voxel.
-bool masked_tiles(const Geometry& g, const MaskedSearch& m, const uint8_t* rows, int* band,
-                  int* zchunk, std::vector<FusedTile>* tiles) {
-    const int nbx = m.tx > 0 ? (g.w + m.tx - 1) / m.tx : 1;
-    // sum[bx][z][y]: active pieces of rows < y of planes < z
-    const size_t sh = size_t(g.h) + 1, sz = sh * (size_t(g.d) + 1);
-    std::vector<uint32_t> sum(sz * nbx, 0u);
+// launch_row_activity's bytes as sums: sum[bx][z][y] counts the active pieces of
+// rows < y of planes < z.
+MaskedRows::MaskedRows(const Geometry& geom, int tile, const uint8_t* rows) : g(geom), tx(tile) {
+    nbx = tx > 0 ? (g.w + tx - 1) / tx : 1;
+    sh = size_t(g.h) + 1;
+    sz = sh * (size_t(g.d) + 1);
+    sum.assign(sz * nbx, 0u);
     uint64_t live = 0;
     for (int bx = 0; bx < nbx; ++bx)
         for (int z = 0; z < g.d; ++z) {
@@ -2208,19 +2284,21 @@ bool masked_tiles(const Geometry& g, const MaskedSearch& m, const uint8_t* rows,
             }
         }
     const uint64_t chunks = uint64_t(g.h) * g.d * nbx *
-                            ((std::min(m.tx > 0 ? m.tx : g.w, g.w) + 63) / 64);
-    const bool keep = m.keep || live * 20 > chunks * 19;
-    auto active = [&](int bx, int y0, int y1, int z0, int z1) {
-        const uint32_t* a = &sum[bx * sz + z0 * sh];
-        const uint32_t* b = &sum[bx * sz + z1 * sh];
-        return b[y1] - b[y0] != a[y1] - a[y0];
-    };
+                            ((std::min(tx > 0 ? tx : g.w, g.w) + 63) / 64);
+    dense = live * 20 > chunks * 19;
+}
+
+// Band and z chunk of a masked fused sweep: the ones with the least
+//   rounds of active tiles x (planes + 3) x (1 + 0.15 waves on the busiest CU)
+// (a tile's halo planes and ramp; the last factor is small_fused_plan's), which is
+// returned (negative, and nothing changed, if no band fits).
+double MaskedRows::search(const MaskedSearch& m, int* band, int* zchunk) const {
     static const int ZC[] = {2, 3, 4, 6, 8, 10, 12, 16, 20, 24, 32, 40, 48, 64};
     const int base_ty = *band, base_zc = *zchunk, cus = m.cus;
-    double best = 1e300;
+    double best = -1.0;
     int ty_last = 0;
     const int ty_max = std::min(m.max_threads / m.lanes - 2, g.h);
-    for (int q = keep ? 0 : 6; q >= 1; --q) {
+    for (int q = 6; q >= 1; --q) {
         const int ty = m.fix_band ? base_ty : std::max(1, ty_max * q / 6);
         if (m.lanes * (ty + 2) > m.max_threads || ty == ty_last) continue;
         ty_last = ty;
@@ -2243,39 +2321,53 @@ bool masked_tiles(const Geometry& g, const MaskedSearch& m, const uint8_t* rows,
             const size_t on_cu = (n + cus - 1) / cus, rounds = (on_cu + per_cu - 1) / per_cu;
             const double cost = double(rounds) * (zc + 3) *
                                 (1.0 + 0.15 * double(std::min(on_cu, size_t(per_cu)) * waves));
-            if (cost < best) { best = cost; *band = ty; *zchunk = zc; }
+            if (best < 0.0 || cost < best) { best = cost; *band = ty; *zchunk = zc; }
             if (m.fix_zchunk) break;
         }
         if (m.fix_band) break;
     }
-    tiles->clear();
+    return best;
+}
+
+// The tiles that own an active voxel, their planes trimmed to the ones with one.
+void MaskedRows::tiles(int band, int zchunk, std::vector<FusedTile>* out) const {
+    out->clear();
     int t = 0;
-    for (int z = 0; z < g.d; z += *zchunk)
-        for (int y = 0; y < g.h; y += *band)
+    for (int z = 0; z < g.d; z += zchunk)
+        for (int y = 0; y < g.h; y += band)
             for (int bx = 0; bx < nbx; ++bx, ++t) {
-                const int y1 = std::min(y + *band, g.h);
-                int z0 = z, z1 = std::min(z + *zchunk, g.d);
+                const int y1 = std::min(y + band, g.h);
+                int z0 = z, z1 = std::min(z + zchunk, g.d);
                 if (!active(bx, y, y1, z0, z1)) continue;
                 while (!active(bx, y, y1, z0, z0 + 1)) ++z0;
                 while (!active(bx, y, y1, z1 - 1, z1)) --z1;
-                tiles->push_back(FusedTile{t, z0, z1});
+                out->push_back(FusedTile{t, z0, z1});
             }
-    return best < 1e300;
 }
 
-// Plan and tiles of the masked fused TGV2 sweep.  The iteration plan where
-// skipping lanes gives less than the prefetch (masked_tiles), and up to MASKED_SMALL
-// voxels, which the latency of a plane step bounds; otherwise two voxels per lane
-// (one on odd widths, four with 64-bit offsets), no prefetch.
+// Plan and tiles of the masked fused TGV2 sweep.  The iteration plan where nearly
+// every 64-voxel chunk of the rows holds an active voxel, so that skipping lanes gives
+// less than the prefetch, and up to MASKED_SMALL voxels, which the latency of a plane
+// step bounds; otherwise no prefetch and two voxels per lane (four with 64-bit
+// offsets).  Odd widths: one voxel per lane; with FP32 fields two where their cost is under
+// 0.4 of that (half the lanes, but twice the bytes per step, stores of single voxels at the
+// row ends and coarser skipping: 181 x 217 x 181, costs 0.36 and 0.55 of one voxel's, 114 /
+// 135 and 32 / 23 us; 161 x 145 x 140, 0.50, 63 / 47).
 // Against the iteration plan and its prefetch, tiles skipped inside the full grid
 // (which left the XCDs unevenly loaded) and every lane of the others loading and
 // storing (us per launch, balls of 3, 11, 31 and 50% of the voxels and a random half):
 // 256^3 147 219 332 353 368 -> 45 103 208 290 368; 181 x 217 x 181 49 87 154 196 199 ->
-// 23 49 135 179 199; 160 x 145 x 140 42 48 87 76 81 -> 16 28 50 67 81; 301 x 250 x 60 45
+// 23 48 114 170 199; 160 x 145 x 140 42 48 87 76 81 -> 16 28 50 67 81; 301 x 250 x 60 45
 // 61 126 155 169 -> 16 30 65 110 147; BF16 256^3 94 153 222 225 234 -> 32 68 158 206 247.
 constexpr size_t MASKED_SMALL = 300000;
 
-bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
+// Tile columns of the masked sweep: the iteration plan's, but the one-voxel form's tiles
+// where that plan runs odd rows whole with two voxels per lane.
+int fused_masked_tx(const Geometry& g, const PlanOverrides& ov, const FusedPlan& base) {
+    return g.w % 2 != 0 && base.vx == 2 && base.tx == 0 && ov.fused_vx <= 0 ? 126 : base.tx;
+}
+
+bool fused_masked_tiles(const Geometry& g, int storage, int device, const PlanOverrides& ov,
                         const FusedPlan& base, const uint8_t* rows, FusedPlan* plan,
                         std::vector<FusedTile>* tiles) {
     int max_lds = 0, cus = 0;
@@ -2283,22 +2375,39 @@ bool fused_masked_tiles(const Geometry& g, int device, const PlanOverrides& ov,
             hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return false;
-    FusedPlan p = base;
-    p.pf = 0;
-    if (p.vx == 4 && !needs_index64(g, ov) && ov.fused_vx <= 0) p.vx = 2;
-    const int row = p.tx > 0 ? p.tx + 2 * p.vx : g.w;
-    MaskedSearch m{};
-    m.cus = cus;
-    m.max_lds = size_t(max_lds);
-    m.tx = p.tx;
-    m.lanes = row / p.vx;
-    m.max_threads = p.vx == 4 ? 512 : 1024;
-    m.max_waves = p.vx == 4 ? 8 : 16;
-    m.lds_row = 8 * size_t(row + m.lanes + 1) * sizeof(float);
-    m.keep = ov.fused_pf == 1 || g.n() <= MASKED_SMALL;
-    m.fix_band = ov.fused_ty > 0;
-    m.fix_zchunk = ov.fused_zchunk > 0;
-    *plan = masked_tiles(g, m, rows, &p.ty, &p.zchunk, tiles) ? p : base;
+    const MaskedRows mr(g, fused_masked_tx(g, ov, base), rows);
+    const bool index64 = needs_index64(g, ov);
+    auto form = [&](int vx, FusedPlan* p) {
+        *p = base;
+        p->pf = 0;
+        p->vx = vx;
+        p->tx = mr.tx;
+        const int row = p->tx > 0 ? p->tx + 2 * vx : (g.w + vx - 1) / vx * vx;
+        MaskedSearch m{};
+        m.cus = cus;
+        m.max_lds = size_t(max_lds);
+        m.lanes = row / vx;
+        m.max_threads = vx == 4 ? 512 : 1024;
+        m.max_waves = vx == 4 ? 8 : 16;
+        m.lds_row = 8 * size_t(row + m.lanes + 1) * sizeof(float);
+        m.fix_band = ov.fused_ty > 0;
+        m.fix_zchunk = ov.fused_zchunk > 0;
+        return mr.search(m, &p->ty, &p->zchunk);
+    };
+    *plan = base;
+    if (ov.fused_pf != 1 && g.n() > MASKED_SMALL && !mr.dense) {
+        const bool odd = fused_odd_ok(g, storage, index64) && mr.tx % 2 == 0 && ov.fused_vx <= 0;
+        const int vx = odd ? 1 : base.vx == 4 && !index64 && ov.fused_vx <= 0 ? 2 : base.vx;
+        FusedPlan p;
+        const double cost = form(vx, &p);
+        if (cost >= 0.0) *plan = p;
+        if (odd) {
+            const double two = form(2, &p);
+            if (two >= 0.0 && (cost < 0.0 || two < 0.4 * cost)) *plan = p;
+        }
+    }
+    if (plan->tx != mr.tx) return false;   // the iteration plan, every tile
+    mr.tiles(plan->ty, plan->zchunk, tiles);
     return true;
 }
 
@@ -2331,7 +2440,7 @@ hipError_t launch_fused_active(hipStream_t s, const uint8_t* act, Geometry g, ui
 }
 
 size_t fused_lds_bytes(const Geometry& g, const FusedPlan& plan) {
-    const int row = plan.tx > 0 ? plan.tx + 2 * plan.vx : g.w;
+    const int row = plan.tx > 0 ? plan.tx + 2 * plan.vx : (g.w + plan.vx - 1) / plan.vx * plan.vx;
     return (plan.vx == 1   ? fused_lds_floats<1>(row, plan.ty)
             : plan.vx == 2 ? fused_lds_floats<2>(row, plan.ty)
                            : fused_lds_floats<4>(row, plan.ty)) *

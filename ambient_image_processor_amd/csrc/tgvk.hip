@@ -1215,7 +1215,7 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     return true;
 }
 
-// The masked loop's band, z chunk and tiles (masked_tiles), the plan's rows or x tiles.
+// The masked loop's band, z chunk and tiles (MaskedRows), the plan's rows or x tiles.
 // Against the whole grid with every lane loading and storing, order 3 (and for
 // order 4 against the two launches), us per iteration, balls of 3, 11, 31 and 50% of the
 // voxels: 256^3 841 847 843 840 -> 95 251 477 709 (1258 1380 1628 1916 -> 244 538 1029
@@ -1228,17 +1228,19 @@ bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOver
             hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return false;
+    const bool tiled = plan->tx < g.w;
+    const MaskedRows mr(g, tiled ? plan->tx : 0, rows);
     MaskedSearch m{};
     m.cus = cus;
     m.max_lds = size_t(max_lds);
-    m.tx = plan->tx < g.w ? plan->tx : 0;
-    m.lanes = plan->tx < g.w ? plan->tx + 2 : g.w;
+    m.lanes = tiled ? plan->tx + 2 : g.w;
     m.max_threads = kfused_max_threads(levels);
     m.max_waves = m.max_threads / 64;
     m.lds_row = size_t(11 + 11 * levels) * m.lanes * sizeof(float);
     m.fix_band = ov.tgvk_fused_ty > 0;
     m.fix_zchunk = ov.tgvk_fused_zchunk > 0;
-    masked_tiles(g, m, rows, &plan->ty, &plan->zchunk, tiles);
+    if (!mr.dense) mr.search(m, &plan->ty, &plan->zchunk);
+    mr.tiles(plan->ty, plan->zchunk, tiles);
     return true;
 }
 

@@ -331,3 +331,37 @@ def test_fused_small_volume_plans(ctx, orc, shape):
     out = ctx.tgv2_deshade_masked(f, _params(native, 4, "l1"), act)
     np.testing.assert_array_equal(out[0], st.u)
     np.testing.assert_array_equal(out[2], st.v[1])
+
+
+# odd widths, two voxels per lane: the last lane of a row holds one voxel.  Chosen by the
+# plan for 257 .. 305 columns, forced for the others (the smallest width, both
+# prefetch forms, the last voxel of the volume in every lane position)
+@pytest.mark.parametrize("shape,force", [((5, 9, 257), {}), ((4, 7, 301), {}), ((2, 5, 305), {})] + [
+    (shape, {"fused_vx": 2, "fused_pf": pf}) for pf in (0, 1)
+    for shape in [(4, 5, 3), (9, 13, 21), (7, 30, 129), (3, 4, 255)]])
+@pytest.mark.parametrize("data_term", ["l1", "l2"])
+def test_fused_odd_two_voxels_per_lane(ctx, orc, shape, force, data_term):
+    from ambient_image_processor_amd import native
+    _say("fused odd", shape, force, data_term)
+    f = _f(shape, 41)
+    for k, v in force.items():
+        ctx.set_override(k, v)
+    out, prof = _profile_counts(ctx, lambda: ctx.tgv2_deshade(f, _params(native, 9, data_term)))
+    assert prof["fused_sweep"][1] == 8
+    st = orc.tgv2(f, 9, data_term=data_term, dtype=np.float32, **PRM)
+    np.testing.assert_array_equal(out[0], st.u)
+    for k in range(3):
+        np.testing.assert_array_equal(out[1 + k], st.v[k])
+
+
+def test_fused_odd_two_voxels_adjoint(ctx):
+    """The form that stores u_bar and v_bar (the adjoint's recompute) at such a width."""
+    from ambient_image_processor_amd import native
+    f = _f((4, 7, 259), 42)
+    p = _params(native, 11, "l2")
+    g = _f((4, 7, 259), 43)
+    a = ctx.tgv2_denoise_adjoint(f, p, g, checkpoint_every=4)
+    ctx.set_override("fused", 0)
+    b = ctx.tgv2_denoise_adjoint(f, p, g, checkpoint_every=4)
+    for x, y in zip(a, b):
+        np.testing.assert_array_equal(x, y)

@@ -310,8 +310,9 @@ def test_unmasked_fused_sweep_counts_every_tile(ctx):
 
 
 # over 300000 voxels the fused masked sweep skips lanes: even and odd widths, whole rows
-# and x tiles (700, 515)
-@pytest.mark.parametrize("shape", [(40, 80, 100), (31, 90, 119), (5, 120, 700), (6, 100, 515)])
+# and x tiles (700, 515, and 259: the plan without a mask runs whole rows there)
+@pytest.mark.parametrize("shape", [(40, 80, 100), (31, 90, 119), (5, 120, 700), (6, 100, 515),
+                                   (9, 140, 259)])
 @pytest.mark.parametrize("mask", ["ball", "sparse", "slab", "random", "all", "none", "corners"])
 @pytest.mark.parametrize("storage", [0, 1])
 def test_masked_fused_lane_skipping(ctx, shape, mask, storage):
