@@ -340,6 +340,8 @@ struct TgvkFusedPlan {
 };
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan);
+int tgvk_masked_tx(const Geometry& g, int levels, const PlanOverrides& ov,
+                   const TgvkFusedPlan& plan);
 bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                        const uint8_t* rows, TgvkFusedPlan* plan, std::vector<FusedTile>* tiles);
 hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_t field_stride,

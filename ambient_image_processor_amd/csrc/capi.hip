@@ -1000,7 +1000,7 @@ amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
     if (fused && c->sp.active) {
         AMB_TRY(fused_active(c));
         std::vector<uint8_t> rows;
-        AMB_TRY(row_activity(c, c->kfplan.tx < c->g.w ? c->kfplan.tx : 0, &rows));
+        AMB_TRY(row_activity(c, tgvk_masked_tx(c->g, c->klevels, c->kov, c->kfplan), &rows));
         if (tgvk_masked_tiles(c->g, c->klevels, c->device, c->kov, rows.data(), &c->kfplan,
                               &c->tiles_host)) {
             AMB_TRY(upload_tiles(c));

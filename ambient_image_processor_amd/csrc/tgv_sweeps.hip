@@ -2283,8 +2283,9 @@ MaskedRows::MaskedRows(const Geometry& geom, int tile, const uint8_t* rows) : g(
                 b[y + 1] = a[y + 1] + acc;
             }
         }
-    const uint64_t chunks = uint64_t(g.h) * g.d * nbx *
-                            ((std::min(tx > 0 ? tx : g.w, g.w) + 63) / 64);
+    uint64_t chunks = 0;
+    for (int bx = 0; bx < nbx; ++bx)
+        chunks += uint64_t(g.h) * g.d * ((std::min(tx > 0 ? tx : g.w, g.w - bx * tx) + 63) / 64);
     dense = live * 20 > chunks * 19;
 }
 

@@ -1215,12 +1215,26 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     return true;
 }
 
-// The masked loop's band, z chunk and tiles (MaskedRows), the plan's rows or x tiles.
+// Tile columns of the masked loop (0: whole rows): tiles of 126 columns, whose rows
+// are two whole waves, instead of the plan's equal tiles, and for two levels
+// instead of whole rows of more than 1.5 such tiles (us per iteration, balls of 31 and
+// 50% of the voxels: order 4 256^3 1025 1418 -> 774 1133, 200^3 490 674 -> 439 652, 161 x
+// 145 x 140 186 271 / 177 283; 301 x 250 x 60 order 3 156 241 -> 131 211, order 4 268 374 -> 220
+// 346).  One level keeps whole rows (256^3 476 703 / 531 749).
+int tgvk_masked_tx(const Geometry& g, int levels, const PlanOverrides& ov,
+                   const TgvkFusedPlan& plan) {
+    const bool tiled = plan.tx < g.w;
+    if (ov.tgvk_fused_tx <= 0 && (tiled || (levels == 2 && g.w > 189))) return 126;
+    return tiled ? plan.tx : 0;
+}
+
+// The masked loop's band, z chunk and tiles (MaskedRows); false: the plan and its whole
+// grid, where nearly every row piece is active.
 // Against the whole grid with every lane loading and storing, order 3 (and for
 // order 4 against the two launches), us per iteration, balls of 3, 11, 31 and 50% of the
-// voxels: 256^3 841 847 843 840 -> 95 251 477 709 (1258 1380 1628 1916 -> 244 538 1029
-// 1419); 161 x 145 x 140 199 200 201 202 -> 23 58 103 150; 96 x 120 x 100 61 61 61 61 ->
-// 14 22 36 51; a random half 256^3 823 -> 786.
+// voxels: 256^3 841 847 843 840 -> 96 250 478 709 (1258 1380 1628 1916 -> 137 394 780
+// 1136); 161 x 145 x 140 199 200 201 202 -> 23 58 103 150; 96 x 120 x 100 61 61 61 61 ->
+// 14 22 36 51; a random half 256^3 823 -> 784.
 bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                        const uint8_t* rows, TgvkFusedPlan* plan, std::vector<FusedTile>* tiles) {
     int max_lds = 0, cus = 0;
@@ -1228,19 +1242,23 @@ bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOver
             hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return false;
-    const bool tiled = plan->tx < g.w;
-    const MaskedRows mr(g, tiled ? plan->tx : 0, rows);
+    const int tx = tgvk_masked_tx(g, levels, ov, *plan);
+    const MaskedRows mr(g, tx, rows);
+    if (mr.dense) return false;
+    TgvkFusedPlan p = *plan;
+    if (tx > 0) p.tx = tx;
     MaskedSearch m{};
     m.cus = cus;
     m.max_lds = size_t(max_lds);
-    m.lanes = tiled ? plan->tx + 2 : g.w;
+    m.lanes = tx > 0 ? tx + 2 : g.w;
     m.max_threads = kfused_max_threads(levels);
     m.max_waves = m.max_threads / 64;
     m.lds_row = size_t(11 + 11 * levels) * m.lanes * sizeof(float);
     m.fix_band = ov.tgvk_fused_ty > 0;
     m.fix_zchunk = ov.tgvk_fused_zchunk > 0;
-    if (!mr.dense) mr.search(m, &plan->ty, &plan->zchunk);
-    mr.tiles(plan->ty, plan->zchunk, tiles);
+    if (mr.search(m, &p.ty, &p.zchunk) < 0.0) return false;
+    mr.tiles(p.ty, p.zchunk, tiles);
+    *plan = p;
     return true;
 }
 
