@@ -2010,7 +2010,7 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
         *plan = bp;
         return true;
     }
-    // odd widths: one voxel per thread (the two- and four-voxel forms need
+    // odd widths: one voxel per thread but for OddIO's cases (the four-voxel form needs
     // lanes that lie wholly inside the row), whole rows only while bands of two
     // rows fit (four rows of lanes): bands of one row read each row three times
     // (257^3 per launch: 755 us, tiles of 126 columns 549 us; 255^3 with bands

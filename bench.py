@@ -461,13 +461,13 @@ def _tgv2_variant(args, f, mask, flags, workload, metric, data, cpu_note):
                    "voxel_iters_per_s": float(act) * args.iterations * args.steps / elapsed}
     kernels = sweep_kernels(prof, 4, n, planar=bool(flags & native.FLAG_PLANAR))
     swept, total = prof["fused_tiles"]
-    if "fused_sweep" in kernels and total and swept < total:
-        # a masked run: the fused launches move the bytes of the tiles they sweep
-        # (tiles of equal size here: the plans divide 256^3 evenly)
+    if "fused_sweep" in kernels and in_mask and total:
+        # a masked run: the fused launches need the bytes of the in-mask voxels (they
+        # also load their neighbours and the rest of the 128-B pieces around them)
         fs = kernels["fused_sweep"]
         fs["tiles_swept_fraction"] = swept / total
         fs["whole_volume_bytes_per_launch"] = fs["bytes_per_launch"]
-        fs["bytes_per_launch"] = int(round(fs["bytes_per_launch"] * swept / total))
+        fs["bytes_per_launch"] = int(round(fs["bytes_per_launch"] * in_mask["fraction"]))
         fs["gbs"] = fs["bytes_per_launch"] / (fs["avg_us"] * 1e-6) / 1e9
         fs.pop("two_sweep_equivalent_gbs", None)
     dom = max(kernels, key=lambda k: kernels[k]["avg_us"] * kernels[k]["launches"])
@@ -516,10 +516,9 @@ def masked_256(args):
     outside): the masked iteration (updates only where mask >= 1), the Poisson
     solve, the shading times the mask, the clamp and the background added back.
     The masked sweeps also read one active byte per voxel (not counted in the
-    algorithmic bytes); fused-sweep tiles that own no active voxel skip, so the
-    fused sweep's bytes are those of the tiles it sweeps (the first launch of a
-    call sweeps all of them), and the line also gives the rate over the in-mask
-    voxels."""
+    algorithmic bytes); the fused sweep skips tiles and lanes that no active voxel
+    needs, so its algorithmic bytes are those of the in-mask voxels, and the line
+    also gives the rate over these."""
     from ambient_image_processor_amd import native, phantoms
     n_side = args.size
     shape = (n_side, n_side, n_side)
@@ -828,6 +827,7 @@ def downsampled_512(args):
     f_dev, m_dev, u_dev, l_dev, r_dev = bufs
     ctx.upload(f_dev, f)
     ctx.upload(m_dev, mask)
+    in_mask = float(mask.mean())
     del f, mask
     elapsed, prof = timed(ctx, lambda: ctx.tgvk_deshade_downsampled_device(
         f_dev, shape, p, 0.5, alpha, m_dev, u_dev, l_dev, r_dev), args.steps, args.warmup)
@@ -836,6 +836,13 @@ def downsampled_512(args):
     value = float(ns) * iters * args.steps / elapsed
     resize_ms, resize_n = prof["resize"]
     kernels, dom = tgvk_kernels(prof, 1, ns)
+    if "tgvk_fused" in kernels:
+        # the masked fused launches need the bytes of the in-mask voxels (the resized
+        # mask's share is the input mask's but for its boundary)
+        fs = kernels["tgvk_fused"]
+        fs["bytes_per_launch"] = int(round(fs["bytes_per_launch"] * in_mask))
+        fs["gbs"] = fs["bytes_per_launch"] / (fs["avg_us"] * 1e-6) / 1e9
+        fs.pop("two_launch_equivalent_gbs", None)
     print(json.dumps({
         "metric": "voxel-iters/s (resized volume) downsampled TGV-k deshade 512^3 -> 256^3",
         "value": value, "unit": "voxel-iters/s", "n_gpus": 1, "steps": args.steps,
