@@ -520,6 +520,11 @@ amb_status begin(amb_context* c, amb_memory mem, const float* f, uint32_t w, uin
     return AMB_OK;
 }
 
+bool in_block(const void* p, const char* block, size_t bytes) {
+    const char* q = static_cast<const char*>(p);
+    return block && q >= block && q < block + bytes;
+}
+
 // Second copy of the 13 ping-ponged fields for the fused TGV2 sweep.  Field k
 // of the state lives either in the state block or in the second block;
 // c->alt[k] is set to the other one.  The second block is packed in the
@@ -533,8 +538,10 @@ amb_status ensure_alt(amb_context* c) {
     const size_t need = fstride * N_FUSED_FIELDS;
     auto main_at = [&](int k) { return static_cast<void*>(c->block + size_t(FUSED_FIELD_MAP[k]) * fstride); };
     if (need > c->alt_cap) {
-        for (int k = 0; k < N_FUSED_FIELDS; ++k)   // state must be in the state block
-            if (c->fields[FUSED_FIELD_MAP[k]] != main_at(k))
+        // the state must not lie in the block that goes (it lies in its own block, or in the
+        // TGV-k sweep's second copies after a TGV-k run that ended there)
+        for (int k = 0; k < N_FUSED_FIELDS; ++k)
+            if (in_block(c->fields[FUSED_FIELD_MAP[k]], c->alt_block, c->alt_cap))
                 return fail(AMB_ERR_NOT_SUPPORTED, "fused-sweep buffers out of step with the state");
         if (c->alt_block) AMB_HIP(hipFree(c->alt_block));
         c->alt_block = nullptr;

@@ -515,3 +515,24 @@ def test_tgvk_fused_masked_lane_skipping(ctx, shape, order, mask):
     ref = ctx.tgvk_deshade_masked(f, _params(native, 6), alpha, act.astype(np.uint8))
     for a, b in zip(out, ref):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("shape,alpha", [((70, 72, 72), (1.0, 2.0, 0.6)),
+                                         ((70, 72, 72), (1.0, 2.0, 0.6, 0.4))])
+@pytest.mark.parametrize("iterations", [2, 3])
+def test_tgv2_iterations_go_on_from_a_fused_tgvk_state(shape, alpha, iterations):
+    """amb_tgv2_iterate on the state a TGV-k run leaves, which after an odd number of
+    fused launches lies in the sweep's second copies: as after the two launches."""
+    from ambient_image_processor_amd import native
+    _say("tgv2 after tgvk", shape, len(alpha), iterations)
+    f = _f(shape, 38)
+    states = []
+    for fused in (1, 0):
+        with native.Context(0) as c:
+            c.set_override("tgvk_fused", fused)
+            c.profile(True)
+            c.tgvk_deshade(f, _params(native, iterations), alpha)
+            assert c.profile_counts()["tgvk_fused"] == (iterations - 1) * fused
+            c.iterate(3)
+            states.append(c.get_state())
+    np.testing.assert_array_equal(states[0], states[1])
