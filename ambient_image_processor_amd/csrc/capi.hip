@@ -135,6 +135,7 @@ struct amb_context {
     FusedPlan fplan_run{0, 0};   // the plan of the call in progress (masked: its own z chunk)
     bool iplan_ok = false;   // the 2-D loop marched along the image's rows
     FusedPlan iplan{0, 0};
+    bool looping = false;    // run() or tgvk_run() is between its first and last launch
     // energy / gap trace: every energy_interval iterations of a call (0 = off)
     // and after its last one; in the fused sweep's energy form where that
     // iteration's primal half runs fused, else the standalone pass
@@ -252,6 +253,43 @@ amb_status check_params(const amb_tgv_params* p) {
     return AMB_OK;
 }
 
+bool in_block(const void* p, const char* block, size_t bytes) {
+    const char* q = static_cast<const char*>(p);
+    return block && q >= block && q < block + bytes;
+}
+
+// Gives the fused TGV-k sweep's second copies back; a state that lies in them moves to
+// its own block.  false: there are none, or an iteration is running on them.
+bool release_tgvk_copies(amb_context* c) {
+    if (c->looping || (!c->kalt13_block && !c->kalt_block)) return false;
+    const size_t fstride = align_up(c->g.n() * 4, 256);
+    for (int m : FUSED_FIELD_MAP) {
+        if (!in_block(c->fields[m], c->kalt13_block, c->kalt13_cap)) continue;
+        void* home = c->block + size_t(m) * fstride;
+        if (hipMemcpyAsync(home, c->fields[m], c->g.n() * 4, hipMemcpyDeviceToDevice, c->stream) !=
+            hipSuccess)
+            return false;
+        c->fields[m] = home;
+    }
+    if (hipStreamSynchronize(c->stream) != hipSuccess) return false;
+    if (c->kalt13_block) (void)hipFree(c->kalt13_block);
+    if (c->kalt_block) (void)hipFree(c->kalt_block);
+    c->kalt13_block = c->kalt_block = nullptr;
+    c->kalt13_cap = c->kalt_cap = 0;
+    return true;
+}
+
+// A buffer that the call cannot do without.  Where it does not fit, the fused TGV-k
+// sweep's second copies, which the two launches do without, make room for it.
+hipError_t device_alloc(amb_context* c, void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory && release_tgvk_copies(c)) {
+        (void)hipGetLastError();   // answered here: no later launch reports it
+        e = hipMalloc(p, bytes);
+    }
+    return e;
+}
+
 // Allocate (or reuse) the state block for geometry g and the storage type.
 amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
     const size_t n = g.n();
@@ -259,10 +297,12 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
     const size_t fstride = align_up(n * elem, 256);
     const size_t need = fstride * N_FIELDS;
     if (need > c->cap_bytes) {
+        c->have_state = false;   // goes with its block
+        for (void*& p : c->fields) p = nullptr;
         if (c->block) AMB_HIP(hipFree(c->block));
         c->block = nullptr;
         c->cap_bytes = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->block), need));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->block), need));
         c->cap_bytes = need;
     }
     for (int k = 0; k < N_FIELDS; ++k) c->fields[k] = c->block + size_t(k) * fstride;
@@ -271,13 +311,13 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
         if (c->fblock) AMB_HIP(hipFree(c->fblock));
         c->fblock = nullptr;
         c->cap_n = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->fblock), fl * (1 + N_SCRATCH)));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->fblock), fl * (1 + N_SCRATCH)));
         c->cap_n = n;
     }
     c->f = reinterpret_cast<float*>(c->fblock);
     for (int k = 0; k < N_SCRATCH; ++k)
         c->scratch[k] = reinterpret_cast<float*>(c->fblock + fl * size_t(1 + k));
-    if (!c->fields_dev) AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->fields_dev), sizeof(void*) * N_FIELDS));
+    if (!c->fields_dev) AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->fields_dev), sizeof(void*) * N_FIELDS));
     AMB_HIP(hipMemcpyAsync(c->fields_dev, c->fields, sizeof(void*) * N_FIELDS,
                            hipMemcpyHostToDevice, c->stream));
     size_t pn = energy_partials_size(g);
@@ -288,10 +328,10 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
     if (pn > c->partials_cap) {
         if (c->partials) AMB_HIP(hipFree(c->partials));
         c->partials = nullptr;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->partials), pn * sizeof(double)));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->partials), pn * sizeof(double)));
         c->partials_cap = pn;
     }
-    if (!c->energy_out) AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->energy_out), 16 * sizeof(double)));
+    if (!c->energy_out) AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->energy_out), 16 * sizeof(double)));
     c->g = g;
     c->storage = storage;
     return AMB_OK;
@@ -339,7 +379,7 @@ amb_status ensure_axis(amb_context* c, int axis, int n, int precision) {
         free_axis(t);
         std::vector<float> eig(size_t(n) + 1);
         for (int k = 0; k <= n; ++k) eig[k] = float(host_cospi(double(float(k) / float(n))));
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&t.eig), (size_t(n) + 1) * 4));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&t.eig), (size_t(n) + 1) * 4));
         AMB_HIP(hipMemcpy(t.eig, eig.data(), (size_t(n) + 1) * 4, hipMemcpyHostToDevice));
         t.n = n;
     }
@@ -353,7 +393,7 @@ amb_status ensure_axis(amb_context* c, int axis, int n, int precision) {
     auto upload = [&](auto** dst, auto value) -> amb_status {
         typedef typename std::remove_reference<decltype(**dst)>::type T;
         T* dev = nullptr;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&dev), size_t(n) * n * sizeof(T)));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&dev), size_t(n) * n * sizeof(T)));
         const size_t rows = std::max<size_t>(1, (size_t(1) << 21) / size_t(n));
         std::vector<T> h;
         for (size_t r0 = 0; r0 < size_t(n); r0 += rows) {
@@ -377,7 +417,7 @@ amb_status ensure_axis(amb_context* c, int axis, int n, int precision) {
                 h[i + 512] = host_bf16_rne(float(v - double(host_bf16_to_float(h[i]))));
             }
         uint16_t* dev = nullptr;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&dev), h.size() * 2));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&dev), h.size() * 2));
         const hipError_t e = hipMemcpy(dev, h.data(), h.size() * 2, hipMemcpyHostToDevice);
         if (e != hipSuccess) { (void)hipFree(dev); return fail_hip(e, "hipMemcpy", __LINE__); }
         *dst = dev;
@@ -520,11 +560,6 @@ amb_status begin(amb_context* c, amb_memory mem, const float* f, uint32_t w, uin
     return AMB_OK;
 }
 
-bool in_block(const void* p, const char* block, size_t bytes) {
-    const char* q = static_cast<const char*>(p);
-    return block && q >= block && q < block + bytes;
-}
-
 // Second copy of the 13 ping-ponged fields for the fused TGV2 sweep.  Field k
 // of the state lives either in the state block or in the second block;
 // c->alt[k] is set to the other one.  The second block is packed in the
@@ -546,7 +581,7 @@ amb_status ensure_alt(amb_context* c) {
         if (c->alt_block) AMB_HIP(hipFree(c->alt_block));
         c->alt_block = nullptr;
         c->alt_cap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->alt_block), need));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->alt_block), need));
         c->alt_cap = need;
     }
     for (int k = 0; k < N_FUSED_FIELDS; ++k) {
@@ -642,7 +677,7 @@ amb_status ensure_active(amb_context* c) {
         if (c->act) AMB_HIP(hipFree(c->act));
         c->act = nullptr;
         c->act_cap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->act), need));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->act), need));
         c->act_cap = need;
     }
     return AMB_OK;
@@ -660,7 +695,7 @@ amb_status ensure_tiles(amb_context* c, size_t need) {
 }
 
 // The fused sweeps' bytes of the active set (launch_fused_active).
-amb_status fused_active(amb_context* c) {
+amb_status ensure_fused_active(amb_context* c) {
     const size_t bytes = align_up(c->g.n(), 256);
     if (bytes > c->fact_cap) {
         if (c->fact) AMB_HIP(hipFree(c->fact));
@@ -669,6 +704,10 @@ amb_status fused_active(amb_context* c) {
         AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->fact), bytes));
         c->fact_cap = bytes;
     }
+    return AMB_OK;
+}
+
+amb_status fused_active(amb_context* c) {
     AMB_HIP(launch_fused_active(c->stream, c->sp.active, c->g, c->fact));
     c->sp.fused_active = c->fact;
     return AMB_OK;
@@ -695,6 +734,13 @@ amb_status upload_tiles(amb_context* c) {
                                c->stream));
     return AMB_OK;
 }
+
+// While an iteration runs, the second copies stay where they are (device_alloc).
+struct Looping {
+    amb_context* c;
+    explicit Looping(amb_context* c_) : c(c_) { c->looping = true; }
+    ~Looping() { c->looping = false; }
+};
 
 // Runs the iteration with updates restricted to c->act; the restriction is
 // dropped again on every exit path.
@@ -734,8 +780,18 @@ amb_status sweep(amb_context* c, int which) {
 amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_iteration_callback cb,
                void* user, bool with_v) {
     const bool image = c->iplan_ok && c->z_zero;
-    const bool fused = (c->fused_ok || image) && iterations > 1;
+    bool fused = (c->fused_ok || image) && iterations > 1;
     if (fused) AMB_TRY(ensure_alt(c));
+    if (fused && c->sp.active) {
+        const amb_status s = ensure_fused_active(c);
+        if (s == AMB_ERR_OUT_OF_MEMORY) {   // the two sweeps need none
+            (void)hipGetLastError();
+            fused = false;
+        } else {
+            AMB_TRY(s);
+        }
+    }
+    const Looping looping(c);
     // the 2-D loop keeps v_z, p_z, q_zz, q_xz, q_yz at +0 in the state; with
     // their second copies cleared too, the fused sweep skips them
     c->sp.planar_zero_z = fused && c->sp.planar && c->storage == 0 && c->z_zero ? 1 : 0;
@@ -840,7 +896,7 @@ amb_status tgvk_begin(amb_context* c, amb_memory mem, const float* f, uint32_t w
         if (c->kblock) AMB_HIP(hipFree(c->kblock));
         c->kblock = nullptr;
         c->kcap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->kblock), need));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->kblock), need));
         c->kcap = need;
     }
     AMB_HIP(launch_zero_fill(c->stream, c->kblock, need));
@@ -849,14 +905,14 @@ amb_status tgvk_begin(amb_context* c, amb_memory mem, const float* f, uint32_t w
         if (c->klv_dev) AMB_HIP(hipFree(c->klv_dev));
         c->klv_dev = nullptr;
         c->klv_cap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->klv_dev), nt * sizeof(float*)));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->klv_dev), nt * sizeof(float*)));
         c->klv_cap = nt;
     }
     if (order > c->kalpha_cap) {
         if (c->kalpha_dev) AMB_HIP(hipFree(c->kalpha_dev));
         c->kalpha_dev = nullptr;
         c->kalpha_cap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->kalpha_dev), order * sizeof(float)));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->kalpha_dev), order * sizeof(float)));
         c->kalpha_cap = order;
     }
     // the tables stay in the context until the copies have run (next sync)
@@ -938,6 +994,20 @@ amb_status ensure_kalt(amb_context* c) {
     return AMB_OK;
 }
 
+// The buffers of a fused TGV-k run (second copies, masked: the active set's bytes).
+// *fused = false where they do not fit: the two launches, which need none, run then
+// (448 B per voxel instead of 236 at order 4).
+amb_status tgvk_fused_buffers(amb_context* c, bool* fused) {
+    amb_status s = c->sp.active ? ensure_fused_active(c) : AMB_OK;
+    if (s == AMB_OK) s = ensure_kalt13(c);
+    if (s == AMB_OK) s = ensure_kalt(c);
+    if (s != AMB_ERR_OUT_OF_MEMORY) return s;
+    (void)hipGetLastError();
+    (void)release_tgvk_copies(c);
+    *fused = false;
+    return AMB_OK;
+}
+
 // Primal half of TGV-k iteration k + dual half of iteration k + 1 into the
 // second copies, then swap the copies in the host tables.
 amb_status tgvk_fused_step(amb_context* c) {
@@ -994,10 +1064,10 @@ amb_status tgvk_upload_tables(amb_context* c) {
 amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
                     amb_iteration_callback cb, void* user) {
     float* const* F = reinterpret_cast<float* const*>(c->fields_dev);
-    const bool fused = c->kfused_ok && iterations > 1;
+    bool fused = c->kfused_ok && iterations > 1;
+    if (fused) AMB_TRY(tgvk_fused_buffers(c, &fused));
+    const Looping looping(c);
     if (fused) {
-        AMB_TRY(ensure_kalt13(c));
-        AMB_TRY(ensure_kalt(c));
         // earlier uploads from the host tables have run before they change
         AMB_HIP(hipStreamSynchronize(c->stream));
     }
@@ -1324,7 +1394,7 @@ AMB_API amb_status amb_context_destroy(amb_context* c) try {
 AMB_API amb_status amb_device_alloc(amb_context* c, size_t bytes, void** ptr) try {
     if (!c || !ptr) return fail(AMB_ERR_INVALID_ARGUMENT, "NULL argument");
     AMB_TRY(set_device(c));
-    AMB_HIP(hipMalloc(ptr, bytes));
+    AMB_HIP(device_alloc(c, ptr, bytes));
     return AMB_OK;
 } catch (...) {
     return guard_exception();
@@ -1643,6 +1713,9 @@ AMB_API amb_status amb_deshade_epilogue(amb_context* c, amb_memory mem, const fl
 static amb_status deshade_tail(amb_context* c, amb_memory mem, const float* mask, uint32_t flags,
                                uint32_t precision, bool masked, float* u, float* shading,
                                float* deshaded) {
+    // the tables first: making room for them may move the state (device_alloc)
+    AMB_TRY(check_precision(c->g, int(precision)));
+    AMB_TRY(ensure_tables(c, c->g, int(precision)));
     // v as FP32 device views (BF16 storage: converted into scratch[2..4])
     const float* v[3];
     for (int k = 0; k < 3; ++k) {
@@ -1814,7 +1887,7 @@ amb_status resize_workspace(amb_context* c, const size_t* bytes, int count, char
         if (c->rblock) AMB_HIP(hipFree(c->rblock));
         c->rblock = nullptr;
         c->rcap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->rblock), need));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->rblock), need));
         c->rcap = need;
     }
     size_t off = 0;
@@ -2043,7 +2116,7 @@ AMB_API amb_status amb_tgv2_denoise_adjoint(amb_context* c, amb_memory mem, cons
         if (c->adj_block) AMB_HIP(hipFree(c->adj_block));
         c->adj_block = nullptr;
         c->adj_cap = 0;
-        AMB_HIP(hipMalloc(reinterpret_cast<void**>(&c->adj_block), need));
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->adj_block), need));
         c->adj_cap = need;
     }
     char* base = c->adj_block;
