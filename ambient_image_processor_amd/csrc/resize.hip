@@ -205,15 +205,18 @@ __global__ __launch_bounds__(XD_LINES) void spline3_decompose_x_kernel(double* _
 // (fewer than four blocks per CU) keep the other kernels.  Reading 16 samples
 // ahead into registers was slower (660, 580 and 390 us).
 constexpr long RESIDENT_ROW = 1024, RESIDENT_COLUMN = 512;
+// A grid holds fewer than 2^32 work-items, 64 per group of lines here: more groups (from 2^28
+// rows or 2^29 columns on) take several launches.
+constexpr long RESIDENT_GRID = 0xffffffffL / 64;
 
 template <int AXIS0>
 __global__ __launch_bounds__(64) void spline3_decompose_resident_kernel(
     const float* __restrict__ in, double* __restrict__ c, Geometry g, int axis, int N,
-    uint32_t lines, Spline3Line sp) {
+    uint32_t lines, uint32_t first, Spline3Line sp) {
     constexpr int LINES = AXIS0 ? 4 : 8;
     extern __shared__ __align__(16) double rows[];   // [LINES][P]
     const int P = N | 1, lane = int(threadIdx.x);
-    const uint32_t l0 = xcd_contiguous(blockIdx.x, gridDim.x) * LINES;
+    const uint32_t l0 = (first + xcd_contiguous(blockIdx.x, gridDim.x)) * LINES;
     const uint32_t W = uint32_t(g.w), st = axis == 1 ? W : W * uint32_t(g.h);
     // y and z: lane -> column lane % 8 of the group, samples lane / 8 + 8 k
     const uint32_t l = l0 + uint32_t(lane & (LINES - 1));
@@ -496,13 +499,13 @@ hipError_t launch_resize_spline3(hipStream_t s, const float* in, Geometry gi, do
             sp.z2n0 = std::pow(sp.z, double(N - 1));
             const long lines = long(n) / N;
             if (resident) {
-                const dim3 grid{unsigned((lines + group - 1) / group), 1, 1};
-                if (axis == 0)
-                    hipLaunchKernelGGL(spline3_decompose_resident_kernel<1>, grid, dim3(64), lds, s,
-                                       in, coef, gi, axis, int(N), uint32_t(lines), sp);
-                else
-                    hipLaunchKernelGGL(spline3_decompose_resident_kernel<0>, grid, dim3(64), lds, s,
-                                       in, coef, gi, axis, int(N), uint32_t(lines), sp);
+                auto kern = axis == 0 ? spline3_decompose_resident_kernel<1>
+                                      : spline3_decompose_resident_kernel<0>;
+                const long groups = (lines + group - 1) / group;
+                for (long first = 0; first < groups; first += RESIDENT_GRID)
+                    hipLaunchKernelGGL(kern, dim3(unsigned(std::min(groups - first, RESIDENT_GRID))),
+                                       dim3(64), lds, s, in, coef, gi, axis, int(N),
+                                       uint32_t(lines), uint32_t(first), sp);
             } else if (axis == 0) {
                 hipLaunchKernelGGL(spline3_decompose_x_kernel,
                                    dim3(unsigned((lines + XD_LINES - 1) / XD_LINES)), dim3(XD_LINES),

@@ -185,3 +185,33 @@ def test_downsampled_cli(orc, tmp_path):
                          timeout=60)
     assert bad.returncode == 1 and "parameter:" in bad.stdout
     assert os.path.exists(prefix + "_deshaded.mha")
+
+
+# thin volumes with more groups of prefilter lines than one grid takes: over 2^28 rows (of 2
+# samples), over 2^29 columns (of 2 planes).  Separable integer data, so the result is
+# the product of the three lines' own.  Tolerance: each line is rounded to FP32 once, and so
+# is the result: 4 x 2^-24 and less.
+@pytest.mark.parametrize("src,dst", [((4097, 65536, 2), (1024, 64, 2)),
+                                     ((2, 8193, 65536), (2, 64, 64))])
+def test_resize_of_thin_volumes_with_many_lines(ctx, orc, src, dst):
+    import torch
+    from ambient_image_processor_amd import native
+    _say("resize many lines", src, "->", dst)
+    rng = np.random.default_rng(9)
+    lines = [rng.integers(1, 12, n).astype(np.float32) for n in src]
+    expected = np.ones((1, 1, 1))
+    for axis, (line, n) in enumerate(zip(lines, dst)):
+        shape = [1, 1, 1]
+        shape[axis] = len(line)
+        out = [1, 1, 1]
+        out[axis] = n
+        expected = expected * orc.resize_spline3(line.reshape(shape), tuple(out)).astype(np.float64)
+    z, y, x = [torch.from_numpy(a).to("cuda:0") for a in lines]
+    vol = z[:, None, None] * y[None, :, None] * x[None, None, :]
+    got = torch.empty(dst, device="cuda:0")
+    torch.cuda.synchronize()
+    native._check(native.lib().amb_resize_bspline3(
+        ctx._h, native.MEM_DEVICE, native._ptr(vol.data_ptr()), *native._dims(src),
+        native._ptr(got.data_ptr()), *native._dims(dst)))
+    err = np.abs(got.cpu().numpy() - expected) / np.abs(expected).max()
+    assert err.max() < 4 * 2.0 ** -24
