@@ -340,6 +340,8 @@ struct TgvkFusedPlan {
 };
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan);
+// whether a masked run uses the list of active tiles
+bool tgvk_masked_list(const Geometry& g);
 int tgvk_masked_tx(const Geometry& g, int levels, const PlanOverrides& ov,
                    const TgvkFusedPlan& plan);
 bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOverrides& ov,

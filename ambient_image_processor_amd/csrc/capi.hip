@@ -132,7 +132,7 @@ struct amb_context {
     void* alt[N_FUSED_FIELDS] = {};
     bool fused_ok = false;
     FusedPlan fplan{0, 0};
-    FusedPlan fplan_run{0, 0};   // the plan of the call in progress (masked: its own z chunk)
+    FusedPlan fplan_run{0, 0};   // the plan of the call in progress (masked: its own)
     bool iplan_ok = false;   // the 2-D loop marched along the image's rows
     FusedPlan iplan{0, 0};
     bool looping = false;    // run() or tgvk_run() is between its first and last launch
@@ -167,6 +167,7 @@ struct amb_context {
     void* kalt13[N_FUSED_FIELDS] = {};
     bool kfused_ok = false;
     TgvkFusedPlan kfplan{0, 0, 0};
+    TgvkFusedPlan kfplan_run{0, 0, 0};   // of the call in progress (masked: its own)
     // resampling and the downsampled deshade: one grow-only workspace
     char* rblock = nullptr;
     size_t rcap = 0;
@@ -713,6 +714,14 @@ amb_status fused_active(amb_context* c) {
     return AMB_OK;
 }
 
+// A buffer that the call can do without: where it does not fit, *have = false.
+amb_status optional_buffer(amb_status s, bool* have) {
+    if (s != AMB_ERR_OUT_OF_MEMORY) return s;
+    (void)hipGetLastError();   // answered here: no later launch reports it
+    *have = false;
+    return AMB_OK;
+}
+
 // Host copy of launch_row_activity's bytes for tiles of tx columns.
 amb_status row_activity(amb_context* c, int tx, std::vector<uint8_t>* rows) {
     rows->resize(row_activity_bytes(c->g, tx));
@@ -782,15 +791,8 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
     const bool image = c->iplan_ok && c->z_zero;
     bool fused = (c->fused_ok || image) && iterations > 1;
     if (fused) AMB_TRY(ensure_alt(c));
-    if (fused && c->sp.active) {
-        const amb_status s = ensure_fused_active(c);
-        if (s == AMB_ERR_OUT_OF_MEMORY) {   // the two sweeps need none
-            (void)hipGetLastError();
-            fused = false;
-        } else {
-            AMB_TRY(s);
-        }
-    }
+    if (fused && c->sp.active)   // (the two sweeps need none)
+        AMB_TRY(optional_buffer(ensure_fused_active(c), &fused));
     const Looping looping(c);
     // the 2-D loop keeps v_z, p_z, q_zz, q_xz, q_yz at +0 in the state; with
     // their second copies cleared too, the fused sweep skips them
@@ -803,19 +805,29 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
     // that own an active voxel, which alone are launched from the second fused
     // launch of the call on (the first one writes every voxel of the second
     // copy, after which both copies agree outside the active set: the masked
-    // sweeps store only active voxels)
+    // sweeps store only active voxels).  Only the rows' activity is fetched before the
+    // loop; the host searches the plan once the first fused launch is queued (0.2 -
+    // 0.7 ms, which the launches that need no list hide), and not at all in calls too short
+    // to use it.
     const FusedTile* tiles = nullptr;
     c->fplan_run = c->fplan;
     if (fused && c->sp.active) AMB_TRY(fused_active(c));
-    if (fused && c->sp.active && !image && !c->sp.planar_zero_z) {
-        std::vector<uint8_t> rows;
-        AMB_TRY(row_activity(c, fused_masked_tx(c->g, c->ov, c->fplan), &rows));
-        if (fused_masked_tiles(c->g, c->storage, c->device, c->ov, c->fplan, rows.data(),
-                               &c->fplan_run, &c->tiles_host)) {
-            AMB_TRY(upload_tiles(c));
-            tiles = reinterpret_cast<const FusedTile*>(c->tiles);
-        }
-    }
+    bool search = fused && c->sp.active && !image && !c->sp.planar_zero_z && iterations > 2;
+    std::vector<uint8_t> rows;
+    if (search)
+        AMB_TRY(optional_buffer(row_activity(c, fused_masked_tx(c->g, c->ov, c->fplan), &rows),
+                                &search));
+    auto masked_tiles = [&]() -> amb_status {
+        search = false;
+        FusedPlan plan;
+        bool have = fused_masked_tiles(c->g, c->storage, c->device, c->ov, c->fplan, rows.data(),
+                                       &plan, &c->tiles_host);
+        if (have) AMB_TRY(optional_buffer(upload_tiles(c), &have));
+        if (!have) return AMB_OK;
+        c->fplan_run = plan;
+        tiles = reinterpret_cast<const FusedTile*>(c->tiles);
+        return AMB_OK;
+    };
     bool need_dual = true, fused_ran = false;
     const uint32_t every = c->energy_interval;
     const bool en_fused = fused && !image && c->fen_ok && !c->sp.planar_zero_z;
@@ -828,6 +840,7 @@ amb_status run(amb_context* c, uint32_t iterations, uint32_t interval, amb_itera
         if (fused && !observed && it + 1 < iterations && (!want_e || en_fused)) {
             double* slot = nullptr;
             if (want_e) AMB_TRY(etrace_slot(c, &slot));
+            else if (fused_ran && search) AMB_TRY(masked_tiles());
             c->sp.tiles = fused_ran ? tiles : nullptr;
             AMB_TRY(fused_step(c, slot));
             fused_ran = true;
@@ -1034,8 +1047,9 @@ amb_status tgvk_fused_step(amb_context* c) {
     {
         ProfScope ps(c, P_TGVK_FUSED);
         AMB_HIP(launch_tgvk_fused(c->stream, t, lv, fstride, td - t, ld - lv, c->f,
-                                  c->sp.fused_active, c->sp.tiles, c->sp.ntiles, c->g, c->klevels, c->sp.tau, c->sp.sigma, c->sp.lambda,
-                                  c->sp.theta, c->kalpha_host.data(), c->sp.planar, c->kfplan));
+                                  c->sp.fused_active, c->sp.tiles, c->sp.ntiles, c->g, c->klevels,
+                                  c->sp.tau, c->sp.sigma, c->sp.lambda, c->sp.theta,
+                                  c->kalpha_host.data(), c->sp.planar, c->kfplan_run));
     }
     for (int k = 0; k < N_FUSED_FIELDS; ++k) std::swap(c->fields[FUSED_FIELD_MAP[k]], c->kalt13[k]);
     for (size_t m = 0; m < np; ++m)
@@ -1064,7 +1078,9 @@ amb_status tgvk_upload_tables(amb_context* c) {
 amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
                     amb_iteration_callback cb, void* user) {
     float* const* F = reinterpret_cast<float* const*>(c->fields_dev);
-    bool fused = c->kfused_ok && iterations > 1;
+    // (masked, two levels: the first fused launch sweeps the whole volume, where the two launches
+    // skip inactive voxels and are as fast: fused only where a listed one follows)
+    bool fused = c->kfused_ok && iterations > (c->sp.active && c->klevels > 1 ? 2u : 1u);
     if (fused) AMB_TRY(tgvk_fused_buffers(c, &fused));
     const Looping looping(c);
     if (fused) {
@@ -1074,16 +1090,24 @@ amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
     // masked loop: as in run()
     const FusedTile* tiles = nullptr;
     bool fused_ran = false;
-    if (fused && c->sp.active) {
-        AMB_TRY(fused_active(c));
-        std::vector<uint8_t> rows;
-        AMB_TRY(row_activity(c, tgvk_masked_tx(c->g, c->klevels, c->kov, c->kfplan), &rows));
-        if (tgvk_masked_tiles(c->g, c->klevels, c->device, c->kov, rows.data(), &c->kfplan,
-                              &c->tiles_host)) {
-            AMB_TRY(upload_tiles(c));
-            tiles = reinterpret_cast<const FusedTile*>(c->tiles);
-        }
-    }
+    c->kfplan_run = c->kfplan;
+    if (fused && c->sp.active) AMB_TRY(fused_active(c));
+    bool search = fused && c->sp.active && iterations > 2 && tgvk_masked_list(c->g);
+    std::vector<uint8_t> rows;
+    if (search)
+        AMB_TRY(optional_buffer(row_activity(c, tgvk_masked_tx(c->g, c->klevels, c->kov, c->kfplan),
+                                             &rows), &search));
+    auto masked_tiles = [&]() -> amb_status {
+        search = false;
+        TgvkFusedPlan plan = c->kfplan;
+        bool have = tgvk_masked_tiles(c->g, c->klevels, c->device, c->kov, rows.data(), &plan,
+                                      &c->tiles_host);
+        if (have) AMB_TRY(optional_buffer(upload_tiles(c), &have));
+        if (!have) return AMB_OK;
+        c->kfplan_run = plan;
+        tiles = reinterpret_cast<const FusedTile*>(c->tiles);
+        return AMB_OK;
+    };
     bool need_dual = true, stale = false;
     for (uint32_t it = 0; it < iterations; ++it) {
         const bool observed = cb && interval > 0 && it > 0 && it % interval == 0;
@@ -1093,6 +1117,7 @@ amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
                                      c->klevels, c->sp.sigma, c->sp.planar, c->kov));
         }
         if (fused && !observed && it + 1 < iterations) {
+            if (fused_ran && search) AMB_TRY(masked_tiles());
             c->sp.tiles = fused_ran ? tiles : nullptr;
             AMB_TRY(tgvk_fused_step(c));
             fused_ran = true;

@@ -335,3 +335,30 @@ def test_masked_fused_lane_skipping(ctx, shape, mask, storage):
     ref = ctx.tgv2_deshade_masked(f, p, act.astype(np.uint8))
     for a, b in zip(out, ref):
         np.testing.assert_array_equal(a, b)
+
+
+def _tiles(ctx, run):
+    """Tiles (swept, in the grids) of the fused launches of a call, and their number."""
+    ctx.profile(True)
+    ctx.profile_reset()
+    run()
+    launches = ctx.profile_counts()["fused_sweep"]
+    swept, total = ctx.profile_fused_tiles()
+    ctx.profile(False)
+    return swept, total, launches
+
+
+@pytest.mark.parametrize("shape", [(40, 80, 100), (31, 90, 119)])
+def test_masked_plan_comes_after_the_first_fused_launch(ctx, shape):
+    """The first fused launch of a masked call sweeps the iteration plan's whole grid; the
+    masked plan and its tiles are made after it, for the launches that use them (none in
+    two iterations, one of two in three)."""
+    from ambient_image_processor_amd import native
+    z, y, x = np.meshgrid(*(np.arange(n) / n - 0.5 for n in shape), indexing="ij")
+    act = (z * z + y * y + x * x <= 0.1).astype(np.uint8)
+    f = (0.4 + 0.2 * np.random.default_rng(6).standard_normal(shape)).astype(np.float32)
+    whole, grid, n = _tiles(ctx, lambda: ctx.tgv2_deshade(f, _params(native, 2)))
+    assert n == 1 and whole == grid
+    assert _tiles(ctx, lambda: ctx.tgv2_deshade_masked(f, _params(native, 2), act)) == (grid, grid, 1)
+    swept, total, n = _tiles(ctx, lambda: ctx.tgv2_deshade_masked(f, _params(native, 3), act))
+    assert n == 2 and total > grid and 0 < swept - grid < total - grid
