@@ -975,7 +975,7 @@ struct FusedPlane {
 // then holds the whole state after the primal half with p and q one dual half
 // ahead (the adjoint's recompute of a segment, one launch per iteration).
 template <class S, class I, int VX, int L2, int MK, int MAXT, int PF, int TL, int P2, int EN = 0,
-          int SB = 0, int OD = 0>
+          int SB = 0, int OD = 0, int SK = 0>
 __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     FusedFields ff, const float* __restrict__ f_, const uint8_t* __restrict__ act, Geometry g,
     float tau, float sigma, float lambda, float alpha0, float alpha1, float theta, int ty,
@@ -984,6 +984,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     static_assert(!EN || P2 == 0, "the in-sweep energy covers the 3-D loop");
     static_assert(!OD || (VX == 2 && P2 == 0 && std::is_same<S, StoreF32>::value), "odd rows");
     static_assert(!SB || P2 == 0, "u_bar / v_bar stores cover the 3-D loop");
+    static_assert(!SK || (MK && !EN && P2 == 0 && !PF), "skipping lanes");
     typedef typename S::T T;
     typedef typename std::conditional<OD != 0, OddIO, VecIO<S, VX>>::type V;
     typedef typename std::conditional<OD != 0, OddIO, VecIO<StoreF32, VX>>::type VF;
@@ -1004,14 +1005,19 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     // of the state agree outside the active set (the host passes tiles only then)
     // the grid is the list of tiles that own an active voxel (fused_masked_tiles),
     // and without the prefetch (whose registers would spill) lanes load and store
-    // only what the active voxels need (act bytes, fused_active_kernel)
-    constexpr bool LISTS = MK && !EN && P2 == 0, SKIPS = LISTS && !PF;
-    const bool listed = LISTS && tiles, skips = SKIPS && tiles;
+    // only what the active voxels need (act bytes, fused_active_kernel).  SK: that form
+    // (always listed); without the list a masked launch runs the form that skips nothing (60 x
+    // 200 x 401, every row active: 174 us per launch, 182 where the same kernel decides).
+    constexpr bool LISTS = MK && !EN && P2 == 0 && (PF || SK);
+    const bool listed = LISTS && tiles;
     const int tile = listed ? tiles[t].tile : t;
     const int tb = TL ? tile / nbx : tile;
     const int y0 = (tb % nb) * ty;
-    const int z0 = listed ? tiles[t].z0 : (tb / nb) * zchunk;
-    const int z1 = listed ? tiles[t].z1 : min(z0 + zchunk, D);
+    // (The tile's planes as offsets, and the act bytes loaded with their plane below: with the
+    // planes selected as values, or load_act's own branch, the prefetch form needs 17 registers
+    // more and spills: 256^3, every row active, 388 us per launch, 368 without.)
+    const int zt = (tb / nb) * zchunk, z0 = zt + (listed ? tiles[t].z0 - zt : 0);
+    const int z1 = min(z0 + (listed ? tiles[t].z1 - tiles[t].z0 : zchunk), D);
     const int y = IMG ? y0 + r : y0 - 1 + r;
     const int xb = TL ? (tile % nbx) * tx - VX + lane * VX : lane * VX;   // global x of element 0
     // (W % VX == 0 and x0 % VX == 0: a lane lies wholly inside or outside the volume;
@@ -1086,9 +1092,9 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     constexpr int GL = std::min(64, 128 / (VX * int(sizeof(T))));
     const int gs = (int(threadIdx.x) & 63) & ~(GL - 1);
     auto group = [&](uint32_t a) {
-        return !skips || ((__ballot(a != 0) >> gs) << (64 - GL)) != 0;
+        return !SK || ((__ballot(a != 0) >> gs) << (64 - GL)) != 0;
     };
-    if (SKIPS) { act_0 = load_act(zs); act_1 = load_act(zs + 1); }
+    if (SK) { act_0 = load_act(zs); act_1 = load_act(zs + 1); }
     const bool live_z = group(act_0);
     if (!SKZ && rowin && zs < D && live_z) {
         const I i = I(zs) * plane + col;
@@ -1118,6 +1124,7 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
             zero(P.u); zero(P.f);
 #pragma unroll
             for (int k = 0; k < 3; ++k) { zero(P.v[k]); zero(P.qnn[k]); }
+            if (!SK) P.act = 0xffffffffu;
         }
         if (CLAMP || ok) {
             const I i = !CLAMP || ok ? I(zz) * plane + col : I(0);
@@ -1142,9 +1149,9 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
                 V::ld(src[G_QZZ], j, P.qnn[0], odd); V::ld(src[G_QXZ], j, P.qnn[1], odd);
                 if (!IMG) V::ld(src[G_QYZ], j, P.qnn[2], odd);
             }
+            if (!SK) P.act = MK ? load_active<VX>(act, i, odd) : 0xffffffffu;
         }
-        if (SKIPS) { P.act = act_0; act_0 = act_1; act_1 = load_act(zz + 2); }
-        else P.act = load_act(zz);
+        if (SK) { P.act = act_0; act_0 = act_1; act_1 = load_act(zz + 2); }
     };
 
     FusedPlane<VX> P;
@@ -1730,10 +1737,12 @@ hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Ge
     size_t lds = (size_t(EN ? 12 : 8) * RT * row + size_t(EN ? 12 : 8) * RT * (L + 1)) * sizeof(float);
     if (EN) lds = std::max(lds, size_t(16 * 10 * sizeof(double)));   // the block reduction
     if (OD && g.w < 3) return hipErrorInvalidValue;
+    const bool list = MK && !EN && P2 == 0 && p.tiles;
     auto kern = fused_sweep_kernel<S, I, VX, L2, MK, MAXT, PF, TL, P2, EN, SB, OD>;
+    if constexpr (MK && !EN && P2 == 0 && !PF)
+        if (list) kern = fused_sweep_kernel<S, I, VX, L2, MK, MAXT, PF, TL, P2, EN, SB, OD, 1>;
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
-    const bool list = MK && !EN && P2 == 0 && p.tiles;
     if (list && p.ntiles == 0) return hipSuccess;   // no active voxel
     hipLaunchKernelGGL(kern, dim3(list ? unsigned(p.ntiles) : unsigned(nbx * nb * nc)), dim3(L * RT), lds, s, ff,
                        f, MK ? p.fused_active : nullptr, g, p.tau,
@@ -2348,7 +2357,8 @@ void MaskedRows::tiles(int band, int zchunk, std::vector<FusedTile>* out) const 
 
 // Plan and tiles of the masked fused TGV2 sweep.  The iteration plan where nearly
 // every 64-voxel chunk of the rows holds an active voxel, so that skipping lanes gives
-// less than the prefetch, and up to MASKED_SMALL voxels, which the latency of a plane
+// less than the prefetch, or than it costs (no prefetch: false, the whole grid without the
+// list), and up to MASKED_SMALL voxels, which the latency of a plane
 // step bounds; otherwise no prefetch and two voxels per lane (four with 64-bit
 // offsets).  Odd widths: one voxel per lane; with FP32 fields two where their cost is under
 // 0.4 of that (half the lanes, but twice the bytes per step, stores of single voxels at the
@@ -2396,6 +2406,7 @@ bool fused_masked_tiles(const Geometry& g, int storage, int device, const PlanOv
         return mr.search(m, &p->ty, &p->zchunk);
     };
     *plan = base;
+    if (mr.dense && !base.pf) return false;
     if (ov.fused_pf != 1 && g.n() > MASKED_SMALL && !mr.dense) {
         const bool odd = fused_odd_ok(g, storage, index64) && mr.tx % 2 == 0 && ov.fused_vx <= 0;
         const int vx = odd ? 1 : base.vx == 4 && !index64 && ov.fused_vx <= 0 ? 2 : base.vx;

@@ -362,3 +362,22 @@ def test_masked_plan_comes_after_the_first_fused_launch(ctx, shape):
     assert _tiles(ctx, lambda: ctx.tgv2_deshade_masked(f, _params(native, 2), act)) == (grid, grid, 1)
     swept, total, n = _tiles(ctx, lambda: ctx.tgv2_deshade_masked(f, _params(native, 3), act))
     assert n == 2 and total > grid and 0 < swept - grid < total - grid
+
+
+@pytest.mark.parametrize("shape,lists", [((40, 80, 100), True), ((31, 90, 119), False)])
+def test_mask_of_nearly_every_row_piece(ctx, shape, lists):
+    """A mask that leaves under 5% of the row pieces inactive keeps the iteration plan; without
+    the prefetch (odd width) also its whole grid, as skipping would cost more than it gives."""
+    from ambient_image_processor_amd import native
+    act = np.ones(shape, np.uint8)
+    act[:2, :, :] = 0           # the first planes ...
+    act[2:, :, :] = 1
+    act[:2, shape[1] // 2:, :] = 1   # ... of half the rows: 2.5 and 3.3%
+    f = (0.4 + 0.2 * np.random.default_rng(7).standard_normal(shape)).astype(np.float32)
+    ctx.set_override("fused_zchunk", 2)
+    swept, total, n = _tiles(ctx, lambda: ctx.tgv2_deshade_masked(f, _params(native, 5), act))
+    assert n == 4 and (swept < total) == lists
+    out = ctx.tgv2_deshade_masked(f, _params(native, 5), act)
+    ctx.set_override("fused", 0)
+    for a, b in zip(out, ctx.tgv2_deshade_masked(f, _params(native, 5), act)):
+        np.testing.assert_array_equal(a, b)
