@@ -2019,18 +2019,22 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
         *plan = bp;
         return true;
     }
-    // odd widths: one voxel per thread but for OddIO's cases (the four-voxel form needs
-    // lanes that lie wholly inside the row), whole rows only while bands of two
-    // rows fit (four rows of lanes): bands of one row read each row three times
-    // (257^3 per launch: 755 us, tiles of 126 columns 549 us; 255^3 with bands
-    // of two rows 431 us, of one row 662 us, tiles 542 us)
-    // odd widths, FP32: two voxels per lane (OddIO) where whole rows then fit bands of
-    // three rows and one voxel per lane would run tiles, or where the override asks
-    // (per launch, against one voxel: 257^3 472 / 562 us, 301 x 250 x 60 121 / 154;
-    // narrower 181 x 217 x 181 201 / 185, 161 x 145 x 140 89.6 / 90; wider, in tiles 2047 x
-    // 128 x 48 392 / 366: the row's last lane stores by itself)
+    // Odd widths: one voxel per thread (the four-voxel form needs lanes that lie wholly
+    // inside the row), whole rows only while bands of two rows fit (four rows of lanes):
+    // bands of one row read each row three times (257^3 per launch: 755 us, tiles of 126
+    // columns 549 us; 255^3 with bands of two rows 431 us, of one row 662 us, tiles 542 us).
+    // With FP32 fields two voxels per lane (OddIO) where whole rows then fit bands of three
+    // rows, one voxel per lane would run tiles, and HBM bounds the launch: its 108 B per voxel
+    // exceed the 256 MB Infinity Cache.  Per launch, against one voxel: 257^3 472 / 562 us, 301 x
+    // 250 x 60 121 / 154; 36 of 70 shapes of 257 to 305 columns x 2 to 400 rows and planes lost up
+    // to 1.6x, all but one of them under 2.2 M voxels (271 x 9 x 53 22 / 13, 291 x 294 x 25 79 / 67,
+    // 279 x 219 x 38 73 / 76, 295 x 250 x 34 73 / 83).  Narrower 181 x 217 x 181 201 / 185, 161 x
+    // 145 x 140 89.6 / 90; wider, in tiles 2047 x 128 x 48 392 / 366: the row's last lane stores by
+    // itself.
+    constexpr size_t ODD_WHOLE_VOXELS = 2200000;
     const bool odd2 = fused_odd_ok(g, storage, big_index) &&
-                      (want_vx == 2 || (4 * g.w > 1024 && 5 * ((g.w + 1) / 2) <= 768));
+                      (want_vx == 2 || (4 * g.w > 1024 && 5 * ((g.w + 1) / 2) <= 768 &&
+                                        g.n() >= ODD_WHOLE_VOXELS));
     for (int vx : {1, 2, 4}) {
         if (want_vx && vx != want_vx) continue;
         if (want_tx > 0) break;   // x tiles forced

@@ -365,3 +365,27 @@ def test_fused_odd_two_voxels_adjoint(ctx):
     b = ctx.tgv2_denoise_adjoint(f, p, g, checkpoint_every=4)
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
+
+
+def _grid(ctx, f):
+    from ambient_image_processor_amd import native
+    ctx.profile(True)
+    ctx.profile_reset()
+    out = ctx.tgv2_deshade(f, _params(native, 2, "l1"))
+    grid = ctx.profile_fused_tiles()[1]
+    ctx.profile(False)
+    return grid, out
+
+
+@pytest.mark.parametrize("shape,whole", [((21, 165, 261), False), ((84, 47, 283), False),
+                                         ((38, 219, 279), True)])
+def test_odd_rows_run_whole_where_hbm_bounds_the_launch(ctx, shape, whole):
+    """257 to 305 columns: whole rows of two-voxel lanes from 2.2 M voxels on, the one-voxel
+    lanes' tiles below; the same results."""
+    f = _f(shape, 57)
+    grid, out = _grid(ctx, f)
+    ctx.set_override("fused_vx", 1)
+    tiles, ref = _grid(ctx, f)
+    assert (grid != tiles) == whole
+    for a, b in zip(out, ref):
+        np.testing.assert_array_equal(a, b)
