@@ -1753,10 +1753,10 @@ hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Ge
     return hipGetLastError();
 }
 
-// The energy form (EN = 1): 32-bit offsets, the 3-D loop, two voxels per
-// thread (FP32 also on odd widths: 161 x 145 x 140 174 us per launch, one voxel 239), no next-plane prefetch, blocks of at most EN_THREADS threads (two
-// waves per SIMD: the FP64 sums and the carried u, v need the registers); the
-// plan comes from fused_energy_plan.
+// The energy form (EN = 1): 32-bit offsets, the 3-D loop, two voxels per thread (one on
+// odd widths with BF16 fields and in the smallest volumes), no next-plane prefetch, blocks
+// of at most EN_THREADS threads (two waves per SIMD: the FP64 sums and the carried u, v
+// need the registers); the plan comes from fused_energy_plan.
 constexpr int EN_THREADS = 512;
 
 template <class S, int MK>
@@ -2185,22 +2185,75 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
     return true;
 }
 
+// Energy form on odd widths with FP32 fields (OddIO): whole rows or tiles of 124 columns (64
+// lanes), the band and z chunk with the least
+//   (rounds of resident blocks) (zc + 2) + 0.12 (waves on the busiest CU) (zc + 1)
+//     + 0.115 (its owned waves) zc + 0.0022 blocks
+// in units of a plane step's latency (200 VGPRs: a block of up to four waves leaves room for a
+// second one; one more launch sums the blocks' results).  The iteration plan's chunk and band do not fit this form, which is bound by
+// its FP64 sums: they gave too few blocks or one-row bands (us per launch, one voxel per
+// lane / two voxels with the iteration plan's band and chunk / this plan: 279 x 219 x 88 359 /
+// 483 / 297, 373 x 96 x 96 195 / 230 / 165, 133 x 281 x 95 340 / 196 / 166, 21 x 27 x 16 14.4 /
+// 19.0 / 13.5).  On 160 shapes of 8 k to 10 M voxels the model's mean error is 3% and its plans
+// are 1.31x the one-voxel form's speed in the mean, 0.93x at worst (83 x 143 x 178 91 / 98).
+// Chunks: those that give every CU k = 1 .. 8 blocks.
+static bool odd_energy_plan(const Geometry& g, int cus, size_t max_lds, const PlanOverrides& ov,
+                            const FusedPlan& base, FusedPlan* plan) {
+    double best = 1e300;
+    // Volumes whose planes one voxel per lane covers in one round of one-plane chunks: that form's
+    // step is the shorter one (151 x 18 x 9 16.1 us, 18.5 with two voxels; 21 x 27 x 16 14.4 /
+    // 16.5), in the lowest bands that do it.
+    if (ov.fused_vx != 2 && ov.fused_ty <= 0 && ov.fused_zchunk <= 0)
+        for (int ty = 1; g.w * (ty + 2) <= EN_THREADS && ty <= g.h; ++ty)
+            if (long((g.h + ty - 1) / ty) * g.d <= cus) {
+                if (fused_lds_floats<1>(g.w, ty, 1) * sizeof(float) > max_lds) break;
+                *plan = FusedPlan{ty, 1, 0, 1, 0};
+                return true;
+            }
+    for (int tx : {0, 124}) {
+        const int lanes = tx ? tx / 2 + 2 : (g.w + 1) / 2, nbx = tx ? (g.w + tx - 1) / tx : 1;
+        if (tx >= g.w || 3 * lanes > EN_THREADS) continue;
+        const int cap = std::min(EN_THREADS / lanes - 2, ov.fused_ty > 0 ? std::min(base.ty, g.h) : g.h);
+        for (int ty = 1; ty <= cap; ty += std::max(1, ty / 8)) {
+            if (fused_lds_floats<2>(2 * lanes, ty, 1) * sizeof(float) > max_lds) break;
+            const int waves = (lanes * (ty + 2) + 63) / 64, per_cu = waves <= 4 ? 2 : 1;
+            const long nb = long((g.h + ty - 1) / ty) * nbx;
+            int last = 0;
+            for (int k = 1; k <= 8; ++k) {
+                const long ncz = std::max(1L, std::min(long(g.d), long(k) * cus / nb));
+                const int zc = ov.fused_zchunk > 0 ? base.zchunk : int((g.d + ncz - 1) / ncz);
+                if (zc == last) continue;
+                last = zc;
+                const long blocks = nb * ((g.d + zc - 1) / zc), on_cu = (blocks + cus - 1) / cus;
+                const long rounds = (blocks + long(cus) * per_cu - 1) / (long(cus) * per_cu);
+                const double cost = double(rounds) * (zc + 2) + 0.12 * double(on_cu * waves) * (zc + 1) +
+                                    0.115 * double(on_cu * ty * lanes) / 64.0 * zc + 0.0022 * double(blocks);
+                if (cost < best) { best = cost; *plan = FusedPlan{ty, zc, 0, 2, tx}; }
+            }
+        }
+    }
+    return best < 1e300;
+}
+
 // The energy form's plan (results do not depend on the plan): two voxels per
 // thread (one on odd widths with BF16 fields), no prefetch, the iteration plan's z chunk; whole
 // rows in bands of up to the iteration plan's height while three rows fit
 // EN_THREADS threads, else x tiles of 124 columns (64 lanes) in bands of up to
-// 6 rows (one voxel per thread: 126 columns, 128 lanes, bands of 2 rows).  None for
-// 64-bit offsets.
+// 6 rows (one voxel per thread: 126 columns, 128 lanes, bands of 2 rows); odd widths with
+// FP32 fields: odd_energy_plan.  None for 64-bit offsets.
 bool fused_energy_plan(const Geometry& g, int storage, int device, const PlanOverrides& ov,
                        const FusedPlan& base, FusedPlan* plan) {
     if (needs_index64(g, ov) || base.ty < 1) return false;
     FusedPlan e = base;
     e.pf = 0;
-    int max_lds = 0;
+    int max_lds = 0, cus = 0;
     if (hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) !=
-        hipSuccess)
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
         return false;
-    if (g.w % 2 != 0 && !fused_odd_ok(g, storage, false)) {
+    if (fused_odd_ok(g, storage, false))
+        return odd_energy_plan(g, cus, size_t(max_lds), ov, base, plan);
+    if (g.w % 2 != 0) {
         e.vx = 1;
         if (base.tx == 0 && 3 * g.w <= EN_THREADS) {
             e.tx = 0;
@@ -2218,20 +2271,17 @@ bool fused_energy_plan(const Geometry& g, int storage, int device, const PlanOve
         return true;
     }
     e.vx = 2;
-    const int lanes = (g.w + 1) / 2;
-    if (base.tx == 0 && 3 * lanes <= EN_THREADS) {
+    if (base.tx == 0 && 3 * (g.w / 2) <= EN_THREADS) {
         e.tx = 0;
-        e.ty = EN_THREADS / lanes - 2;
-        if (base.vx != 1) e.ty = std::min(base.ty, e.ty);
+        e.ty = std::min(base.ty, EN_THREADS / (g.w / 2) - 2);
     } else {
         e.tx = base.tx > 0 && base.vx == 2 ? base.tx : 124;
-        if (base.vx == 1 && e.tx >= g.w) return false;
         if (e.tx >= g.w) e.tx = 124;
         e.ty = std::min(std::min(base.tx > 0 ? base.ty : 6, 6), EN_THREADS / (e.tx / 2 + 2) - 2);
     }
     e.ty = std::min(e.ty, g.h);
     if (e.ty < 1) return false;
-    const int row = e.tx > 0 ? e.tx + 4 : 2 * lanes;
+    const int row = e.tx > 0 ? e.tx + 4 : g.w;
     if (fused_lds_floats<2>(row, e.ty, 1) * sizeof(float) > size_t(max_lds)) return false;
     *plan = e;
     return true;

@@ -165,3 +165,39 @@ def test_trace_256_headline_configuration(ctx):
     ctx.iterate(75)
     ref = ctx.energy()
     assert _close(trace[2, 1:], ref, abs(ref[0])), (trace[2], ref)
+
+
+# odd widths with FP32 fields: one voxel per lane for the smallest volumes (33, 63), else two in
+# whole rows (33 x 40 x 70, 129 x 30 x 40) or tiles of 124 columns (from 341 columns on):
+# ragged ones (401), a last tile of one column, whose voxel is also the halo of the tile
+# before (373), and one of two (499)
+ODD_SHAPES = [(9, 10, 33), (6, 8, 63), (70, 40, 33), (40, 30, 129), (6, 11, 401), (5, 9, 373),
+              (4, 7, 499)]
+
+
+@pytest.mark.parametrize("shape", ODD_SHAPES)
+@pytest.mark.parametrize("data_term", ["l1", "l2"])
+def test_trace_on_odd_widths(ctx, orc, shape, data_term):
+    test_trace_matches_standalone_pass(ctx, orc, shape, data_term, 0)
+
+
+@pytest.mark.parametrize("shape", [(70, 40, 33), (6, 11, 401), (5, 9, 373)])
+def test_masked_trace_on_odd_widths(ctx, shape):
+    """The masked energy form with two voxels per lane: every row against the masked loop of
+    that many iterations and the standalone pass."""
+    from ambient_image_processor_amd import native
+    f = _volume(shape, seed=11)
+    active = (np.random.default_rng(11).random(shape) < 0.6).astype(np.uint8)
+    ctx.set_energy_interval(4)
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.tgv2_deshade_masked(f, _params(native, 14, "l1"), active)
+    assert ctx.profile_counts()["fused_sweep_energy"] == 3
+    ctx.profile(False)
+    trace = ctx.energy_trace()
+    ctx.set_energy_interval(0)
+    assert [int(c) for c in trace[:, 0]] == [4, 8, 12, 14]
+    for row in trace:
+        ctx.tgv2_deshade_masked(f, _params(native, int(row[0]), "l1"), active)
+        ref = ctx.energy()
+        assert _close(row[1:], ref, max(abs(ref[0]), 1e-30)), (row, ref)
