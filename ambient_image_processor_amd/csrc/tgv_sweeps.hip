@@ -996,9 +996,11 @@ __global__ __launch_bounds__(MAXT) void fused_sweep_kernel(
     const int RWD = L * VX;               // floats per LDS row
     const int lane = int(threadIdx.x) % L, r = int(threadIdx.x) / L;
     const int nbx = TL ? (W + tx - 1) / tx : 1, nb = (H + ty - 1) / ty;
-    // (FP32 with the prefetch and more blocks than CUs, not a multiple of 8: the plain
-    // order; 50 x 139 x 110 in 481 blocks 29.7 us, contiguous 32.6; 142 x 232 x 297 in 507
-    // 250 / 257)
+    // (With the prefetch and more blocks than the 256 CUs, not a multiple of 8: the plain
+    // order.  The two orders are equal in the mean there, 23 shapes 0.94 to 1.12x, so the
+    // one that came first stays.  Without the prefetch contiguous ranges win there, 98 shapes
+    // 1.08x in the mean, 0.89 at worst (launches of 12 us), 1.37 at best; up to 256 blocks they
+    // win everywhere.)
     const bool plain = PF && (gridDim.x & 7) != 0 && gridDim.x > 256 && !(MK && tiles);
     const int t = plain ? int(blockIdx.x) : xcd_tile(blockIdx.x, gridDim.x);
     // masked loop: voxels that are not active keep their values, so once both copies
@@ -1814,19 +1816,22 @@ hipError_t fused_shape(hipStream_t s, const FusedFields& ff, const float* f, Geo
                              : fused_launch<S, I, 4, 0, MK, 512, PF>(s, ff, f, g, p, plan);
 }
 
-// Odd widths, FP32 fields: two voxels per lane (OddIO).
+// Odd widths, FP32 fields: two voxels per lane (OddIO).  Tiles come from the masked plan only
+// (fused_masked_tiles), which has no prefetch.
 template <int MK, int SB = 0>
 hipError_t fused_odd(hipStream_t s, const FusedFields& ff, const float* f, Geometry g,
                      const SweepParams& p, const FusedPlan& plan) {
     typedef StoreF32 S;
     typedef uint32_t I;
-    const int lanes = plan.tx > 0 ? plan.tx / 2 + 2 : (g.w + 1) / 2;
-    const bool pf = plan.pf && lanes * (plan.ty + 2) <= 768;
+    const bool pf = plan.pf && (g.w + 1) / 2 * (plan.ty + 2) <= 768;
     auto go = [&](auto L2C) {
         constexpr int L2 = decltype(L2C)::value;
-        if (plan.tx > 0)
-            return pf ? fused_launch<S, I, 2, L2, MK, 768, 1, 1, 0, 0, SB, 1>(s, ff, f, g, p, plan)
-                      : fused_launch<S, I, 2, L2, MK, 1024, 0, 1, 0, 0, SB, 1>(s, ff, f, g, p, plan);
+        if (plan.tx > 0) {
+            if constexpr (MK)
+                if (!plan.pf)
+                    return fused_launch<S, I, 2, L2, MK, 1024, 0, 1, 0, 0, SB, 1>(s, ff, f, g, p, plan);
+            return hipErrorInvalidValue;
+        }
         return pf ? fused_launch<S, I, 2, L2, MK, 768, 1, 0, 0, 0, SB, 1>(s, ff, f, g, p, plan)
                   : fused_launch<S, I, 2, L2, MK, 1024, 0, 0, 0, 0, SB, 1>(s, ff, f, g, p, plan);
     };
@@ -1925,9 +1930,13 @@ hipError_t fused_bars_dispatch(hipStream_t s, const FusedFields& ff, const float
 
 }  // namespace
 
+// Odd widths whose rows the two-voxel forms can run (OddIO).
+static bool fused_odd_ok(const Geometry& g, int storage, bool index64) {
+    return g.w % 2 != 0 && g.w >= 3 && storage == 0 && !index64 && g.d > 1;
+}
+
 // Small volumes (FP32 fields, at most SMALL_VOXELS or SMALL_VOXELS_ODD, 8 planes
-// or more): the launch
-// is bound by the latency of a block's zc + 2 dependent plane steps (load, two
+// or more): the launch is bound by the latency of a block's zc + 2 dependent plane steps (load, two
 // barriers, two chains of square roots and divisions), not by bandwidth, so the
 // plan minimises, in units of one step's latency,
 //   (zc + 2) + c (waves on the busiest CU) (zc + 1) + e (waves of a block) (zc + 2),
@@ -1943,11 +1952,6 @@ hipError_t fused_bars_dispatch(hipStream_t s, const FusedFields& ff, const float
 // at 34x32x250), and so do images and slabs of fewer than 8 planes (500^2: 17.1
 // / 11.3).
 constexpr size_t SMALL_VOXELS = 400000, SMALL_VOXELS_ODD = 170000;
-
-// Odd widths whose rows the two-voxel forms can run (OddIO).
-static bool fused_odd_ok(const Geometry& g, int storage, bool index64) {
-    return g.w % 2 != 0 && g.w >= 3 && storage == 0 && !index64 && g.d > 1;
-}
 
 bool small_fused_plan(const Geometry& g, int cus, int max_lds, FusedPlan* plan) {
     const bool even = g.w % 2 == 0;
@@ -2416,8 +2420,10 @@ void MaskedRows::tiles(int band, int zchunk, std::vector<FusedTile>* out) const 
 // step bounds; otherwise no prefetch and two voxels per lane (four with 64-bit
 // offsets).  Odd widths: one voxel per lane; with FP32 fields two where their cost is under
 // 0.4 of that (half the lanes, but twice the bytes per step, stores of single voxels at the
-// row ends and coarser skipping: 181 x 217 x 181, costs 0.36 and 0.55 of one voxel's, 114 /
-// 135 and 32 / 23 us; 161 x 145 x 140, 0.50, 63 / 47).
+// row ends and coarser skipping).  On 44 shapes of 0.3 to 16 M voxels x 8 balls the choice is
+// the better form but for 6% at worst (255 x 200 x 200, radius 0.25: 71 / 67 us); one voxel
+// throughout is up to 1.17x slower (255 x 247 x 150, radius 0.36: 109 / 128), two 1.3x in the
+// mean.
 // Against the iteration plan and its prefetch, tiles skipped inside the full grid
 // (which left the XCDs unevenly loaded) and every lane of the others loading and
 // storing (us per launch, balls of 3, 11, 31 and 50% of the voxels and a random half):
