@@ -1142,13 +1142,15 @@ int tgvk_blocks(const Geometry& g, const PlanOverrides& ov, int* zchunk) {
 // Plan of the fused TGV-k sweep (one or two levels): blocks of up to 1024 or 768
 // threads (one per CU: they hold all its registers), all LDS arrays within the
 // device's limit.  Whole rows (tx = W), with the tallest band that fits, while a
-// band of two rows fits, or one of one row that fills the block (W = 256, two
-// levels): rows then start on cache lines and halo rows fall on whole waves,
-// which skip the dual half.  Other rows run in equal tiles of at most 128 columns
+// band of two rows fits: rows then start on cache lines and halo rows fall on whole
+// waves, which skip the dual half.  Other rows run in equal tiles of at most 128 columns
 // plus a halo column on each side; a band of one whole row would run the dual half
 // three times per voxel (us, one row / tiles: two levels 100x200x200 489 / 409,
-// 120x100x250 383 / 291, 256^3 1489 / 1623; one level 100x300x300 755 / 573,
-// 40x320x320 287 / 250).
+// 120x100x250 383 / 291; one level 100x300x300 755 / 573, 40x320x320 287 / 250).  Rows of whole
+// waves keep one-row bands where their plane steps on the busiest CU are fewer than 1.38x the
+// tiles', whose steps take about that much longer (two levels, W = 256, steps x and us, one row
+// / tiles: 256^3 1.36, 1513 / 1676; 256x128x128 1.27, 394 / 414; 256x200x60 1.24, 327 / 317;
+// 256x60x200 1.46, 293 / 272; 256x180x180 1.48, 840 / 784; 256x300x20 1.5, 181 / 160).
 // Measured on MI355X at 256^3, one level: whole rows, band 2, 767 us per launch; 64- and
 // 128-column tiles with bands of 4 to 13 rows, 1027-1385 us (their rows are
 // 264- or 520-B pieces off cache-line boundaries, and every wave then holds
@@ -1186,33 +1188,39 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     if (!want_tx && !want_ty && !want_zc && g.n() <= KFUSED_SMALL && (levels > 1 || g.n() > KFUSED_TINY))
         return false;
     const int max_threads = kfused_max_threads(levels), rows = 11 + 11 * levels;
-    int tx = g.w;
-    if (want_tx > 0) tx = std::min(want_tx, g.w);
-    else if (4 * g.w > max_threads && 3 * g.w != max_threads)
-        tx = (g.w + (g.w + 127) / 128 - 1) / ((g.w + 127) / 128);
-    if (!want_tx && !want_ty && !want_zc && levels > 1 &&
-        (g.d < 4 || (tx < g.w && g.n() <= KFUSED_TILED_SMALL)))
-        return false;
-    const int txh = tx < g.w ? tx + 2 : g.w;
-    int ty = std::min(max_threads / txh - 2, g.h);
-    while (ty >= 1 && size_t(rows) * (ty + 2) * txh * sizeof(float) > size_t(max_lds)) --ty;
-    if (want_ty > 0) {
-        if (want_ty > ty) return false;   // does not fit
-        ty = want_ty;
+    // the plan of a tile width: its plane steps on the busiest CU, negative if nothing fits
+    auto steps = [&](int tx, TgvkFusedPlan* p) {
+        const int txh = tx < g.w ? tx + 2 : g.w;
+        int ty = std::min(max_threads / txh - 2, g.h);
+        while (ty >= 1 && size_t(rows) * (ty + 2) * txh * sizeof(float) > size_t(max_lds)) --ty;
+        if (ty < 1 || want_ty > ty) return -1L;
+        if (want_ty > 0) ty = want_ty;
+        const long nb = long((g.w + tx - 1) / tx) * ((g.h + ty - 1) / ty);
+        int best_zc = g.d;
+        long best = -1;
+        for (int nc = 1; nc <= g.d; ++nc) {
+            const int zc = (g.d + nc - 1) / nc;
+            const long rounds = (nb * ((g.d + zc - 1) / zc) + cus - 1) / cus;
+            const long cost = rounds * (zc + 1);
+            if (best < 0 || cost < best) { best = cost; best_zc = zc; }
+        }
+        if (want_zc > 0) best_zc = std::min(want_zc, g.d);
+        *p = TgvkFusedPlan{tx, ty, best_zc};
+        return best;
+    };
+    const bool whole = want_tx > 0 || 4 * g.w <= max_threads;
+    const int tiles = (g.w + 127) / 128, tx = want_tx > 0 ? std::min(want_tx, g.w)
+                                              : whole     ? g.w
+                                                          : (g.w + tiles - 1) / tiles;
+    const long cost = steps(tx, plan);
+    if (cost < 0) return false;
+    if (!whole && g.w % 64 == 0 && 3 * g.w <= max_threads) {
+        TgvkFusedPlan p;
+        const long one = steps(g.w, &p);
+        if (one >= 0 && one * 100 < cost * 138) *plan = p;
     }
-    if (ty < 1) return false;
-    const long nb = long((g.w + tx - 1) / tx) * ((g.h + ty - 1) / ty);
-    int best_zc = g.d;
-    long best = -1;
-    for (int nc = 1; nc <= g.d; ++nc) {
-        const int zc = (g.d + nc - 1) / nc;
-        const long rounds = (nb * ((g.d + zc - 1) / zc) + cus - 1) / cus;
-        const long cost = rounds * (zc + 1);
-        if (best < 0 || cost < best) { best = cost; best_zc = zc; }
-    }
-    if (want_zc > 0) best_zc = std::min(want_zc, g.d);
-    *plan = TgvkFusedPlan{tx, ty, best_zc};
-    return true;
+    return want_tx || want_ty || want_zc || levels == 1 ||
+           (g.d >= 4 && (plan->tx == g.w || g.n() > KFUSED_TILED_SMALL));
 }
 
 // Tile columns of the masked loop (0: whole rows): tiles of 126 columns, whose rows
