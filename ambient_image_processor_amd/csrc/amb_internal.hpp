@@ -337,6 +337,7 @@ struct TgvkFusedPlan {
     int tx;       // owned x columns per block (W: whole rows)
     int ty;       // owned y rows per block
     int zchunk;   // planes per block
+    bool masked_only = false;   // without a mask the two launches are faster
 };
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan);

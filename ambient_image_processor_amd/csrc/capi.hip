@@ -1080,7 +1080,8 @@ amb_status tgvk_run(amb_context* c, uint32_t iterations, uint32_t interval,
     float* const* F = reinterpret_cast<float* const*>(c->fields_dev);
     // (masked, two levels: the first fused launch sweeps the whole volume, where the two launches
     // skip inactive voxels and are as fast: fused only where a listed one follows)
-    bool fused = c->kfused_ok && iterations > (c->sp.active && c->klevels > 1 ? 2u : 1u);
+    bool fused = c->kfused_ok && iterations > (c->sp.active && c->klevels > 1 ? 2u : 1u) &&
+                 (c->sp.active || !c->kfplan.masked_only);
     if (fused) AMB_TRY(tgvk_fused_buffers(c, &fused));
     const Looping looping(c);
     if (fused) {

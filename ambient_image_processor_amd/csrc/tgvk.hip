@@ -1167,11 +1167,16 @@ int tgvk_blocks(const Geometry& g, const PlanOverrides& ov, int* zchunk) {
 // where both take the launches' own time (14x12x10: 7.7 against 7.8).  Two levels
 // in tiles start to win above KFUSED_TILED_SMALL (60x70x250 100 against 93, 120x100x250
 // 291 against 379), and volumes of under four planes have no plane to carry
-// (1x1200x256 43 against 27): two launches.  Three
+// (1x1200x256 43 against 27): two launches.  Two levels of up to as many voxels also run
+// them, unless a mask lets lanes skip, in bands of up to four rows (with two halo rows each)
+// whose plane steps have under KFUSED_STEP_VOXELS voxels of their own for a block's 768
+// threads: 14 of 85 shapes, 0.81 to 0.98x fused (256x400x8 96 against 78, 181x173x25 86 / 75,
+// 191x384x15 118 / 106; at the line 140x160x42 89.5 / 89.3).  Three
 // levels (217 registers, 512 threads) gained 1.1x at 300x200x40 and lost 0.73x at
 // 256^3: two launches.  The overrides tgvk_fused = 0 disable the
 // fused sweep, tgvk_fused_tx, _ty and _zchunk set the plan.
 constexpr size_t KFUSED_SMALL = 300000, KFUSED_TINY = 16384, KFUSED_TILED_SMALL = 1200000;
+constexpr long KFUSED_STEP_VOXELS = 300;
 
 bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverrides& ov,
                      TgvkFusedPlan* plan) {
@@ -1212,13 +1217,16 @@ bool tgvk_fused_plan(const Geometry& g, int levels, int device, const PlanOverri
     const int tiles = (g.w + 127) / 128, tx = want_tx > 0 ? std::min(want_tx, g.w)
                                               : whole     ? g.w
                                                           : (g.w + tiles - 1) / tiles;
-    const long cost = steps(tx, plan);
+    long cost = steps(tx, plan);
     if (cost < 0) return false;
     if (!whole && g.w % 64 == 0 && 3 * g.w <= max_threads) {
         TgvkFusedPlan p;
         const long one = steps(g.w, &p);
-        if (one >= 0 && one * 100 < cost * 138) *plan = p;
+        if (one >= 0 && one * 100 < cost * 138) { *plan = p; cost = one; }
     }
+    plan->masked_only = !want_tx && !want_ty && !want_zc && levels > 1 &&
+                        plan->ty <= 4 && g.n() <= KFUSED_TILED_SMALL &&
+                        cost * cus * KFUSED_STEP_VOXELS > long(g.n());
     return want_tx || want_ty || want_zc || levels == 1 ||
            (g.d >= 4 && (plan->tx == g.w || g.n() > KFUSED_TILED_SMALL));
 }

@@ -536,3 +536,30 @@ def test_tgv2_iterations_go_on_from_a_fused_tgvk_state(shape, alpha, iterations)
             c.iterate(3)
             states.append(c.get_state())
     np.testing.assert_array_equal(states[0], states[1])
+
+
+# order 4, whole rows, up to 1.2 M voxels: fused where a plane step owns 300 voxels or more per block
+@pytest.mark.parametrize("shape,fused", [((12, 300, 180), False), ((25, 173, 181), False),
+                                         ((34, 289, 59), True), ((93, 70, 118), True)])
+def test_order_4_of_short_chunks_runs_two_launches(ctx, shape, fused):
+    """... unless a mask lets lanes skip; the results are the same."""
+    from ambient_image_processor_amd import native
+    _say("order 4 short chunks", shape)
+    f = _f(shape, 39)
+    alpha = (1.0, 2.0, 0.3, 0.2)
+    act = (np.random.default_rng(39).random(shape) < 0.02).astype(np.uint8)
+
+    def run(call, *a):
+        ctx.profile(True)
+        ctx.profile_reset()
+        out = call(f, _params(native, 4), alpha, *a)
+        n = ctx.profile_counts()["tgvk_fused"]
+        ctx.profile(False)
+        return out, n
+    plain, n = run(ctx.tgvk_deshade)
+    assert n == (3 if fused else 0)
+    masked, n = run(ctx.tgvk_deshade_masked, act)
+    assert n == 3
+    ctx.set_override("tgvk_fused", 0)
+    for a, b in zip(plain + masked, run(ctx.tgvk_deshade)[0] + run(ctx.tgvk_deshade_masked, act)[0]):
+        np.testing.assert_array_equal(a, b)
