@@ -408,19 +408,27 @@ amb_status ensure_axis(amb_context* c, int axis, int n, int precision) {
         *dst = dev;
         return AMB_OK;
     };
+    // the split table: its fragments lie in order of their 16 rows
     auto upload_split = [&](uint16_t** dst, auto value) -> amb_status {
-        std::vector<uint16_t> h(dct_fragment_count(n), uint16_t(0));
-        for (int k = 0; k < n; ++k)
-            for (int m = 0; m < n; ++m) {
-                const double v = value(k, m);
-                const size_t i = dct_fragment_index(n, k, m);
-                h[i] = host_bf16_rne(float(v));
-                h[i + 512] = host_bf16_rne(float(v - double(host_bf16_to_float(h[i]))));
-            }
         uint16_t* dev = nullptr;
-        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&dev), h.size() * 2));
-        const hipError_t e = hipMemcpy(dev, h.data(), h.size() * 2, hipMemcpyHostToDevice);
-        if (e != hipSuccess) { (void)hipFree(dev); return fail_hip(e, "hipMemcpy", __LINE__); }
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&dev), dct_fragment_count(n) * 2));
+        const int tiles = (n + 15) / 16;
+        const size_t tile = dct_fragment_count(n) / size_t(tiles);
+        const int per = std::max(1, int((size_t(1) << 21) / tile));
+        std::vector<uint16_t> h;
+        for (int t0 = 0; t0 < tiles; t0 += per) {
+            const int t1 = std::min(t0 + per, tiles);
+            h.assign(tile * size_t(t1 - t0), uint16_t(0));
+            for (int k = t0 * 16; k < std::min(t1 * 16, n); ++k)
+                for (int m = 0; m < n; ++m) {
+                    const double v = value(k, m);
+                    const size_t i = dct_fragment_index(n, k, m) - tile * size_t(t0);
+                    h[i] = host_bf16_rne(float(v));
+                    h[i + 512] = host_bf16_rne(float(v - double(host_bf16_to_float(h[i]))));
+                }
+            const hipError_t e = hipMemcpy(dev + tile * size_t(t0), h.data(), h.size() * 2, hipMemcpyHostToDevice);
+            if (e != hipSuccess) { (void)hipFree(dev); return fail_hip(e, "hipMemcpy", __LINE__); }
+        }
         *dst = dev;
         return AMB_OK;
     };

@@ -8,9 +8,9 @@
 //   forward  C[k][m] = cos(pi (m + 1/2) k / n)
 //   inverse  C[k][m] = w_m cos(pi (k + 1/2) m / n), w_0 = 1, w_m = 2 (the
 //            reference's "X[0] + 2 sum_{m>=1}" folded into the matrix)
-// The last (z) pass applies the reference's *8 (forward) or 1/(W*H*D*8)
-// (inverse), and can fuse the Poisson eigenvalue divide of
-// solve_poisson_in_cosine_domain.cu:42-53 into its epilogue.
+// The last pass (z, or y or x where the axes after it have one voxel and no pass)
+// applies the reference's *8 (forward) or 1/(W*H*D*8) (inverse), and can fuse the
+// Poisson eigenvalue divide of solve_poisson_in_cosine_domain.cu:42-53 into its epilogue.
 //
 // Precisions:
 //   F32     v_mfma_f32_16x16x4_f32, FP32 operands, FP32 accumulate
@@ -263,7 +263,9 @@ __device__ __forceinline__ void split4(const float (&x)[4], uint2& hi, uint2& lo
 // ---------------------------------------------------------------------------
 // BF16x3 panel kernel.
 //
-// A block of 8 waves walks through panels of columns (lines of the axis), 64
+// An item is a panel of columns (lines of the axis) and a group of up to 16 output tiles of 16
+// rows: axes of up to 256 values have one group, longer ones load and split each panel once
+// per group (512: twice).  A block of 8 waves walks through its items, 64
 // summed indices (a stage) at a time: the stage's data lie in LDS as bf16 hi/lo
 // splits, two buffers, and each wave multiplies them with its two 16-row tiles
 // of the table (x 16 CT columns).  The table's fragments come straight from L2 in

@@ -46,3 +46,9 @@ def test_poisson_solve_against_oracle(ctx, orc, shape, precision, tol):
     ref = orc.integrate_poisson(*[c.astype(np.float64) for c in v], dtype=np.float64)
     out = ctx.integrate_gradients_poisson(*v, precision=precision)
     assert _rel(out, ref) < tol
+
+
+# axes whose split table goes to the device in several pieces (from 1025 values on)
+@pytest.mark.parametrize("shape", [(1, 3, 2100), (1, 2065, 4), (4096, 1, 2)])
+def test_long_axes_against_scipy(ctx, shape):
+    test_transforms_against_scipy(ctx, shape, 2, 4e-5)
