@@ -349,8 +349,9 @@ bool tgvk_masked_tiles(const Geometry& g, int levels, int device, const PlanOver
                        const uint8_t* rows, TgvkFusedPlan* plan, std::vector<FusedTile>* tiles);
 hipError_t launch_tgvk_fused(hipStream_t s, const void* t, const void* lv, size_t field_stride,
                              ptrdiff_t dt, ptrdiff_t dl, const float* f, const uint8_t* active,
-                             const FusedTile* tiles, size_t ntiles, Geometry g, int levels, float tau, float sigma, float lambda,
-                             float theta, const float* alpha, int planar,
+                             const FusedTile* tiles, size_t ntiles, Geometry g, int levels,
+                             float tau, float sigma, float lambda, float theta,
+                             const float* alpha, int planar,
                              const TgvkFusedPlan& plan);
 
 // Cubic B-spline resampling (resize.hip): in (gi) to out (go, the kept voxels);

@@ -318,7 +318,8 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
     c->f = reinterpret_cast<float*>(c->fblock);
     for (int k = 0; k < N_SCRATCH; ++k)
         c->scratch[k] = reinterpret_cast<float*>(c->fblock + fl * size_t(1 + k));
-    if (!c->fields_dev) AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->fields_dev), sizeof(void*) * N_FIELDS));
+    if (!c->fields_dev)
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->fields_dev), sizeof(void*) * N_FIELDS));
     AMB_HIP(hipMemcpyAsync(c->fields_dev, c->fields, sizeof(void*) * N_FIELDS,
                            hipMemcpyHostToDevice, c->stream));
     size_t pn = energy_partials_size(g);
@@ -332,7 +333,8 @@ amb_status ensure_buffers(amb_context* c, Geometry g, int storage) {
         AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->partials), pn * sizeof(double)));
         c->partials_cap = pn;
     }
-    if (!c->energy_out) AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->energy_out), 16 * sizeof(double)));
+    if (!c->energy_out)
+        AMB_HIP(device_alloc(c, reinterpret_cast<void**>(&c->energy_out), 16 * sizeof(double)));
     c->g = g;
     c->storage = storage;
     return AMB_OK;
@@ -426,7 +428,8 @@ amb_status ensure_axis(amb_context* c, int axis, int n, int precision) {
                     h[i] = host_bf16_rne(float(v));
                     h[i + 512] = host_bf16_rne(float(v - double(host_bf16_to_float(h[i]))));
                 }
-            const hipError_t e = hipMemcpy(dev + tile * size_t(t0), h.data(), h.size() * 2, hipMemcpyHostToDevice);
+            const hipError_t e = hipMemcpy(dev + tile * size_t(t0), h.data(), h.size() * 2,
+                                           hipMemcpyHostToDevice);
             if (e != hipSuccess) { (void)hipFree(dev); return fail_hip(e, "hipMemcpy", __LINE__); }
         }
         *dst = dev;
@@ -1181,8 +1184,8 @@ amb_status check_precision(const Geometry& g, int precision) {
     return AMB_OK;
 }
 
-// One separable transform of src into dst through the scratch volumes a and b
-// (src is read by the first pass only, so b and dst may be src's buffer).  poisson_flags >= 0 fuses
+// One separable transform of src into dst through the scratch volumes a and b (src is read
+// by the first pass only, so b and dst may be src's buffer).  poisson_flags >= 0 fuses
 // the eigenvalue divide into the last forward pass (MFMA precisions only).
 amb_status transform3(amb_context* c, const float* src, float* a, float* b, float* dst,
                       int inverse, int precision, int poisson_flags = -1) {

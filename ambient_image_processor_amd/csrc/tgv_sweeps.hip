@@ -46,19 +46,21 @@ namespace {
 // 8 XCDs) receives a contiguous range of tiles, the first nblocks % 8 XCDs one more, so
 // that halo rows are found in the L2 (fused sweep with block counts that 8 does not
 // divide, us per launch against the plain order: 161 x 145 x 140 97 -> 90, 301 x 250
-// x 60 BF16 92 -> 78, 291 x 101 x 142 BF16 84 -> 67; 75 of 78 shapes 1.01-1.26x).
-__device__ __forceinline__ int xcd_tile(int bid, int nblocks) {
+// x 60 BF16 92 -> 78, 291 x 101 x 142 BF16 84 -> 67; 75 of 78 shapes 1.01-1.26x).  Where a mask
+// lets whole blocks skip (uneven), such counts keep the plain order, which spreads the
+// mask over the XCDs (two sweeps, 312 x 357 x 68, a ball of radius 0.42: 356 us contiguous, 315).
+__device__ __forceinline__ int xcd_tile(int bid, int nblocks, bool uneven = false) {
     if ((nblocks & 7) != 0)
-        return (bid & 7) * (nblocks >> 3) + min(bid & 7, nblocks & 7) + (bid >> 3);
+        return uneven ? bid : (bid & 7) * (nblocks >> 3) + min(bid & 7, nblocks & 7) + (bid >> 3);
     return (bid & 7) * (nblocks >> 3) + (bid >> 3);
 }
 
 template <int TX, int TY>
 struct TileCoord {
     int x0, y0, z0, z1, tx, ty, x, y;
-    __device__ __forceinline__ TileCoord(const Geometry& g, int zchunk) {
+    __device__ __forceinline__ TileCoord(const Geometry& g, int zchunk, bool masked) {
         const int nbx = (g.w + TX - 1) / TX, nby = (g.h + TY - 1) / TY;
-        const int t = xcd_tile(blockIdx.x, gridDim.x);
+        const int t = xcd_tile(blockIdx.x, gridDim.x, masked);
         const int bx = t % nbx, r = t / nbx, by = r % nby, bz = r / nby;
         x0 = bx * TX; y0 = by * TY;
         z0 = bz * zchunk; z1 = min(z0 + zchunk, g.d);
@@ -93,7 +95,7 @@ __global__ __launch_bounds__(TX * TY) void dual_sweep_kernel(
     __shared__ float sU[TY + 2][TX + 2];
     __shared__ float sV[3][TY + 2][TX + 2];
 
-    const TileCoord<TX, TY> c(g, zchunk);
+    const TileCoord<TX, TY> c(g, zchunk, MK);
     const int W = g.w, H = g.h, D = g.d;
     const I plane = I(W) * I(H);
     const bool in = (c.x < W) && (c.y < H);
@@ -246,7 +248,7 @@ __global__ __launch_bounds__(TX * TY) void primal_sweep_kernel(
     float tau, float lambda, float theta, int zchunk) {
     __shared__ float sL[L_N][TY + 2][TX + 2];
 
-    const TileCoord<TX, TY> c(g, zchunk);
+    const TileCoord<TX, TY> c(g, zchunk, MK);
     const int W = g.w, H = g.h, D = g.d;
     const I plane = I(W) * I(H);
     const bool in = (c.x < W) && (c.y < H);
@@ -528,10 +530,10 @@ __device__ __forceinline__ void vstore(typename S::T* p, I i, const float (&v)[V
 template <int TX, int TY, int VX>
 struct TileCoordV {
     int x0, y0, z0, z1, tx, ty, xb, y;
-    __device__ __forceinline__ TileCoordV(const Geometry& g, int zchunk) {
+    __device__ __forceinline__ TileCoordV(const Geometry& g, int zchunk, bool masked) {
         constexpr int RW = TX * VX;
         const int nbx = (g.w + RW - 1) / RW, nby = (g.h + TY - 1) / TY;
-        const int t = xcd_tile(blockIdx.x, gridDim.x);
+        const int t = xcd_tile(blockIdx.x, gridDim.x, masked);
         const int bx = t % nbx, r = t / nbx, by = r % nby, bz = r / nby;
         x0 = bx * RW; y0 = by * TY;
         z0 = bz * zchunk; z1 = min(z0 + zchunk, g.d);
@@ -564,7 +566,7 @@ __global__ __launch_bounds__(TX * TY) void dual_sweep_vec_kernel(
     __shared__ float sXp[TY][TX + 1];                   // u_bar element 0 per thread; [ty][TX] = +x halo
     __shared__ float sXm[3][TY][TX + 1];                // v_bar element VX-1 at [ty][tx+1]; [ty][0] = -x halo
 
-    const TileCoordV<TX, TY, VX> c(g, zchunk);
+    const TileCoordV<TX, TY, VX> c(g, zchunk, MK);
     const int W = g.w, H = g.h, D = g.d;
     const I plane = I(W) * I(H);
     const bool in = (c.xb < W) && (c.y < H);
@@ -740,7 +742,7 @@ __global__ __launch_bounds__(TX * TY) void primal_sweep_vec_kernel(
     __shared__ float sXp[3][TY][TX + 1];    // q_xx, q_xy, q_xz element 0; [ty][TX] = +x halo
     __shared__ float sXm[TY][TX + 1];       // p_x element VX-1 at [ty][tx+1]; [ty][0] = -x halo
 
-    const TileCoordV<TX, TY, VX> c(g, zchunk);
+    const TileCoordV<TX, TY, VX> c(g, zchunk, MK);
     const int W = g.w, H = g.h, D = g.d;
     const I plane = I(W) * I(H);
     const bool in = (c.xb < W) && (c.y < H);
@@ -1746,8 +1748,8 @@ hipError_t fused_launch(hipStream_t s, const FusedFields& ff, const float* f, Ge
     hipError_t e = ensure_dynamic_lds(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
     if (list && p.ntiles == 0) return hipSuccess;   // no active voxel
-    hipLaunchKernelGGL(kern, dim3(list ? unsigned(p.ntiles) : unsigned(nbx * nb * nc)), dim3(L * RT), lds, s, ff,
-                       f, MK ? p.fused_active : nullptr, g, p.tau,
+    hipLaunchKernelGGL(kern, dim3(list ? unsigned(p.ntiles) : unsigned(nbx * nb * nc)),
+                       dim3(L * RT), lds, s, ff, f, MK ? p.fused_active : nullptr, g, p.tau,
                        p.sigma, p.lambda, p.alpha0, p.alpha1, p.theta, plan.ty, plan.zchunk,
                        p.planar, TL ? plan.tx : 0, EN ? p.energy_partials : nullptr,
                        list ? p.tiles : nullptr,
@@ -2194,10 +2196,10 @@ bool fused_plan(const Geometry& g, int storage, int device, const PlanOverrides&
 //   (rounds of resident blocks) (zc + 2) + 0.12 (waves on the busiest CU) (zc + 1)
 //     + 0.115 (its owned waves) zc + 0.0022 blocks
 // in units of a plane step's latency (200 VGPRs: a block of up to four waves leaves room for a
-// second one; one more launch sums the blocks' results).  The iteration plan's chunk and band do not fit this form, which is bound by
-// its FP64 sums: they gave too few blocks or one-row bands (us per launch, one voxel per
-// lane / two voxels with the iteration plan's band and chunk / this plan: 279 x 219 x 88 359 /
-// 483 / 297, 373 x 96 x 96 195 / 230 / 165, 133 x 281 x 95 340 / 196 / 166, 21 x 27 x 16 14.4 /
+// second one; one more launch sums the blocks' results).  The iteration plan's chunk and
+// band do not fit this form, which is bound by its FP64 sums: they gave too few blocks or
+// one-row bands (us per launch, one voxel per lane / two voxels with the iteration plan's band
+// and chunk / this plan: 279 x 219 x 88 359 / 483 / 297, 373 x 96 x 96 195 / 230 / 165, 133 x 281 x 95 340 / 196 / 166, 21 x 27 x 16 14.4 /
 // 19.0 / 13.5).  On 160 shapes of 8 k to 10 M voxels the model's mean error is 3% and its plans
 // are 1.31x the one-voxel form's speed in the mean, 0.93x at worst (83 x 143 x 178 91 / 98).
 // Chunks: those that give every CU k = 1 .. 8 blocks.
@@ -2231,7 +2233,8 @@ static bool odd_energy_plan(const Geometry& g, int cus, size_t max_lds, const Pl
                 const long blocks = nb * ((g.d + zc - 1) / zc), on_cu = (blocks + cus - 1) / cus;
                 const long rounds = (blocks + long(cus) * per_cu - 1) / (long(cus) * per_cu);
                 const double cost = double(rounds) * (zc + 2) + 0.12 * double(on_cu * waves) * (zc + 1) +
-                                    0.115 * double(on_cu * ty * lanes) / 64.0 * zc + 0.0022 * double(blocks);
+                                    0.115 * double(on_cu * ty * lanes) / 64.0 * zc +
+                                    0.0022 * double(blocks);
                 if (cost < best) { best = cost; *plan = FusedPlan{ty, zc, 0, 2, tx}; }
             }
         }
@@ -2427,9 +2430,9 @@ void MaskedRows::tiles(int band, int zchunk, std::vector<FusedTile>* out) const 
 // Against the iteration plan and its prefetch, tiles skipped inside the full grid
 // (which left the XCDs unevenly loaded) and every lane of the others loading and
 // storing (us per launch, balls of 3, 11, 31 and 50% of the voxels and a random half):
-// 256^3 147 219 332 353 368 -> 45 103 208 290 368; 181 x 217 x 181 49 87 154 196 199 ->
-// 23 48 114 170 199; 160 x 145 x 140 42 48 87 76 81 -> 16 28 50 67 81; 301 x 250 x 60 45
-// 61 126 155 169 -> 16 30 65 110 147; BF16 256^3 94 153 222 225 234 -> 32 68 158 206 247.
+// 256^3 147 219 332 353 368 -> 46 103 208 277 370; 181 x 217 x 181 49 87 154 196 199 ->
+// 24 49 114 168 196; 160 x 145 x 140 42 48 87 76 83 -> 18 29 52 69 83; 301 x 250 x 60 45
+// 61 126 155 169 -> 16 30 65 107 131; BF16 256^3 94 153 222 225 236 -> 32 67 157 198 232.
 constexpr size_t MASKED_SMALL = 300000;
 
 // Tile columns of the masked sweep: the iteration plan's, but the one-voxel form's tiles
